@@ -83,6 +83,7 @@ struct holo_ctx {
   DevBuf amp, phase, u, v, y, w, partial, small, b, pos, ph;
   DevBuf mc_wc, mc_xy, mc_info;  // product-grid Monte Carlo (McLattice)
   DevBuf layout;                 // source layout of device-pointer FP64 calls
+  DevBuf pairs;                  // lattice-to-lattice kernel: target lattice, flags, outcome
   DevBuf errb;                   // error report: subset, FP64 values, partials
   DevBuf pos64, ph64;            // FP64 Monte Carlo records for the error report
   // recorded on the previous stream when holo_set_stream switches streams
@@ -136,6 +137,9 @@ struct holo_plan {
   double g64_cx0 = 0, g64_cx1 = 0, g64_cy0 = 0, g64_cy1 = 0;
   float g64_rho_y = 0;
   DevBuf g64_centre;
+  // the same lattice for the lattice-to-lattice kernel (pp.n_tiles = 0: none)
+  holo::PairPlan pp;
+  DevBuf pr_wq, pr_ts, pr_tail;
   // Every call rewrites the weight buffers above.  `ran` is recorded after
   // each call on its stream; a call on another stream waits for it first.
   mutable hipEvent_t ran = nullptr;
@@ -749,7 +753,7 @@ holo_status plan_build_tiles(holo_ctx* ctx, const holo_plan* p, const double* u_
 }
 
 // The 16-row tiles of grid (and their tail), if any, onto the device.
-holo_status upload_grid16(holo_ctx* ctx, holo_plan* p, const HostGrid& grid) {
+holo_status upload_grid16(holo_ctx* ctx, holo_plan* p, const HostGrid& grid, const double* u) {
   const size_t n16 = grid.centre16.size(), nt = grid.tail.size();
   if (!n16) return HOLO_OK;
   if (256 * n16 + nt > kMaxCount) return fail(HOLO_EINVAL, "too many tile slots");
@@ -809,6 +813,30 @@ holo_status upload_grid16(holo_ctx* ctx, holo_plan* p, const HostGrid& grid) {
     HOLO_HIP(hipMemcpyAsync(p->g64_centre.ptr, grid.centre64.data(), n64 * sizeof(double4),
                             hipMemcpyHostToDevice, ctx->stream));
   }
+  holo::PairPlan& pp = p->pp;
+  pp.x0 = u[0];
+  pp.y0 = u[1];
+  pp.z = grid.z;
+  pp.px = grid.px;
+  pp.py = grid.py;
+  pp.nx = (uint32_t)grid.nx;
+  pp.ny = (uint32_t)grid.ny;
+  pp.tj = (uint32_t)((grid.ny + 63) / 64);
+  const size_t np = (grid.nx + 31) / 32 * pp.tj;
+  pp.n_tail = (uint32_t)nt;
+  pp.tail_same = true;
+  for (const int32_t n : grid.tail)
+    for (int d = 0; d < 3; ++d)
+      pp.tail_same = pp.tail_same && u[3 * (size_t)n + d] == u[3 * (size_t)grid.tail[0] + d];
+  HOLO_TRY(ensure(p->pr_wq, 1024 * np * sizeof(uint4), ctx->device));
+  HOLO_TRY(ensure(p->pr_ts, np * sizeof(float), ctx->device));
+  HOLO_TRY(ensure(p->pr_tail, std::max<size_t>(nt, 1) * sizeof(float2), ctx->device));
+  pp.u = static_cast<const double*>(p->u.ptr);
+  pp.tail_perm = static_cast<const int32_t*>(p->g16_perm.ptr) + 256 * n16;
+  pp.wq = static_cast<uint4*>(p->pr_wq.ptr);
+  pp.tscale = static_cast<float*>(p->pr_ts.ptr);
+  pp.tail_wc = static_cast<float2*>(p->pr_tail.ptr);
+  pp.n_tiles = (uint32_t)np;
   return HOLO_OK;
 }
 
@@ -840,11 +868,11 @@ holo_status plan_upload_tiles(holo_ctx* ctx, holo_plan* p, const double* u_host)
                             hipMemcpyHostToDevice, ctx->stream));
     HOLO_HIP(hipMemcpyAsync(p->g_perm.ptr, grid.perm.data(), 64 * nt * sizeof(int32_t),
                             hipMemcpyHostToDevice, ctx->stream));
-    HOLO_TRY(upload_grid16(ctx, p, grid));
+    HOLO_TRY(upload_grid16(ctx, p, grid, u_host));
   } else if (p->tile == 64 && build_grid16_padded(u_host, p->N, grid)) {
     p->grid_nx = grid.nx;
     p->grid_ny = grid.ny;
-    HOLO_TRY(upload_grid16(ctx, p, grid));
+    HOLO_TRY(upload_grid16(ctx, p, grid, u_host));
   }
   // host vectors are freed on return: wait for the copies
   HOLO_HIP(hipStreamSynchronize(ctx->stream));
@@ -914,6 +942,11 @@ holo_status plan_build(holo_ctx* ctx, holo_plan* p, const double* u, size_t N,
   return HOLO_OK;
 }
 
+// Up to this many sources a call prepares the weights of both lattice paths in
+// one launch: a second launch costs 3 us (also when it has nothing to do), the
+// 16-row kernels' operands less than that (40 bytes a source).
+constexpr size_t kPrepareBoth = 131072;
+
 // y (device) = sum over the plan's sources; weights already device-resident.
 holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int sign,
                           bool obliquity, double lambda, holo::WeightForm wf,
@@ -933,13 +966,42 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
     const bool pairs = p->g32_tiles && holo::tuning().grid32;
     const bool quads = pairs && p->g64_tiles && holo::tuning().grid64;
     const int nkc = quads ? 4 : (pairs ? 2 : 1);
-    HOLO_HIP(holo::launch_tile_weights(wf, w0, w1, static_cast<const int32_t*>(p->g16_perm.ptr),
-                                       256 * nt + p->g16_tail,
-                                       static_cast<float2*>(p->g16_wc.ptr), ctx->stream));
-    HOLO_HIP(holo::launch_grid16_weights(static_cast<const float2*>(p->g16_wc.ptr), (uint32_t)nt,
-                                         nkc, static_cast<uint4*>(p->g16_wq.ptr),
-                                         static_cast<uint4*>(p->g16_wqn.ptr),
-                                         static_cast<float*>(p->g16_ts.ptr), ctx->stream));
+    // Targets on a lattice of their own take the lattice-to-lattice kernel, which
+    // looks at them on the device; `skip` then tells the 16-row launches below
+    // that the call is done.  (Options that pick a 16-row tile shape keep it.)
+    const uint32_t* skip = nullptr;
+    int Sp = 1;
+    const int S16 = holo::grid_splits(M, quads ? p->g64_tiles : (pairs ? p->g32_tiles : nt));
+    const holo::Tuning& tu = holo::tuning();
+    holo::Grid16Prep prep;
+    prep.wf = (int)wf;
+    prep.w0 = w0;
+    prep.w1 = w1;
+    prep.perm = static_cast<const int32_t*>(p->g16_perm.ptr);
+    prep.n_tiles = (uint32_t)nt;
+    prep.n_tail = (uint32_t)p->g16_tail;
+    prep.group = (uint32_t)nkc;
+    prep.wc = static_cast<float2*>(p->g16_wc.ptr);
+    prep.wq = static_cast<uint4*>(p->g16_wq.ptr);
+    prep.wqn = static_cast<uint4*>(p->g16_wqn.ptr);
+    prep.tscale = static_cast<float*>(p->g16_ts.ptr);
+    bool prepared = false;
+    if (tu.grid_pairs && tu.grid32 && tu.grid64 && p->pp.n_tiles && M >= holo::kPairMinTargets) {
+      Sp = holo::pair_splits(M, p->pp.n_tiles);
+      const size_t pe = std::max(Sp, S16) > 1 ? (size_t)std::max(Sp, S16) * M : 0;
+      if (pe) HOLO_TRY(ensure(ctx->partial, pe * sizeof(double2), ctx->device));
+      HOLO_TRY(ensure(ctx->pairs, 256 + holo::kPairFlags * sizeof(uint32_t), ctx->device));
+      char* b = static_cast<char*>(ctx->pairs.ptr);
+      uint32_t* handled = reinterpret_cast<uint32_t*>(b + 128);
+      HOLO_HIP(holo::launch_superpose_pairs(
+          sign, obliquity, p->pp, wf, w0, w1, v, M, lambda, Sp,
+          reinterpret_cast<holo::PairTargets*>(b), reinterpret_cast<uint32_t*>(b + 256), handled,
+          Sp > 1 ? static_cast<double2*>(ctx->partial.ptr) : reinterpret_cast<double2*>(y),
+          p->N <= kPrepareBoth ? &prep : nullptr, ctx->stream));
+      skip = handled;
+      prepared = p->N <= kPrepareBoth;
+    }
+    if (!prepared) HOLO_HIP(holo::launch_grid16_weights(prep, ctx->stream, skip));
     holo::GridTiles g16;  // the 16 x 16 tiles
     g16.perm = static_cast<const int32_t*>(p->g16_perm.ptr);
     g16.u = static_cast<const double*>(p->u.ptr);
@@ -984,8 +1046,7 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
       gt.cy1 = p->g64_cy1;
       gt.rho_y = p->g64_rho_y;
     }
-    const int S = holo::grid_splits(M, gt.n_tiles);
-    const size_t pe = S > 1 ? (size_t)S * M : 0;
+    const size_t pe = S16 > 1 ? (size_t)S16 * M : 0;
     if (pe) HOLO_TRY(ensure(ctx->partial, pe * sizeof(double2), ctx->device));
     HOLO_HIP(holo::launch_superpose_grid16(sign, obliquity, nkc, gt, g32, g16,
                                            static_cast<const float2*>(p->g16_wc.ptr),
@@ -994,7 +1055,7 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
                                            static_cast<const float*>(p->g16_ts.ptr), v, M,
                                            lambda, reinterpret_cast<double2*>(y),
                                            static_cast<double2*>(ctx->partial.ptr), pe,
-                                           ctx->stream));
+                                           ctx->stream, skip, Sp));
   } else if (p->grid_tiles && holo::tuning().grid) {
     const size_t nt = p->grid_tiles;
     HOLO_HIP(holo::launch_tile_weights(wf, w0, w1, static_cast<const int32_t*>(p->g_perm.ptr),
@@ -1206,6 +1267,8 @@ holo_status holo_set_option(const char* name, long value) {
     t.grid_near = value != 0;
   } else if (n == "grid_rows") {
     t.grid_rows = value != 0;
+  } else if (n == "grid_pairs") {
+    t.grid_pairs = value != 0;
   } else if (n == "mc_lattice") {
     t.mc_lattice = value != 0;
   } else if (n == "mc_passes") {
@@ -1235,6 +1298,7 @@ long holo_get_option(const char* name) {
   if (n == "grid_series") return t.grid_series ? 1 : 0;
   if (n == "grid_near") return t.grid_near ? 1 : 0;
   if (n == "grid_rows") return t.grid_rows ? 1 : 0;
+  if (n == "grid_pairs") return t.grid_pairs ? 1 : 0;
   if (n == "mc_lattice") return t.mc_lattice ? 1 : 0;
   if (n == "mc_passes") return t.mc_passes;
   return -1;

@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "holo_internal.hpp"
 #include "holo_math.hpp"
 
 namespace holo {
@@ -146,6 +147,19 @@ __device__ __forceinline__ void sincos_rev_f32(float t, float& s, float& c) {
 
 // ---------------------------------------------------------------------------
 // FP32-split helpers shared by the tiled and lattice kernels.
+
+// The FP32 weight (re, im) of source n: polar (wf = kPolar: amplitudes w0, phases
+// w1) or interleaved complex w0; 0 for a padding slot (n < 0).
+__device__ __forceinline__ float2 slot_weight(int wf, const double* __restrict__ w0,
+                                              const double* __restrict__ w1, int32_t n) {
+  if (n < 0) return make_float2(0.f, 0.f);
+  if (wf == kPolar) {
+    double sn, cs;
+    sincos(w1[n], &sn, &cs);
+    return make_float2((float)(w0[n] * cs), (float)(w0[n] * sn));
+  }
+  return make_float2((float)w0[2 * (size_t)n], (float)w0[2 * (size_t)n + 1]);
+}
 
 // One pair of the FP32-split formulation from its squared distance s and
 // axial offset dz: d (to a few 1e-15, not always correctly rounded) and the

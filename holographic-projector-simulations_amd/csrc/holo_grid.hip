@@ -49,14 +49,13 @@
 
 #include "holo_device.hpp"
 #include "holo_internal.hpp"
+#include "holo_weights.hpp"
 
 namespace holo {
 
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 
-constexpr int kGridWaves = kBlock / 64;
 constexpr int kGridFlush = 8;  // tiles summed in FP32 between FP64 flushes
 constexpr float kFourPi = 12.566370614359172f;
 
@@ -93,20 +92,6 @@ __device__ __forceinline__ bool grid_pairs_ok(float Pm, float Qm, float rx2, flo
   const float ampsep = kappa * kappa * Pm * Qm;
   return round_err <= kGuardCycles && trunc_err <= 0.05f * kGuardCycles && cross <= 1.5e-3f &&
          beta * rx2 * Qm <= 1e-6f && ampsep <= 1e-6f;
-}
-
-// x = hi + lo in f16: hi is x rounded to 11 significant bits (ties away from
-// zero) by integer arithmetic, so hi is exact in f16 for |x| >= 2^-14 and
-// every conversion instruction yields the same hi; lo = x - hi is exact in
-// FP32 and |lo| <= 2^-11 |x|.  (Splitting as lo = x - (float)(half)x is not
-// safe: the compiler may fold the product that made x into the f16
-// conversion -- one rounding instead of two -- for one use of hi and not for
-// another, and at exact ties hi + lo is then off by one f16 ulp.)
-__device__ __forceinline__ void split_f16(float x, _Float16& hi, _Float16& lo) {
-  const float h =
-      __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, x) + 0x1000u) & 0xffffe000u);
-  hi = (_Float16)h;
-  lo = (_Float16)(x - h);
 }
 
 // The GEMM's Y operand for one column, Y' = am (c, s) with am = 1 + kappa Q
@@ -419,11 +404,6 @@ hipError_t launch_superpose_grid(int sign, bool obliquity, const GridTiles& gt,
 // 8 rb + 2g, 8 rb + 2g + 1 for target j.
 
 constexpr int kGrid16Flush = 2;  // tiles summed in FP32 between FP64 flushes
-// f16 scales of the correction operands: the weight side carries k_a kCrossW W
-// (and k_a^2 kCross2W W), the column side the inverse, so that both sides stay
-// in f16's normal range from a few cm to about a metre.
-constexpr float kCrossW = 0x1p-4f;
-constexpr float kCross2W = 0x1p-8f;
 constexpr double kRowMid = 28.25;  // midpoint of k_a^2 over a tile's 16 rows
 constexpr float kRowDev = 28.f;    // largest |k_a^2 - kRowMid|
 
@@ -585,98 +565,17 @@ __device__ __forceinline__ void series_tile_pairs(const float2* __restrict__ w, 
   }
 }
 
-// MFMA operands of the 16 x 16 tiles' weights, one wave per tile: for row
-// block rb, wq[(6t + 3rb + q) * 64 + lane] holds, for lane l = 16 g + i,
-// row i = 2a' + c (a = 8 rb + a') and columns 4g .. 4g + 3 (re, im) of the real
-// form of W / tscale split into f16 hi (q = 0) and lo (q = 1), and of
-// i k_a kCrossW W / tscale (q = 2, its f16 hi part).  wqn (nullable), the
-// near-field GEMM's extra operands: wqn[(4t + 2rb + q) * 64 + lane] holds the
-// lo part of i k_a kCrossW W / tscale (q = 0) and k_a^2 kCross2W W / tscale in
-// the real form of W (q = 1).  wc: 256 slots per tile, slot 16 a + b.
-// group (1, 2 or 4): tiles group T .. group T + group - 1 (the halves of a
-// 16 x 32 tile, the quarters of a 16 x 64 one) share one tscale, the power of
-// two above the largest of their largest components.
-__global__ __launch_bounds__(kBlock) void k_grid16_weights(const float2* __restrict__ wc,
-                                                           uint32_t n_tiles, uint32_t group,
-                                                           uint4* __restrict__ wq,
-                                                           uint4* __restrict__ wqn,
-                                                           float* __restrict__ tscale) {
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t t = blockIdx.x * kGridWaves + (threadIdx.x >> 6);
-  if (t >= n_tiles) return;  // uniform per wave
-  const uint32_t i = lane & 15, g = lane >> 4, ap = i >> 1, co = i & 1;
-  float2 w[2][4];
-  float mx = 0.f;
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      w[rb][q] = wc[(size_t)t * 256 + 16 * (8 * rb + ap) + 4 * g + q];
-      mx = fmaxf(mx, fmaxf(fabsf(w[rb][q].x), fabsf(w[rb][q].y)));
-    }
-  for (uint32_t o = 1; o < group; ++o) {  // n_tiles is a multiple of group
-    const uint32_t tt = (t & ~(group - 1u)) | ((t + o) & (group - 1u));
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float2 x = wc[(size_t)tt * 256 + 16 * (8 * rb + ap) + 4 * g + q];
-        mx = fmaxf(mx, fmaxf(fabsf(x.x), fabsf(x.y)));
-      }
-  }
-  for (int off = 32; off; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-  int e = 0;
-  if (mx > 0.f && __builtin_isfinite(mx)) frexpf(mx, &e);
-  e = e < -126 ? -126 : (e > 127 ? 127 : e);
-  const float is = ldexpf(1.f, -e);
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
-    const float kr = (float)(8 * rb + ap) - 7.5f;
-    const float ka = kr * kCrossW, ka2 = kr * kr * kCross2W;
-    h8v hi, lo, cr, crl, c2;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float vr = w[rb][q].x * is, vi = w[rb][q].y * is;
-      // real form: rows (a, re) = (Vr, -Vi), (a, im) = (Vi, Vr)
-      const float A0 = co ? vi : vr, A1 = co ? vr : -vi;
-      // i k W: real part -k Wi, imaginary part k Wr
-      const float C0 = co ? ka * vr : -ka * vi, C1 = co ? -ka * vi : -ka * vr;
-      _Float16 h, l;
-      split_f16(A0, h, l);
-      hi[2 * q] = h;
-      lo[2 * q] = l;
-      split_f16(A1, h, l);
-      hi[2 * q + 1] = h;
-      lo[2 * q + 1] = l;
-      split_f16(C0, h, l);
-      cr[2 * q] = h;
-      crl[2 * q] = l;
-      split_f16(C1, h, l);
-      cr[2 * q + 1] = h;
-      crl[2 * q + 1] = l;
-      // k^2 W (real scaling): the same real form as W
-      c2[2 * q] = (_Float16)(ka2 * A0);
-      c2[2 * q + 1] = (_Float16)(ka2 * A1);
-    }
-    wq[((size_t)t * 6 + 3 * rb + 0) * 64 + lane] = __builtin_bit_cast(uint4, hi);
-    wq[((size_t)t * 6 + 3 * rb + 1) * 64 + lane] = __builtin_bit_cast(uint4, lo);
-    wq[((size_t)t * 6 + 3 * rb + 2) * 64 + lane] = __builtin_bit_cast(uint4, cr);
-    if (wqn) {
-      wqn[((size_t)t * 4 + 2 * rb + 0) * 64 + lane] = __builtin_bit_cast(uint4, crl);
-      wqn[((size_t)t * 4 + 2 * rb + 1) * 64 + lane] = __builtin_bit_cast(uint4, c2);
-    }
-  }
-  if (lane == 0) tscale[t] = ldexpf(1.f, e);
+__global__ __launch_bounds__(kBlock) void k_grid16_weights(Grid16Prep a,
+                                                           const uint32_t* __restrict__ skip) {
+  if (skip && *skip) return;
+  grid16_weights(a, blockIdx.x);
 }
 
-hipError_t launch_grid16_weights(const float2* wc, uint32_t n_tiles, int group, uint4* wq,
-                                 uint4* wqn, float* tscale, hipStream_t stream) {
-  if (!n_tiles) return hipSuccess;
-  if ((group != 1 && group != 2 && group != 4) || n_tiles % (uint32_t)group)
+hipError_t launch_grid16_weights(const Grid16Prep& a, hipStream_t stream, const uint32_t* skip) {
+  if (!a.n_tiles) return hipSuccess;
+  if ((a.group != 1 && a.group != 2 && a.group != 4) || a.n_tiles % a.group)
     return hipErrorInvalidValue;
-  const unsigned blocks = (n_tiles + kGridWaves - 1) / kGridWaves;
-  k_grid16_weights<<<blocks, kBlock, 0, stream>>>(wc, n_tiles, (uint32_t)group, wq, wqn,
-                                                  tscale);
+  k_grid16_weights<<<grid16_weight_blocks(a), kBlock, 0, stream>>>(a, skip);
   return hipGetLastError();
 }
 
@@ -1094,7 +993,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
     const double4* __restrict__ centre16, GridBounds gb16, const double* __restrict__ axes,
     LatticeAxes ax,
     const int32_t* __restrict__ tail_perm, const float2* __restrict__ tail_wc, uint32_t n_tail,
-    double2* __restrict__ out) {
+    const uint32_t* __restrict__ skip, double2* __restrict__ out) {
+  if (skip && *skip) return;
   __shared__ Grid16Lds lds;
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const uint32_t base = blockIdx.x * kBlock + wv * 64;
@@ -1156,7 +1056,8 @@ hipError_t launch_superpose_grid16(int sign, bool obliquity, int nkc, const Grid
                                    const float2* wc, const uint4* wq, const uint4* wqn,
                                    const float* tscale, const double* v, size_t M,
                                    double lambda, double2* y, double2* partial,
-                                   size_t partial_cap, hipStream_t stream) {
+                                   size_t partial_cap, hipStream_t stream,
+                                   const uint32_t* skip, int Sp) {
   if (M == 0) return hipSuccess;
   if (nkc != 1 && nkc != 2 && nkc != 4) return hipErrorInvalidValue;
   if (nkc > 1 && (halves.n_tiles != (uint32_t)nkc * gt.n_tiles || !halves.centre))
@@ -1192,21 +1093,22 @@ hipError_t launch_superpose_grid16(int sign, bool obliquity, int nkc, const Grid
         k_superpose_grid16<sg.value, (bool)obl.value, 4><<<grid, kBlock, 0, stream>>>(
             gt.centre, gt.perm, gt.u, wc, wq, wqn, tscale, gt.n_tiles, chunk, v, (uint32_t)M,
             il, gt.px, gt.py, gb, pairs.centre, gb32, halves.centre, gb16, axes, ax,
-            gt.tail_perm, gt.tail_wc, gt.n_tail, out);
+            gt.tail_perm, gt.tail_wc, gt.n_tail, skip, out);
       else if (nkc == 2)
         k_superpose_grid16<sg.value, (bool)obl.value, 2><<<grid, kBlock, 0, stream>>>(
             gt.centre, gt.perm, gt.u, wc, wq, wqn, tscale, gt.n_tiles, chunk, v, (uint32_t)M,
             il, gt.px, gt.py, gb, gt.centre, gb, halves.centre, gb16, axes, ax, gt.tail_perm,
-            gt.tail_wc, gt.n_tail, out);
+            gt.tail_wc, gt.n_tail, skip, out);
       else
         k_superpose_grid16<sg.value, (bool)obl.value, 1><<<grid, kBlock, 0, stream>>>(
             gt.centre, gt.perm, gt.u, wc, wq, wqn, tscale, gt.n_tiles, chunk, v, (uint32_t)M,
             il, gt.px, gt.py, gb, gt.centre, gb, gt.centre, gb, axes, ax, gt.tail_perm,
-            gt.tail_wc, gt.n_tail, out);
+            gt.tail_wc, gt.n_tail, skip, out);
     });
   });
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (skip) return launch_reduce_either(partial, skip, Sp, S, M, y, stream);
   return launch_reduce_partials(S, M, partial, y, stream);
 }
 

@@ -6,6 +6,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 namespace holo {
@@ -71,6 +72,7 @@ struct Tuning {
   bool grid_series = true; // 16-row kernels: near-field pairs by the q-series, not exactly
   bool grid_near = true;   // 16-row kernels: waves off the far-field bounds take the near-field GEMM
   bool grid_rows = true;   // 16-row kernels: exact pairs read row x's and column y's from tables
+  bool grid_pairs = true;  // 16-row kernels: lattice targets take the lattice-to-lattice kernel
   bool mc_lattice = true; // per-target FP32-split MC: table gather on product grids
   int mc_passes = 0;      // per-target MC: source ranges, one launch each (0 = automatic)
 };
@@ -171,8 +173,8 @@ hipError_t launch_superpose_grid(int sign, bool obliquity, const GridTiles& gt,
                                  double lambda, double2* y, double2* partial,
                                  size_t partial_cap, hipStream_t stream);
 // 16 x 16 tiles of a uniform lattice (pitches gt.px, gt.py; gt.goff unused):
-// wc holds 256 slots per tile (slot 16a + b), launch_grid16_weights lays them
-// out as wq (6 x 8 f16 per tile and lane), wqn (the near-field GEMM's 4 x 8 f16
+// launch_grid16_weights forms the weights wc, 256 slots per tile (slot 16a + b),
+// and those of n_tail slots after them, and lays the tiles' out as wq (6 x 8 f16 per tile and lane), wqn (the near-field GEMM's 4 x 8 f16
 // per tile and lane; nullable) and tscale; tiles group T .. group T + group - 1
 // share one tscale (group 1, 2 or 4).  launch_superpose_grid16 with nkc = 1
 // takes the 16 x 16 tiles gt (pairs and halves unused); with nkc = 2 it takes
@@ -185,18 +187,80 @@ hipError_t launch_superpose_grid(int sign, bool obliquity, const GridTiles& gt,
 // same sources as 16 x 32 tiles (2 gt.n_tiles) and halves as 16 x 16 tiles
 // (4 gt.n_tiles): a wave failing the 16 x 64 bounds takes the 16 x 32 tiles if
 // it passes theirs, else the 16 x 16 ones.
-hipError_t launch_grid16_weights(const float2* wc, uint32_t n_tiles, int group, uint4* wq,
-                                 uint4* wqn, float* tscale, hipStream_t stream);
+// skip (nullable, device): nonzero makes the launch do nothing.
+struct Grid16Prep {
+  int wf = 0;
+  const double* w0 = nullptr;
+  const double* w1 = nullptr;
+  const int32_t* perm = nullptr;
+  uint32_t n_tiles = 0, n_tail = 0, group = 1;
+  float2* wc = nullptr;
+  uint4* wq = nullptr;
+  uint4* wqn = nullptr;
+  float* tscale = nullptr;
+};
+// workgroups of 4 tiles, then of 256 tail slots
+inline unsigned grid16_weight_blocks(const Grid16Prep& a) {
+  return (a.n_tiles + 3) / 4 + (a.n_tail + 255) / 256;
+}
+hipError_t launch_grid16_weights(const Grid16Prep& a, hipStream_t stream,
+                                 const uint32_t* skip = nullptr);
 // wqn null: no near-field GEMM (the waves off the far-field bounds take the
-// series and exact paths per (target, tile))
+// series and exact paths per (target, tile)).  skip (nullable): nonzero when
+// the lattice-to-lattice kernel has done the call in Sp splits (in `partial`
+// when Sp > 1), which are then the ones summed into y.
 hipError_t launch_superpose_grid16(int sign, bool obliquity, int nkc, const GridTiles& gt,
                                    const GridTiles& pairs, const GridTiles& halves,
                                    const float2* wc, const uint4* wq, const uint4* wqn,
                                    const float* tscale, const double* v, size_t M,
                                    double lambda, double2* y, double2* partial,
-                                   size_t partial_cap, hipStream_t stream);
+                                   size_t partial_cap, hipStream_t stream,
+                                   const uint32_t* skip = nullptr, int Sp = 1);
 // Source splits the lattice kernel uses for M targets over n_tiles tiles.
 int grid_splits(size_t M, size_t n_tiles);
+
+// Lattice-to-lattice kernel (holo_pairs.hip): the sources of a uniform lattice
+// x0 + i px, y0 + j py, z (n = i ny + j, i < nx, j < ny), cut into 32 x 64 tiles
+// (tj per row of tiles), followed by n_tail others (tail_perm: their indices;
+// tail_same: all at one point).  wq: 16 x 64 uint4 per tile, tscale: one float
+// per tile, tail_wc: n_tail float2, all written by each launch.
+struct PairPlan {
+  double x0 = 0, y0 = 0, z = 0, px = 0, py = 0;
+  uint32_t nx = 0, ny = 0, tj = 0, n_tiles = 0, n_tail = 0;
+  bool tail_same = false;
+  const double* u = nullptr;
+  const int32_t* tail_perm = nullptr;
+  uint4* wq = nullptr;
+  float* tscale = nullptr;
+  float2* tail_wc = nullptr;
+};
+
+// The lattice of a call's targets as found on the device (x_0 + i p_x, y_0 +
+// j p_y, z, then copies of target 0), and the form the kernel takes (0: not a
+// lattice within the kernel's bounds).
+struct PairTargets {
+  double x0, y0, z, px, py;
+  uint32_t nx, ny, mode;
+};
+constexpr size_t kPairFlags = 256;  // words: one per workgroup that checks targets
+// Smallest call: both sides of the targets' lattice are at least 16 (a 16 x 17
+// lattice to 18 x 16 targets takes as long as on the 16-row kernels, 39 and 41 us;
+// thinner lattices would mostly be padding).
+constexpr size_t kPairMinTargets = 256;
+int pair_splits(size_t M, size_t n_tiles);
+// Launches the weights' and targets' preparation and the kernel (with, where
+// grid16 is given, the 16-row kernels' weights in the same launch): *handled
+// (device) becomes 1 and out holds the S splits' sums (S M double2; y itself when S = 1),
+// or 0 and out is untouched.
+hipError_t launch_superpose_pairs(int sign, bool obliquity, const PairPlan& pp, WeightForm wf,
+                                  const double* w0, const double* w1, const double* v, size_t M,
+                                  double lambda, int S, PairTargets* pt, uint32_t* flags,
+                                  uint32_t* handled, double2* out, const Grid16Prep* grid16,
+                                  hipStream_t stream);
+// y = the sum of partial's Sp splits when *handled, else of its Sg splits
+// (nothing where that is one: y holds the result).
+hipError_t launch_reduce_either(const double2* partial, const uint32_t* handled, int Sp, int Sg,
+                                size_t M, double2* y, hipStream_t stream);
 
 // wc[slot] = a e^{i phi} (polar input) or w (cartesian input) of source
 // perm[slot] as (re, im); with polar_out as (|w|, arg w / 2 pi in [-1/2, 1/2)).

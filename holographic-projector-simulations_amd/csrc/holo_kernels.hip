@@ -558,27 +558,22 @@ __global__ __launch_bounds__(kBlock) void k_tile_weights(
   if (s >= n_slots) return;
   const int32_t n = perm[s];
   float2 r = make_float2(0.f, 0.f);
-  if (n >= 0) {
+  if (!polar_out) {
+    r = slot_weight(wf, w0, w1, n);
+  } else if (n >= 0) {
+    // (|w|, arg w in cycles, reduced to [-1/2, 1/2))
     constexpr double kInv2Pi = 0.15915494309189535;
-    if (polar_out) {  // (|w|, arg w in cycles, reduced to [-1/2, 1/2))
-      double a, t;
-      if (wf == kPolar) {
-        a = w0[n];
-        t = w1[n] * kInv2Pi + (a < 0.0 ? 0.5 : 0.0);
-        a = __builtin_fabs(a);
-      } else {
-        const double re = w0[2 * (size_t)n], im = w0[2 * (size_t)n + 1];
-        a = hypot(re, im);
-        t = atan2(im, re) * kInv2Pi;
-      }
-      r = make_float2((float)a, (float)(t - __builtin_rint(t)));
-    } else if (wf == kPolar) {
-      double sn, cs;
-      sincos(w1[n], &sn, &cs);
-      r = make_float2((float)(w0[n] * cs), (float)(w0[n] * sn));
+    double a, t;
+    if (wf == kPolar) {
+      a = w0[n];
+      t = w1[n] * kInv2Pi + (a < 0.0 ? 0.5 : 0.0);
+      a = __builtin_fabs(a);
     } else {
-      r = make_float2((float)w0[2 * (size_t)n], (float)w0[2 * (size_t)n + 1]);
+      const double re = w0[2 * (size_t)n], im = w0[2 * (size_t)n + 1];
+      a = hypot(re, im);
+      t = atan2(im, re) * kInv2Pi;
     }
+    r = make_float2((float)a, (float)(t - __builtin_rint(t)));
   }
   wc[s] = r;
 }

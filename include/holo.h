@@ -130,7 +130,7 @@ holo_status holo_synchronize(holo_ctx *ctx);
  * 1 = one launch), "mc_lattice" (0/1: per-target
  * FP32-split Monte Carlo on product-grid sources reads positions from row
  * and column tables; same results; default 1).  Results do not depend on them beyond summation order and, for "grid",
- * "grid16", "grid32" and "grid64", the FP32-split rounding (all paths stay within
+ * "grid16", "grid32", "grid64" and "grid_pairs", the FP32-split rounding (all paths stay within
  * ~1e-6).  Replaces the blockDim/gridDim/thread_size/n_streams hints of
  * cuda/input.h:116-122. */
 holo_status holo_set_option(const char *name, long value);
