@@ -82,7 +82,6 @@ struct holo_ctx {
   // staging buffers for host-pointer calls and scratch
   DevBuf amp, phase, u, v, y, w, partial, small, b, pos, ph;
   DevBuf mc_wc, mc_xy, mc_info;  // product-grid Monte Carlo (McLattice)
-  DevBuf layout;                 // source layout of device-pointer FP64 calls
   DevBuf pairs;                  // lattice-to-lattice kernel: target lattice, flags, outcome
   DevBuf errb;                   // error report: subset, FP64 values, partials
   DevBuf pos64, ph64;            // FP64 Monte Carlo records for the error report
@@ -158,17 +157,15 @@ struct holo_plan {
 namespace {
 
 // ---- scratch of holo_transform_full_noalloc --------------------------------
-// The split partials and source-layout words of the no-allocation entry point
-// live in this file-scope device array: one copy per device, allocated when
+// The split partials of the no-allocation entry point live in this file-scope
+// device array: one copy per device, allocated when
 // the code object loads on that device and held until the process ends.  In
 // host code `scratch` names a host-side stand-in, not device memory: kernels
 // and copies get the address hipGetSymbolAddress returns for the current
 // device, kept per device in g_scratch.
 constexpr size_t kNoallocScratchBytes = HOLO_NOALLOC_SCRATCH_BYTES;
-constexpr size_t kNoallocLayoutBytes = 256;  // 4 layout words, padded
 constexpr int kMaxDevices = 64;
-static_assert(kNoallocScratchBytes % 256 == 0 && kNoallocScratchBytes > kNoallocLayoutBytes,
-              "scratch size");
+static_assert(kNoallocScratchBytes % 256 == 0, "scratch size");
 __device__ __align__(256) unsigned char scratch[kNoallocScratchBytes];
 
 std::mutex g_scratch_mu;
@@ -323,9 +320,11 @@ holo_status report_error(holo_ctx* ctx, bool fp64, const double* v, size_t M, co
   return HOLO_OK;
 }
 
+// Partial values of an FP64 launch with source splits, at most (1 GiB).
+constexpr size_t kMaxPartial = size_t(1) << 26;
+
 size_t split_elems_f64(size_t M, size_t N) {
-  const int R = holo::tuning().r_f64;
-  const int S = N ? holo::choose_splits(M, R == 1 || R == 4 ? R : 2, N, 1024) : 1;
+  const int S = holo::f64_shape(M, N, kMaxPartial).S;
   return S > 1 ? (size_t)S * M : 0;
 }
 
@@ -1334,11 +1333,9 @@ holo_status holo_transform_full(holo_ctx* ctx, holo_precision precision, int sig
     const double K = (2 * M_PI) / lambda;  // TWO_PI_OVER_LAMBDA, cuda/macros.h:29-31
     if (dev && !holo::tuning().f64_libm) {
       // device positions: their layout is found on the device
-      HOLO_TRY(ensure(ctx->layout, 4 * sizeof(uint32_t), ctx->device));
       HOLO_HIP(holo::launch_superpose_f64_auto(
           sign, holo::kPolar, obl, da, dp, du, N, dv, M, K, reinterpret_cast<double2*>(dy),
-          static_cast<double2*>(ctx->partial.ptr), pe, static_cast<uint32_t*>(ctx->layout.ptr),
-          ctx->stream));
+          static_cast<double2*>(ctx->partial.ptr), pe, ctx->stream));
     } else {
       const bool uz = !dev && uniform_z(u, N);
       const size_t row = uz ? row_length(u, N) : 0;
@@ -1383,14 +1380,12 @@ holo_status holo_transform_full_noalloc(int sign, double lambda, const double* a
     HOLO_HIP(holo::launch_zero(y, 2 * M, st));
     return HOLO_OK;
   }
-  uint32_t* layout = static_cast<uint32_t*>(base);
-  double2* partial =
-      reinterpret_cast<double2*>(static_cast<unsigned char*>(base) + kNoallocLayoutBytes);
-  const size_t cap = (kNoallocScratchBytes - kNoallocLayoutBytes) / sizeof(double2);
+  double2* partial = static_cast<double2*>(base);
+  const size_t cap = kNoallocScratchBytes / sizeof(double2);
   const double K = (2 * M_PI) / lambda;  // TWO_PI_OVER_LAMBDA, cuda/macros.h:29-31
   HOLO_HIP(holo::launch_superpose_f64_auto(sign, holo::kPolar, flags & HOLO_OBLIQUITY, amp,
                                            phase, u, N, v, M, K, reinterpret_cast<double2*>(y),
-                                           partial, cap, layout, st));
+                                           partial, cap, st));
   return HOLO_OK;
 }
 

@@ -145,6 +145,29 @@ __device__ __forceinline__ void sincos_rev_f32(float t, float& s, float& c) {
   c = __builtin_amdgcn_cosf(t);
 }
 
+// sum of p[0], p[M], .. p[(S - 1) M], in order (deterministic)
+__device__ __forceinline__ double2 sum_splits(const double2* __restrict__ p, uint32_t S,
+                                              uint32_t M) {
+  double re = 0.0, im = 0.0;
+  uint32_t s = 0;
+  for (; s + 8 <= S; s += 8) {
+    double2 v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = p[(size_t)(s + q) * M];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      re += v[q].x;
+      im += v[q].y;
+    }
+  }
+  for (; s < S; ++s) {
+    const double2 v = p[(size_t)s * M];
+    re += v.x;
+    im += v.y;
+  }
+  return make_double2(re, im);
+}
+
 // ---------------------------------------------------------------------------
 // FP32-split helpers shared by the tiled and lattice kernels.
 

@@ -58,7 +58,7 @@ struct GridTiles {
 };
 
 struct Tuning {
-  int r_f64 = 4;          // targets per lane, FP64 kernel (1, 2, 4)
+  int r_f64 = 4;          // targets per lane, FP64 kernel (1, 2, 4), at most
   int r_f32 = 2;          // targets per lane, FP32-split kernel (1, 2, 4)
   int splits = 0;         // source splits (0 = automatic)
   int target_waves = 16384;
@@ -112,6 +112,12 @@ inline void with_r(int R, F&& f) {
 int choose_splits(size_t M, int R, size_t units, size_t min_units_per_split,
                   size_t max_splits = 64);
 
+// Targets per lane and source splits of an FP64 launch.
+struct F64Shape {
+  int R, S;
+};
+F64Shape f64_shape(size_t M, size_t N, size_t cap);
+
 // Source splits of a launch over a few hundred targets (the error report's
 // subset): enough workgroups to fill the 256 CUs.
 constexpr size_t kFewTargetSplits = 1024;
@@ -134,20 +140,12 @@ hipError_t launch_superpose_f64(int sign, WeightForm wf, bool obliquity, bool un
                                 bool few_targets = false);
 
 // The same sum for sources whose layout the host has not scanned (device
-// pointers): launch_source_layout writes it to `layout` (4 words of device
-// memory) and the kernel reads it there, taking the uniform-z and rows paths
-// of launch_superpose_f64 where they apply (the same bits).
+// pointers): the kernel finds it and takes the uniform-z and rows paths of
+// launch_superpose_f64 where they apply (the same bits).
 hipError_t launch_superpose_f64_auto(int sign, WeightForm wf, bool obliquity,
                                      const double* w0, const double* w1, const double* u,
                                      size_t N, const double* v, size_t M, double K, double2* y,
-                                     double2* partial, size_t partial_cap, uint32_t* layout,
-                                     hipStream_t stream);
-// layout[0] bit 0: every source has the z of source 0; bit 1: rows of
-// layout[1] (>= 4) consecutive sources that share one x, the last row
-// possibly shorter; the same rules as the host scan.  Bits not in `allow`
-// stay clear.
-hipError_t launch_source_layout(const double* u, size_t N, uint32_t* layout,
-                                hipStream_t stream, unsigned allow = 3u);
+                                     double2* partial, size_t partial_cap, hipStream_t stream);
 
 // y[m] = sum_s partial[s*M + m] in fixed order (nothing to do for S <= 1).
 hipError_t launch_reduce_partials(int S, size_t M, const double2* partial, double2* y,

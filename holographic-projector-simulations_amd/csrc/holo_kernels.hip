@@ -26,6 +26,21 @@ Tuning& tuning() {
   return t;
 }
 
+// f64_shape's estimates, in ns, from sweeps of R and S over 1e6 .. 4e10 pairs
+// (lattice sources; within 5 % of the measured times from 2e8 pairs up).  A SIMD
+// that takes c waves one after the other or together needs w (c + k), w = a wave's
+// pairs at kF64Pair[R] each and k the last wave's latency that nothing hides; c is
+// the largest count of workgroups per CU.  A workgroup loads the sin/cos table
+// (kF64Start), and a split writes partial values that a reduction reads.
+struct F64Cost {
+  int R;
+  double pair, k;
+};
+constexpr F64Cost kF64Cost[] = {{4, 58.5, 0.475}, {2, 59.4, 0.75}, {1, 62.6, 1.62}};
+constexpr double kF64Start = 1500, kF64Reduce = 3000, kF64Partial = 0.008;
+constexpr size_t kF64Cus = 256, kF64Resident = 5;
+constexpr size_t kF64MinSources = 32;  // per split
+
 int choose_splits(size_t M, int R, size_t units, size_t min_units, size_t max_splits) {
   const Tuning& tu = tuning();
   if (tu.splits > 0) return (int)std::min<size_t>(tu.splits, std::max<size_t>(units, 1));
@@ -37,19 +52,56 @@ int choose_splits(size_t M, int R, size_t units, size_t min_units, size_t max_sp
   return (int)std::max<size_t>(S, 1);
 }
 
+// 1024 sources on 4096 targets: 367 us as 4 workgroups, 15 us by this rule; 7680 on
+// 30000: 499 and 270 us; 65536 on 262144: 15.7 ms (16 splits) and 15.1 - 15.7 ms.
+// Launch shape of the FP64 kernel: the targets per lane R (at most r_f64) and source
+// splits S of the smallest estimated time, S M at most `cap` partial values (unless
+// S = 1).  With `splits` set by the caller R = r_f64 and S = splits.
+F64Shape f64_shape(size_t M, size_t N, size_t cap) {
+  const Tuning& tu = tuning();
+  const int top = tu.r_f64 == 1 || tu.r_f64 == 4 ? tu.r_f64 : 2;
+  F64Shape best{top, 1};
+  if (N == 0 || M == 0) return best;
+  if (tu.splits > 0) {
+    best.S = (int)std::min<size_t>((size_t)tu.splits, N);
+    while (best.S > 1 && (size_t)best.S * M > cap) --best.S;
+    return best;
+  }
+  double least = 1e300;
+  for (const F64Cost& f : kF64Cost) {
+    if (f.R > top) continue;
+    const size_t tb = (M + (size_t)kBlock * f.R - 1) / ((size_t)kBlock * f.R);
+    for (const int S : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 40, 48, 64, 96, 128}) {
+      const size_t blocks = tb * (size_t)S, c = (blocks + kF64Cus - 1) / kF64Cus;
+      if (S > 1 && ((size_t)S * M > cap || N < (size_t)S * kF64MinSources ||
+                    blocks > (size_t)tu.target_waves))
+        break;
+      const double w = (double)((N + S - 1) / S) * f.R * f.pair;
+      double t = w * ((double)c + f.k) + kF64Start * (double)((c + kF64Resident - 1) / kF64Resident);
+      if (S > 1) t += kF64Reduce + (double)S * (double)M * kF64Partial;
+      if (t < least) {
+        least = t;
+        best = F64Shape{f.R, S};
+      }
+    }
+  }
+  return best;
+}
+
 // ---------------------------------------------------------------------------
 // FP64 brute force.
 
 // PZ: every source has the z of source 0, so dz = vz - uz is formed once per
 // target (the same bits as per pair).
-// ROWS (with PZ): the sources come in rows of `row` consecutive sources that
-// share one x (a lattice in x-slow order, cuda/init.h:89-158), so dx^2 is
-// formed once per (target, row): again the same bits as per pair.
+// ROWS (with PZ): from source `first` on, the sources come in rows of `row`
+// consecutive sources that share one x, and those before it (of this split) share
+// one too (a lattice in x-slow order, cuda/init.h:89-158), so dx^2 is formed once
+// per (target, row): again the same bits as per pair.
 // s_tab: the sin/cos table, already in LDS.
 template <int SIGN, int R, int WF, int MATH, bool OBL, bool PZ, bool ROWS>
 __device__ __forceinline__ void superpose_f64_body(
     const double* __restrict__ w0, const double* __restrict__ w1,
-    const double* __restrict__ u, uint32_t N, uint32_t chunk, uint32_t row,
+    const double* __restrict__ u, uint32_t N, uint32_t chunk, uint32_t first, uint32_t row,
     const double* __restrict__ v, uint32_t M, double K,
     double2* __restrict__ out, const double* s_tab) {
   static_assert(!ROWS || PZ, "rows need sources in one plane");
@@ -69,7 +121,7 @@ __device__ __forceinline__ void superpose_f64_body(
   }
   double dz0[R];
 #pragma unroll
-  for (int r = 0; r < R; ++r) dz0[r] = PZ && N ? vz[r] - u[2] : 0.0;
+  for (int r = 0; r < R; ++r) dz0[r] = PZ && n0 < n1 ? vz[r] - u[3 * (size_t)n0 + 2] : 0.0;
   // sources [a, b); with ROWS their dx^2 per target is dxx
   auto sources = [&](uint32_t a, uint32_t b, const double(&dxx)[R]) {
     for (uint32_t n = a; n < b; ++n) {
@@ -116,7 +168,8 @@ __device__ __forceinline__ void superpose_f64_body(
   };
   if constexpr (ROWS) {
     for (uint32_t n = n0; n < n1;) {
-      const uint32_t e = min(n1, (n / row + 1) * row);  // end of n's row
+      // end of n's row
+      const uint32_t e = min(n1, n < first ? first : first + ((n - first) / row + 1) * row);
       const double ux = u[3 * (size_t)n];
       double dxx[R];
 #pragma unroll
@@ -158,96 +211,106 @@ __global__ __launch_bounds__(kBlock) void k_superpose_f64(
     double2* __restrict__ out) {
   __shared__ double s_tab[kTab];
   load_sincos_table(s_tab);
-  superpose_f64_body<SIGN, R, WF, MATH, OBL, PZ, ROWS>(w0, w1, u, N, chunk, row, v, M, K, out,
-                                                        s_tab);
+  superpose_f64_body<SIGN, R, WF, MATH, OBL, PZ, ROWS>(w0, w1, u, N, chunk, 0u, row, v, M, K,
+                                                        out, s_tab);
 }
 
-// The same sum with the source layout read from device memory (written by
-// launch_source_layout): layout[0] bit 0 = every source has the z of source
-// 0, bit 1 = rows of layout[1] sources with one x.  The branch is uniform over
-// the launch, and every branch gives the same bits.
+// The same sum for sources whose layout the host has not scanned (device
+// pointers; the host-pointer and plan paths scan the positions on the host): every
+// workgroup looks at the sources of its own split first, which takes a few loads a
+// lane against 60 ns per source and target of a wave, and no launch.
+// allow: bit 0 = look for one z, bit 1 = look for rows too.  Returns 3 (one z, and
+// rows of at least 4 from `first`, the last one possibly shorter), 1 (one z) or 0.
+// s_w: 4 words of LDS.
+__device__ uint32_t split_layout(const double* __restrict__ u, uint32_t n0, uint32_t n1,
+                                 uint32_t allow, uint32_t* s_w, uint32_t& first,
+                                 uint32_t& row) {
+  first = row = n1;
+  if (!(allow & 1u) || n0 >= n1) return 0u;
+  if (threadIdx.x < 4) s_w[threadIdx.x] = threadIdx.x < 2 ? n1 : 0u;
+  __syncthreads();
+  const double x0 = u[3 * (size_t)n0], z0 = u[3 * (size_t)n0 + 2];
+  bool planar = true;
+  uint32_t hit = n1;  // the first source with another x
+  for (uint32_t n = n0 + threadIdx.x; n < n1; n += kBlock) {
+    planar = planar && u[3 * (size_t)n + 2] == z0;
+    if (hit == n1 && u[3 * (size_t)n] != x0) hit = n;
+  }
+  if (hit < n1) atomicMin(&s_w[0], hit);
+  if (!planar) s_w[2] = 1u;
+  __syncthreads();
+  if (s_w[2]) return 0u;
+  if (!(allow & 2u)) return 1u;
+  first = __builtin_amdgcn_readfirstlane(s_w[0]);  // (scalar: the loops' bounds)
+  if (first == n1) return 3u;  // one x
+  const double x1 = u[3 * (size_t)first];
+  for (uint32_t n = first + threadIdx.x; n < n1; n += kBlock)
+    if (u[3 * (size_t)n] != x1) {
+      atomicMin(&s_w[1], n);
+      break;
+    }
+  __syncthreads();
+  row = __builtin_amdgcn_readfirstlane(s_w[1]) - first;
+  bool rows = row >= 4;
+  if (rows)
+    for (uint32_t n = first + threadIdx.x; n < n1; n += kBlock)
+      rows = rows && u[3 * (size_t)n] == u[3 * (size_t)(n - (n - first) % row)];
+  if (!rows) s_w[3] = 1u;
+  __syncthreads();
+  return s_w[3] ? 1u : 3u;
+}
+
+// The branch is uniform over the workgroup, and every branch gives the same bits.
+// 98 VGPRs, 4 waves a SIMD: held to 96 for 5 it was up to 3 % slower.
 template <int SIGN, int R, int WF, bool OBL>
 __global__ __launch_bounds__(kBlock) void k_superpose_f64_auto(
     const double* __restrict__ w0, const double* __restrict__ w1,
-    const double* __restrict__ u, uint32_t N, uint32_t chunk,
-    const uint32_t* __restrict__ layout, const double* __restrict__ v, uint32_t M, double K,
-    double2* __restrict__ out) {
-  __shared__ double s_tab[kTab];
+    const double* __restrict__ u, uint32_t N, uint32_t chunk, uint32_t allow,
+    const double* __restrict__ v, uint32_t M, double K, double2* __restrict__ out) {
+  __shared__ double s_tab[kTab];  // 32 KB: with any more LDS only 4 workgroups fit a CU
+  uint32_t first, row;
+  const uint32_t n0 = min(N, blockIdx.y * chunk);
+  const uint32_t mode = split_layout(u, n0, min(N, n0 + chunk), allow,
+                                     reinterpret_cast<uint32_t*>(s_tab), first, row);
+  __syncthreads();
   load_sincos_table(s_tab);
-  const uint32_t mode = layout[0], row = layout[1];
-  if ((mode & 3u) == 3u)
-    superpose_f64_body<SIGN, R, WF, 0, OBL, true, true>(w0, w1, u, N, chunk, row, v, M, K, out,
-                                                        s_tab);
-  else if (mode & 1u)
-    superpose_f64_body<SIGN, R, WF, 0, OBL, true, false>(w0, w1, u, N, chunk, 0u, v, M, K, out,
-                                                         s_tab);
+  if (mode == 3u)
+    superpose_f64_body<SIGN, R, WF, 0, OBL, true, true>(w0, w1, u, N, chunk, first, row, v, M, K,
+                                                        out, s_tab);
+  else if (mode == 1u)
+    superpose_f64_body<SIGN, R, WF, 0, OBL, true, false>(w0, w1, u, N, chunk, 0u, 0u, v, M, K,
+                                                         out, s_tab);
   else
-    superpose_f64_body<SIGN, R, WF, 0, OBL, false, false>(w0, w1, u, N, chunk, 0u, v, M, K,
+    superpose_f64_body<SIGN, R, WF, 0, OBL, false, false>(w0, w1, u, N, chunk, 0u, 0u, v, M, K,
                                                           out, s_tab);
 }
 
-// Source layout on the device, for calls on device pointers (the host-pointer
-// and plan paths scan the positions on the host with the same rules):
-//   layout[0] bit 0: every z equals source 0's (== on values);
-//   layout[0] bit 1: the sources form rows of L = layout[1] consecutive
-//   sources that share the row's first x (L = the run of source 0's x, at
-//   least 4; the last row may be shorter);
-//   layout[1]: L.
-__global__ __launch_bounds__(kBlock) void k_layout_init(uint32_t N, uint32_t allow,
-                                                        uint32_t* __restrict__ layout) {
-  if (threadIdx.x == 0) {
-    layout[0] = allow;
-    layout[1] = N;
-  }
-}
-
-// L = the first n with x_n != x_0 (N if none): an atomic minimum, order-free.
-__global__ __launch_bounds__(kBlock) void k_layout_run(const double* __restrict__ u, uint32_t N,
-                                                       uint32_t* __restrict__ layout) {
-  const double x0 = u[0];
-  for (uint32_t n = blockIdx.x * kBlock + threadIdx.x; n < N; n += gridDim.x * kBlock)
-    if (u[3 * (size_t)n] != x0) {  // this thread's first hit is its smallest
-      atomicMin(&layout[1], n);
-      break;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_layout_check(const double* __restrict__ u,
-                                                         uint32_t N,
-                                                         uint32_t* __restrict__ layout) {
-  const uint32_t L = layout[1];
-  const double z0 = u[2];
-  bool planar = true, rows = L >= 4;
-  for (uint32_t n = blockIdx.x * kBlock + threadIdx.x; n < N; n += gridDim.x * kBlock) {
-    planar = planar && u[3 * (size_t)n + 2] == z0;
-    rows = rows && u[3 * (size_t)n] == u[3 * (size_t)(n - n % L)];
-  }
-  const uint32_t clear = (planar ? 0u : 3u) | (rows ? 0u : 2u);
-  if (clear) atomicAnd(&layout[0], ~clear);
-}
-
-hipError_t launch_source_layout(const double* u, size_t N, uint32_t* layout,
-                                hipStream_t stream, unsigned allow) {
-  k_layout_init<<<1, kBlock, 0, stream>>>((uint32_t)N, allow, layout);
-  if (!N) return hipGetLastError();
-  const unsigned blocks = (unsigned)std::min<size_t>((N + kBlock - 1) / kBlock, 2048);
-  k_layout_run<<<blocks, kBlock, 0, stream>>>(u, (uint32_t)N, layout);
-  k_layout_check<<<blocks, kBlock, 0, stream>>>(u, (uint32_t)N, layout);
-  return hipGetLastError();
-}
-
+// One thread per target, the splits in order, eight loads in flight.
 __global__ __launch_bounds__(kBlock) void k_reduce_partials(
     const double2* __restrict__ partial, uint32_t S, uint32_t M,
     double2* __restrict__ y) {
   const uint32_t m = blockIdx.x * kBlock + threadIdx.x;
-  if (m >= M) return;
-  double re = 0.0, im = 0.0;
-  for (uint32_t s = 0; s < S; ++s) {  // fixed order: deterministic
-    const double2 p = partial[(size_t)s * M + m];
-    re += p.x;
-    im += p.y;
+  if (m < M) y[m] = sum_splits(partial + m, S, M);
+}
+
+// Fewer targets than fill the GPU: 32 targets by 8 ranges of splits per workgroup,
+// each range summed in order, then the ranges.
+__global__ __launch_bounds__(kBlock) void k_reduce_partials_few(
+    const double2* __restrict__ partial, uint32_t S, uint32_t M, double2* __restrict__ y) {
+  __shared__ double2 s_part[8][32];
+  const uint32_t t = threadIdx.x & 31, q = threadIdx.x >> 5;
+  const uint32_t m = blockIdx.x * 32 + t;
+  const uint32_t a = q * S / 8, b = (q + 1) * S / 8;
+  if (m < M) s_part[q][t] = sum_splits(partial + (size_t)a * M + m, b - a, M);
+  __syncthreads();
+  if (q == 0 && m < M) {
+    double2 r = s_part[0][t];
+    for (int k = 1; k < 8; ++k) {
+      r.x += s_part[k][t].x;
+      r.y += s_part[k][t].y;
+    }
+    y[m] = r;
   }
-  y[m] = make_double2(re, im);
 }
 
 // Few targets over many splits (the error report's 256 targets over up to
@@ -278,12 +341,21 @@ __global__ __launch_bounds__(kBlock) void k_reduce_partials_wide(
   if (t == 0) y[m] = make_double2(s_re[0], s_im[0]);
 }
 
+// Up to this many targets one thread each leaves most of the GPU idle (30000
+// targets, 64 splits: 17.9 us; by ranges 5.5 us).
+constexpr size_t kReduceFew = 131072;
+
 hipError_t launch_reduce_partials(int S, size_t M, const double2* partial, double2* y,
                                   hipStream_t stream) {
   if (S <= 1 || M == 0) return hipSuccess;
   if (M <= 4096 && S >= 64) {
     k_reduce_partials_wide<<<(unsigned)M, kBlock, 0, stream>>>(partial, (uint32_t)S,
                                                                (uint32_t)M, y);
+    return hipGetLastError();
+  }
+  if (M <= kReduceFew && S >= 8) {
+    k_reduce_partials_few<<<(unsigned)((M + 31) / 32), kBlock, 0, stream>>>(
+        partial, (uint32_t)S, (uint32_t)M, y);
     return hipGetLastError();
   }
   const unsigned blocks = (unsigned)((M + kBlock - 1) / kBlock);
@@ -299,10 +371,12 @@ hipError_t launch_superpose_f64(int sign, WeightForm wf, bool obliquity, bool un
                                 double2* y, double2* partial,
                                 size_t partial_cap, hipStream_t stream, bool few_targets) {
   if (M == 0) return hipSuccess;
-  int R = few_targets ? 1 : tuning().r_f64;
-  if (R != 1 && R != 2 && R != 4) R = 2;
-  int S = N ? choose_splits(M, R, N, 1024, few_targets ? kFewTargetSplits : 64) : 1;
-  while (S > 1 && (size_t)S * M > partial_cap) --S;
+  F64Shape shape = f64_shape(M, N, partial_cap);
+  if (few_targets) {
+    shape = F64Shape{1, N ? choose_splits(M, 1, N, 128, kFewTargetSplits) : 1};
+    while (shape.S > 1 && (size_t)shape.S * M > partial_cap) --shape.S;
+  }
+  const int R = shape.R, S = shape.S;
   const uint32_t chunk = N ? (uint32_t)((N + S - 1) / S) : 0;
   const dim3 grid((unsigned)((M + (size_t)kBlock * R - 1) / ((size_t)kBlock * R)),
                   (unsigned)S);
@@ -339,17 +413,13 @@ hipError_t launch_superpose_f64(int sign, WeightForm wf, bool obliquity, bool un
 hipError_t launch_superpose_f64_auto(int sign, WeightForm wf, bool obliquity,
                                      const double* w0, const double* w1, const double* u,
                                      size_t N, const double* v, size_t M, double K, double2* y,
-                                     double2* partial, size_t partial_cap, uint32_t* layout,
+                                     double2* partial, size_t partial_cap,
                                      hipStream_t stream) {
   if (M == 0) return hipSuccess;
   // the options switch the paths off as they do for host-scanned sources
-  const unsigned allow = tuning().f64_planar ? (tuning().f64_rows ? 3u : 1u) : 0u;
-  hipError_t e = launch_source_layout(u, N, layout, stream, allow);
-  if (e != hipSuccess) return e;
-  int R = tuning().r_f64;
-  if (R != 1 && R != 2 && R != 4) R = 2;
-  int S = N ? choose_splits(M, R, N, 1024) : 1;
-  while (S > 1 && (size_t)S * M > partial_cap) --S;
+  const uint32_t allow = tuning().f64_planar ? (tuning().f64_rows ? 3u : 1u) : 0u;
+  const F64Shape shape = f64_shape(M, N, partial_cap);
+  const int R = shape.R, S = shape.S;
   const uint32_t chunk = N ? (uint32_t)((N + S - 1) / S) : 0;
   const dim3 grid((unsigned)((M + (size_t)kBlock * R - 1) / ((size_t)kBlock * R)),
                   (unsigned)S);
@@ -360,13 +430,13 @@ hipError_t launch_superpose_f64_auto(int sign, WeightForm wf, bool obliquity,
         with_bool(obliquity, [&](auto obl) {
           constexpr int wfv = cart.value ? kCartesian : kPolar;
           k_superpose_f64_auto<sg.value, rr.value, wfv, (bool)obl.value>
-              <<<grid, kBlock, 0, stream>>>(w0, w1, u, (uint32_t)N, chunk, layout, v,
+              <<<grid, kBlock, 0, stream>>>(w0, w1, u, (uint32_t)N, chunk, allow, v,
                                             (uint32_t)M, K, out);
         });
       });
     });
   });
-  e = hipGetLastError();
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   return launch_reduce_partials(S, M, partial, y, stream);
 }

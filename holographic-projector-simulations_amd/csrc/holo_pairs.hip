@@ -889,15 +889,8 @@ __global__ __launch_bounds__(kBlock) void k_reduce_either(const double2* __restr
                                                           double2* __restrict__ y) {
   const uint32_t S = *handled ? Sp : Sg;
   if (S <= 1) return;
-  for (uint32_t m = blockIdx.x * kBlock + threadIdx.x; m < M; m += gridDim.x * kBlock) {
-    double re = 0.0, im = 0.0;
-    for (uint32_t s = 0; s < S; ++s) {  // fixed order: deterministic
-      const double2 p = partial[(size_t)s * M + m];
-      re += p.x;
-      im += p.y;
-    }
-    y[m] = make_double2(re, im);
-  }
+  const uint32_t m = blockIdx.x * kBlock + threadIdx.x;
+  if (m < M) y[m] = sum_splits(partial + m, S, M);
 }
 
 hipError_t launch_reduce_either(const double2* partial, const uint32_t* handled, int Sp, int Sg,

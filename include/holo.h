@@ -104,7 +104,8 @@ void holo_destroy(holo_ctx *ctx);
 holo_status holo_set_stream(holo_ctx *ctx, void *stream);
 holo_status holo_synchronize(holo_ctx *ctx);
 
-/* Tuning knobs (process-wide): "r_f64", "r_f32" targets per lane (1, 2, 4),
+/* Tuning knobs (process-wide): "r_f64", "r_f32" targets per lane (1, 2, 4;
+ * the FP64 kernel takes fewer where that fills the GPU better, unless "splits" is set),
  * "splits" source splits (0 = automatic), "target_waves", "f64_libm" (0/1:
  * use the device libm sqrt/div/sincos in the FP64 kernel), "f64_planar"
  * (0/1: when every source of a plan, or of a host-pointer transform, has the
@@ -156,10 +157,10 @@ holo_status holo_transform_full(holo_ctx *ctx, holo_precision precision,
  * HOLO_OBLIQUITY is accepted), ordered on `stream` (a hipStream_t of the
  * current device, NULL = its null stream) without synchronising.  It needs no
  * context and calls no allocating routine: its scratch (the source-split
- * partial fields and four words of source layout) is a static device array of
+ * partial fields) is a static device array of
  * HOLO_NOALLOC_SCRATCH_BYTES per device, held from the library's first use
  * on a device (holo_create, or the first call of this function there) until
- * the process ends.  The call uses at most (HOLO_NOALLOC_SCRATCH_BYTES - 256)
+ * the process ends.  The call uses at most HOLO_NOALLOC_SCRATCH_BYTES
  * / (16 M) source splits, so every M below 2^31 fits (one split writes y
  * directly).  Every call on a device shares that device's array: calls that
  * overlap on one device (other streams, other threads) race and must be
