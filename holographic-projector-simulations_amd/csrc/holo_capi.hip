@@ -100,6 +100,7 @@ struct holo_plan {
   size_t n_tiles = 0;
   double max_offset = 0.0;
   bool planar = true;
+  double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};  // the sources' bounds, set with the tiles
   // The spatial tiling for k_superpose_f32s.  A lattice plan defers it to
   // the first call that needs it (the lattice kernel does not).
   mutable bool tiles_built = false;
@@ -351,6 +352,7 @@ struct HostTiles {
   std::vector<float4> geo;
   std::vector<int32_t> perm;
   double max_offset = 0.0;
+  double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
   bool planar = true;
 };
 
@@ -406,11 +408,17 @@ void build_tiles(const double* u, size_t N, unsigned T, HostTiles& out) {
   out = HostTiles();
   if (N == 0) return;
   double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  bool finite = true;
   for (size_t n = 0; n < N; ++n)
     for (int d = 0; d < 3; ++d) {
       lo[d] = std::min(lo[d], u[3 * n + d]);
       hi[d] = std::max(hi[d], u[3 * n + d]);
+      finite = finite && std::isfinite(u[3 * n + d]);
     }
+  for (int d = 0; d < 3; ++d) {
+    out.lo[d] = lo[d];
+    out.hi[d] = finite ? hi[d] : INFINITY;  // NaN would not show in the bounds
+  }
   double ext[3], emax = 0.0;
   for (int d = 0; d < 3; ++d) {
     ext[d] = hi[d] - lo[d];
@@ -746,6 +754,8 @@ holo_status plan_build_tiles(holo_ctx* ctx, const holo_plan* p, const double* u_
   holo_plan* q = const_cast<holo_plan*>(p);
   q->n_tiles = n_tiles;
   q->max_offset = t.max_offset;
+  std::copy(t.lo, t.lo + 3, q->lo);
+  std::copy(t.hi, t.hi + 3, q->hi);
   q->planar = t.planar;
   p->tiles_built = true;
   return HOLO_OK;
@@ -1094,9 +1104,41 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
       if (!p->tiles_built) HOLO_TRY(plan_build_tiles(ctx, p, nullptr));
     }
     const size_t slots = p->n_tiles * p->tile;
-    HOLO_HIP(holo::launch_tile_weights(wf, w0, w1, static_cast<const int32_t*>(p->perm.ptr),
-                                       slots, static_cast<float2*>(p->wc.ptr), ctx->stream,
-                                       true));
+    const size_t pe = split_elems_f32(M, p->n_tiles);
+    // Targets on a lattice take the point-to-lattice kernel (default tiles; `skip`
+    // as for the 16-row kernels above)
+    const holo::Tuning& tu = holo::tuning();
+    const uint32_t* skip = nullptr;
+    int Sp = 1;
+    if (tu.grid && tu.grid_pairs && p->tile == 64 && p->N >= holo::kPointMinSources &&
+        M >= holo::kPairMinTargets) {
+      holo::PointPlan pp;
+      pp.u = static_cast<const double*>(p->u.ptr);
+      pp.perm = static_cast<const int32_t*>(p->perm.ptr);
+      pp.wc = static_cast<float2*>(p->wc.ptr);
+      pp.n_slots = (uint32_t)slots;
+      for (int d = 0; d < 3; ++d) {
+        pp.lo[d] = p->lo[d];
+        pp.hi[d] = p->hi[d];
+      }
+      Sp = holo::point_splits(M, slots);
+      const size_t pp_elems = Sp > 1 ? (size_t)Sp * M : 0;
+      if (std::max(pe, pp_elems))
+        HOLO_TRY(ensure(ctx->partial, std::max(pe, pp_elems) * sizeof(double2), ctx->device));
+      HOLO_TRY(ensure(ctx->pairs, 256 + holo::kPairFlags * sizeof(uint32_t), ctx->device));
+      char* b = static_cast<char*>(ctx->pairs.ptr);
+      uint32_t* handled = reinterpret_cast<uint32_t*>(b + 128);
+      HOLO_HIP(holo::launch_superpose_points(
+          sign, obliquity, pp, wf, w0, w1, v, M, lambda, Sp,
+          reinterpret_cast<holo::PairTargets*>(b), reinterpret_cast<uint32_t*>(b + 256), handled,
+          Sp > 1 ? static_cast<double2*>(ctx->partial.ptr) : reinterpret_cast<double2*>(y),
+          ctx->stream));
+      skip = handled;
+    } else {
+      HOLO_HIP(holo::launch_tile_weights(wf, w0, w1, static_cast<const int32_t*>(p->perm.ptr),
+                                         slots, static_cast<float2*>(p->wc.ptr), ctx->stream,
+                                         true));
+    }
     holo::TileSet ts;
     ts.centre = static_cast<const double4*>(p->centre.ptr);
     ts.geo = static_cast<const float4*>(p->geo.ptr);
@@ -1105,13 +1147,12 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
     ts.n_tiles = (uint32_t)p->n_tiles;
     ts.tile = p->tile;
     ts.planar = p->planar;
-    const size_t pe = split_elems_f32(M, p->n_tiles);
     if (pe) HOLO_TRY(ensure(ctx->partial, pe * sizeof(double2), ctx->device));
     HOLO_HIP(holo::launch_superpose_f32s(sign, obliquity, ts,
                                          static_cast<const float2*>(p->wc.ptr), v, M,
                                          lambda, reinterpret_cast<double2*>(y),
                                          static_cast<double2*>(ctx->partial.ptr), pe,
-                                         ctx->stream));
+                                         ctx->stream, skip, Sp));
   }
   return HOLO_OK;
 }

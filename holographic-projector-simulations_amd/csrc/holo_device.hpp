@@ -145,6 +145,37 @@ __device__ __forceinline__ void sincos_rev_f32(float t, float& s, float& c) {
   c = __builtin_amdgcn_cosf(t);
 }
 
+// The FP32 weight (re, im) of source n: polar (wf = kPolar: amplitudes w0, phases
+// w1) or interleaved complex w0; 0 for a padding slot (n < 0).
+__device__ __forceinline__ float2 slot_weight(int wf, const double* __restrict__ w0,
+                                              const double* __restrict__ w1, int32_t n) {
+  if (n < 0) return make_float2(0.f, 0.f);
+  if (wf == kPolar) {
+    double sn, cs;
+    sincos(w1[n], &sn, &cs);
+    return make_float2((float)(w0[n] * cs), (float)(w0[n] * sn));
+  }
+  return make_float2((float)w0[2 * (size_t)n], (float)w0[2 * (size_t)n + 1]);
+}
+
+// The same as (|w|, arg w in cycles, reduced to [-1/2, 1/2)).
+__device__ __forceinline__ float2 slot_weight_polar(int wf, const double* __restrict__ w0,
+                                                    const double* __restrict__ w1, int32_t n) {
+  if (n < 0) return make_float2(0.f, 0.f);
+  constexpr double kInv2Pi = 0.15915494309189535;
+  double a, t;
+  if (wf == kPolar) {
+    a = w0[n];
+    t = w1[n] * kInv2Pi + (a < 0.0 ? 0.5 : 0.0);
+    a = __builtin_fabs(a);
+  } else {
+    const double re = w0[2 * (size_t)n], im = w0[2 * (size_t)n + 1];
+    a = hypot(re, im);
+    t = atan2(im, re) * kInv2Pi;
+  }
+  return make_float2((float)a, (float)(t - __builtin_rint(t)));
+}
+
 // sum of p[0], p[M], .. p[(S - 1) M], in order (deterministic)
 __device__ __forceinline__ double2 sum_splits(const double2* __restrict__ p, uint32_t S,
                                               uint32_t M) {
@@ -170,19 +201,6 @@ __device__ __forceinline__ double2 sum_splits(const double2* __restrict__ p, uin
 
 // ---------------------------------------------------------------------------
 // FP32-split helpers shared by the tiled and lattice kernels.
-
-// The FP32 weight (re, im) of source n: polar (wf = kPolar: amplitudes w0, phases
-// w1) or interleaved complex w0; 0 for a padding slot (n < 0).
-__device__ __forceinline__ float2 slot_weight(int wf, const double* __restrict__ w0,
-                                              const double* __restrict__ w1, int32_t n) {
-  if (n < 0) return make_float2(0.f, 0.f);
-  if (wf == kPolar) {
-    double sn, cs;
-    sincos(w1[n], &sn, &cs);
-    return make_float2((float)(w0[n] * cs), (float)(w0[n] * sn));
-  }
-  return make_float2((float)w0[2 * (size_t)n], (float)w0[2 * (size_t)n + 1]);
-}
 
 // One pair of the FP32-split formulation from its squared distance s and
 // axial offset dz: d (to a few 1e-15, not always correctly rounded) and the

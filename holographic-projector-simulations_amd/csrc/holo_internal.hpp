@@ -152,11 +152,13 @@ hipError_t launch_reduce_partials(int S, size_t M, const double2* partial, doubl
                                   hipStream_t stream);
 
 // FP32-split: weights wc (float2 per slot, polar: launch_tile_weights with
-// polar_out), tiles as above.
+// polar_out), tiles as above.  skip, Sp: as launch_superpose_grid16, for the
+// point-to-lattice kernel.
 hipError_t launch_superpose_f32s(int sign, bool obliquity, const TileSet& ts,
                                  const float2* wc, const double* v, size_t M,
                                  double lambda, double2* y, double2* partial,
-                                 size_t partial_cap, hipStream_t stream);
+                                 size_t partial_cap, hipStream_t stream,
+                                 const uint32_t* skip = nullptr, int Sp = 1);
 
 // Lattice kernel (FP32-split on product-grid tiles).  wc: per-slot FP32
 // weights (launch_tile_weights with the grid perm).  launch_grid_weights
@@ -245,6 +247,10 @@ constexpr size_t kPairFlags = 256;  // words: one per workgroup that checks targ
 // lattice to 18 x 16 targets takes as long as on the 16-row kernels, 39 and 41 us;
 // thinner lattices would mostly be padding).
 constexpr size_t kPairMinTargets = 256;
+// Smallest call of the point-to-lattice kernel: 357 jittered sources to 51 x 127 targets
+// take 38 us (tiled kernel: 63 us), one source to 20 x 30 the same 36 us on either, but
+// with 1.7e-7 of the field for 1.0e-7.
+constexpr size_t kPointMinSources = 256;
 int pair_splits(size_t M, size_t n_tiles);
 // Launches the weights' and targets' preparation and the kernel (with, where
 // grid16 is given, the 16-row kernels' weights in the same launch): *handled
@@ -255,6 +261,22 @@ hipError_t launch_superpose_pairs(int sign, bool obliquity, const PairPlan& pp, 
                                   double lambda, int S, PairTargets* pt, uint32_t* flags,
                                   uint32_t* handled, double2* out, const Grid16Prep* grid16,
                                   hipStream_t stream);
+// Point-to-lattice kernel (holo_points.hip): n_slots slots of sources u[perm[slot]]
+// (perm < 0: none) within [lo, hi]; wc: n_slots float2, the slots' polar weights,
+// written by each launch.
+struct PointPlan {
+  const double* u = nullptr;
+  const int32_t* perm = nullptr;
+  float2* wc = nullptr;
+  uint32_t n_slots = 0;
+  double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+};
+int point_splits(size_t M, size_t n_slots);
+hipError_t launch_superpose_points(int sign, bool obliquity, const PointPlan& pp, WeightForm wf,
+                                   const double* w0, const double* w1, const double* v, size_t M,
+                                   double lambda, int S, PairTargets* pt, uint32_t* flags,
+                                   uint32_t* handled, double2* out, hipStream_t stream);
+
 // y = the sum of partial's Sp splits when *handled, else of its Sg splits
 // (nothing where that is one: y holds the result).
 hipError_t launch_reduce_either(const double2* partial, const uint32_t* handled, int Sp, int Sg,

@@ -465,7 +465,8 @@ __global__ __launch_bounds__(kBlock) void k_superpose_f32s(
     const float2* __restrict__ wc, const int32_t* __restrict__ perm,
     const double* __restrict__ u, uint32_t n_tiles, uint32_t chunk_tiles,
     const double* __restrict__ v, uint32_t M, double lambda,
-    double inv_lambda, double2* __restrict__ out) {
+    double inv_lambda, const uint32_t* __restrict__ skip, double2* __restrict__ out) {
+  if (skip && *skip) return;
   const uint32_t t0 = blockIdx.y * chunk_tiles;
   const uint32_t t1 = min(n_tiles, t0 + chunk_tiles);
   const uint32_t base = blockIdx.x * (kBlock * R) + threadIdx.x;
@@ -590,7 +591,8 @@ static bool with_tile(unsigned T, F&& f) {
 hipError_t launch_superpose_f32s(int sign, bool obliquity, const TileSet& ts,
                                  const float2* wc, const double* v, size_t M,
                                  double lambda, double2* y, double2* partial,
-                                 size_t partial_cap, hipStream_t stream) {
+                                 size_t partial_cap, hipStream_t stream,
+                                 const uint32_t* skip, int Sp) {
   if (M == 0) return hipSuccess;
   int R = tuning().r_f32;
   if (R != 1 && R != 2 && R != 4) R = 2;
@@ -608,7 +610,7 @@ hipError_t launch_superpose_f32s(int sign, bool obliquity, const TileSet& ts,
           with_bool(obliquity, [&](auto obl) {
             k_superpose_f32s<sg.value, rr.value, tt.value, (bool)pl.value, (bool)obl.value>
                 <<<grid, kBlock, 0, stream>>>(ts.centre, ts.geo, wc, ts.perm, ts.u, ts.n_tiles,
-                                              chunk, v, (uint32_t)M, lambda, il, out);
+                                              chunk, v, (uint32_t)M, lambda, il, skip, out);
           });
         });
       });
@@ -617,6 +619,7 @@ hipError_t launch_superpose_f32s(int sign, bool obliquity, const TileSet& ts,
   if (!ok) return hipErrorInvalidValue;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (skip) return launch_reduce_either(partial, skip, Sp, S, M, y, stream);
   return launch_reduce_partials(S, M, partial, y, stream);
 }
 
@@ -626,26 +629,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_weights(
     float2* __restrict__ wc, int polar_out) {
   const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
   if (s >= n_slots) return;
-  const int32_t n = perm[s];
-  float2 r = make_float2(0.f, 0.f);
-  if (!polar_out) {
-    r = slot_weight(wf, w0, w1, n);
-  } else if (n >= 0) {
-    // (|w|, arg w in cycles, reduced to [-1/2, 1/2))
-    constexpr double kInv2Pi = 0.15915494309189535;
-    double a, t;
-    if (wf == kPolar) {
-      a = w0[n];
-      t = w1[n] * kInv2Pi + (a < 0.0 ? 0.5 : 0.0);
-      a = __builtin_fabs(a);
-    } else {
-      const double re = w0[2 * (size_t)n], im = w0[2 * (size_t)n + 1];
-      a = hypot(re, im);
-      t = atan2(im, re) * kInv2Pi;
-    }
-    r = make_float2((float)a, (float)(t - __builtin_rint(t)));
-  }
-  wc[s] = r;
+  wc[s] = polar_out ? slot_weight_polar(wf, w0, w1, perm[s]) : slot_weight(wf, w0, w1, perm[s]);
 }
 
 hipError_t launch_tile_weights(WeightForm wf, const double* w0,

@@ -63,54 +63,14 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
-#include <type_traits>
-
 #include "holo_device.hpp"
 #include "holo_internal.hpp"
+#include "holo_mfma.hpp"
 #include "holo_weights.hpp"
 
 namespace holo {
 
-typedef float pf16 __attribute__((ext_vector_type(16)));
-typedef _Float16 ph2 __attribute__((ext_vector_type(2)));
-typedef _Float16 ph8 __attribute__((ext_vector_type(8)));
-typedef uint32_t pu4 __attribute__((ext_vector_type(4)));
-
-constexpr int kPairTile = 32;   // rows and columns of a target tile, rows of a source tile
-// PairTargets::mode: a form, with kPairWide the source tiles of 64 columns
-constexpr uint32_t kPairFar = 1, kPairNear = 2, kPairWide = 4;
-constexpr float kPairMid = 15.5f;
-constexpr uint32_t kPairMaxRow = 16384;  // longest row of targets looked for
-constexpr int kPairWaves = kBlock / 64;
-constexpr float kFourPi = 12.566370614359172f;
-
-// The bounds of every dropped term over all tile pairs: rxm, rym the largest
-// lateral distances between tile centres, hx, hy the largest |rho|, dz the
-// distance of the planes (the smallest D).  kPairFar, kPairNear or 0.
-// cross = |C| of the first order at its largest; rho has a triangular
-// distribution, so the mean square of an order-n term over a tile pair is below
-// 0.07 (n = 2), 0.022 (n = 4) of its largest: 1.9e-7 for the far form's
-// cross^2 / 2, 2e-7 for the near form's cross^4 / 24, in the tile pairs that are
-// furthest off axis.  NaN gives 0.
-__device__ __forceinline__ uint32_t pair_form(float rxm, float rym, float hx, float hy, float dz,
-                                              float inv_lambda, bool obl) {
-  const float id = 1.f / dz, id2 = id * id, ia = id * inv_lambda;  // D = dz at least
-  const float Pm = 2.f * rxm * hx + hx * hx, Qm = 2.f * rym * hy + hy * hy;
-  const float big = fmaxf(Pm, Qm), sum = Pm + Qm;
-  const float cross = 1.5707964f * ia * id2 * Pm * Qm;
-  const float c3 = 0.0625f * ia * id2 * id2;
-  const float cubic = 18.849556f * c3 * Pm * Qm * sum;  // rad, the c3 part of C
-  const float sq = sum * id2;
-  // alpha P, which cycles32 has to hold, and c2 P^2, in 2^-32 cycles an int32
-  if (!(0.5f * ia * sum <= 0x1p17f && 0.125f * ia * id2 * big * big <= 0.25f)) return 0u;
-  if (cross <= 2.4e-3f && cubic <= 1e-6f && c3 * big * big * big <= 1e-8f &&
-      (obl ? 1.f : 0.5f) * sq * sq <= 1e-7f)
-    return kPairFar;
-  const float q4 = 0.0390625f * sum * sum * sum * sum * ia * id2 * id2 * id2;
-  if (cross <= 0.12f && cubic <= 4e-4f && q4 <= 1e-8f && sq * sq * sq <= 1e-7f) return kPairNear;
-  return 0u;
-}
-
+constexpr int kPairTile = 32;  // rows and columns of a target tile, rows of a source tile
 // MFMA operands of one 32 x 64 source tile's weights by one workgroup, and the
 // target lattice by the n_probe workgroups after them (tail sources' weights by
 // one before those); the rest, if any, prepare the 16-row kernels' weights.
@@ -121,12 +81,7 @@ __device__ __forceinline__ uint32_t pair_form(float rxm, float rym, float hx, fl
 // largest component); slots beyond the lattice are 0.  Wave v of the workgroup
 // forms step v.
 //
-// Targets: every probe workgroup finds the row length (the first target with
-// another x) and the number of rows (the first row that starts with target 0's
-// x again: the generator fills up with copies of point 0), then checks its
-// share of the targets against x_0 + i p_x, y_0 + j p_y, z_0 to 1e-9 of a pitch
-// (a product of one x per row and one y per column to the bit), and the rest
-// against target 0.  flags[b] = 1 when its share passes.
+// Targets: probe_targets.
 struct PairPrep {
   const double* w0;
   const double* w1;
@@ -221,97 +176,36 @@ __device__ void pair_tail_weights(const PairPrep& a, double* s_red) {
   if (threadIdx.x == 0) a.tail_wc[0] = make_float2((float)s_red[0], (float)s_red[kBlock]);
 }
 
-// first k in [1, lim) for which hit(k) holds, else lim; the whole workgroup
-template <typename F>
-__device__ uint32_t block_first(uint32_t lim, uint32_t* s_min, F&& hit) {
-  constexpr int kEach = 4;
-  for (uint32_t base = 1; base < lim; base += kEach * kBlock) {
-    uint32_t first = lim;
-#pragma unroll
-    for (int q = 0; q < kEach; ++q) {
-      const uint32_t k = base + q * kBlock + threadIdx.x;
-      if (k < lim && hit(k)) first = min(first, k);
-    }
-    for (int off = 32; off; off >>= 1)
-      first = min(first, (uint32_t)__shfl_xor((int)first, off, 64));
-    __syncthreads();  // the previous round's reads of s_min are done
-    if ((threadIdx.x & 63) == 0) s_min[threadIdx.x >> 6] = first;
-    __syncthreads();
-    first = min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]));
-    if (first < lim) return first;
+// The form and source tile width for targets with the first and last tile centres
+// (cx0, cy0), (cx1, cy1).  rho has a triangular distribution, so the mean square of
+// an order-n term over a tile pair is below 0.07 (n = 2), 0.022 (n = 4) of its
+// largest: 1.9e-7 for the far form's cross^2 / 2 at 2.4e-3, 2e-7 for the near form's
+// cross^4 / 24 at 0.12, in the tile pairs that are furthest off axis.
+__device__ uint32_t pair_mode(const PairPrep& a, const PairTargets& t, double cx0, double cx1,
+                              double cy0, double cy1) {
+  const auto far = [](double a0, double a1, double b0, double b1) {
+    return fmax(fmax(fabs(a0 - b0), fabs(a0 - b1)), fmax(fabs(a1 - b0), fabs(a1 - b1)));
+  };
+  // source tile centres: rows, and columns of wide and of narrow tiles
+  const double sx0 = a.sx + (double)kPairMid * a.spx;
+  const double sx1 = sx0 + (double)(((a.nx + 31) / 32 - 1) * 32) * a.spx;
+  uint32_t mode = 0u;
+  const float rxm = (float)far(cx0, cx1, sx0, sx1);
+  const float hx = (float)((double)kPairMid * (fabs(t.px) + fabs(a.spx)));
+  const float dz = (float)fabs(t.z - a.sz), il = (float)a.inv_lambda;
+  for (int wide = 1; wide >= 0; --wide) {
+    const double mid = wide ? 31.5 : (double)kPairMid;
+    const uint32_t cols = wide ? 64 : 32;
+    const double sy0 = a.sy + mid * a.spy;
+    const double sy1 = sy0 + (double)(((a.ny + cols - 1) / cols - 1) * cols) * a.spy;
+    const float rym = (float)far(cy0, cy1, sy0, sy1);
+    const float hy = (float)((double)kPairMid * fabs(t.py) + mid * fabs(a.spy));
+    const uint32_t f = pair_form(rxm, rym, hx, hy, dz, il, a.obl != 0, 2.4e-3f, 0.12f);
+    // a wide far form beats everything, and a narrow far form a wide near one
+    if (f && (!mode || (f == kPairFar && mode != (kPairFar | kPairWide))))
+      mode = f | (wide ? kPairWide : 0u);
   }
-  return lim;
-}
-
-__device__ void pair_probe(const PairPrep& a, uint32_t b, uint32_t* s_min) {
-  const double* v = a.v;
-  const uint32_t M = a.M;
-  const double x0 = v[0], y0 = v[1], z0 = v[2];
-  const uint32_t lim = min(M, kPairMaxRow);
-  const uint32_t ny = block_first(lim, s_min, [&](uint32_t k) { return v[3 * (size_t)k] != x0; });
-  uint32_t nx = ny < lim && ny >= 16 ? M / ny : 0u;
-  if (nx >= 16)
-    nx = block_first(nx, s_min, [&](uint32_t k) { return v[3 * (size_t)k * ny] == x0; });
-  bool ok = nx >= 16;
-  double px = 0.0, py = 0.0;
-  if (ok) {
-    const uint32_t body = nx * ny;
-    px = (v[3 * (size_t)(nx - 1) * ny] - x0) / (double)(nx - 1);
-    py = (v[3 * (size_t)(ny - 1) + 1] - y0) / (double)(ny - 1);
-    const double tx = 1e-9 * fabs(px), ty = 1e-9 * fabs(py);
-    ok = tx > 0.0 && ty > 0.0 && __builtin_isfinite(px) && __builtin_isfinite(py);
-    for (uint32_t m = b * kBlock + threadIdx.x; m < M; m += a.n_probe * kBlock) {
-      const double x = v[3 * (size_t)m], y = v[3 * (size_t)m + 1], z = v[3 * (size_t)m + 2];
-      if (m < body) {
-        const uint32_t i = m / ny, j = m - i * ny;
-        ok = ok && x == v[3 * (size_t)i * ny] && y == v[3 * (size_t)j + 1] && z == z0 &&
-             fabs(x - (x0 + (double)i * px)) <= tx && fabs(y - (y0 + (double)j * py)) <= ty;
-      } else {
-        ok = ok && x == x0 && y == y0 && z == z0;
-      }
-    }
-  }
-  const int all = __syncthreads_and(ok ? 1 : 0);
-  if (threadIdx.x) return;
-  a.flags[b] = all ? 1u : 0u;
-  if (b) return;
-  PairTargets t;
-  t.x0 = x0;
-  t.y0 = y0;
-  t.z = z0;
-  t.px = px;
-  t.py = py;
-  t.nx = nx;
-  t.ny = ny;
-  t.mode = 0u;
-  if (all) {
-    // tile centres of the targets: first and last
-    const double cx0 = x0 + (double)kPairMid * px, cy0 = y0 + (double)kPairMid * py;
-    const double cx1 = cx0 + (double)(((nx + 31) / 32 - 1) * 32) * px;
-    const double cy1 = cy0 + (double)(((ny + 31) / 32 - 1) * 32) * py;
-    const auto far = [](double a0, double a1, double b0, double b1) {
-      return fmax(fmax(fabs(a0 - b0), fabs(a0 - b1)), fmax(fabs(a1 - b0), fabs(a1 - b1)));
-    };
-    // source tile centres: rows, and columns of wide and of narrow tiles
-    const double sx0 = a.sx + (double)kPairMid * a.spx;
-    const double sx1 = sx0 + (double)(((a.nx + 31) / 32 - 1) * 32) * a.spx;
-    const float rxm = (float)far(cx0, cx1, sx0, sx1);
-    const float hx = (float)((double)kPairMid * (fabs(px) + fabs(a.spx)));
-    const float dz = (float)fabs(z0 - a.sz), il = (float)a.inv_lambda;
-    for (int wide = 1; wide >= 0; --wide) {
-      const double mid = wide ? 31.5 : (double)kPairMid;
-      const uint32_t cols = wide ? 64 : 32;
-      const double sy0 = a.sy + mid * a.spy;
-      const double sy1 = sy0 + (double)(((a.ny + cols - 1) / cols - 1) * cols) * a.spy;
-      const float rym = (float)far(cy0, cy1, sy0, sy1);
-      const float hy = (float)((double)kPairMid * fabs(py) + mid * fabs(a.spy));
-      const uint32_t f = pair_form(rxm, rym, hx, hy, dz, il, a.obl != 0);
-      // a wide far form beats everything, and a narrow far form a wide near one
-      if (f && (!t.mode || (f == kPairFar && t.mode != (kPairFar | kPairWide))))
-        t.mode = f | (wide ? kPairWide : 0u);
-    }
-  }
-  *a.pt = t;
+  return mode;
 }
 
 __global__ __launch_bounds__(kBlock) void k_pair_prep(PairPrep a, Grid16Prep g) {
@@ -330,7 +224,10 @@ __global__ __launch_bounds__(kBlock) void k_pair_prep(PairPrep a, Grid16Prep g) 
     --b;
   }
   if (b < a.n_probe)
-    pair_probe(a, b, reinterpret_cast<uint32_t*>(s_buf));
+    probe_targets(a.v, a.M, b, a.n_probe, a.pt, a.flags, reinterpret_cast<uint32_t*>(s_buf),
+                  [&](const PairTargets& t, double cx0, double cx1, double cy0, double cy1) {
+                    return pair_mode(a, t, cx0, cx1, cy0, cy1);
+                  });
   else
     grid16_weights(g, b - a.n_probe);
 }
@@ -344,56 +241,6 @@ struct PairLds {
   uint32_t tF[kPairWaves][64], sF[kPairWaves][96];
   float tp[kPairWaves][64], sp[kPairWaves][96];
 };
-
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// x added to this lane's own word of LDS, without reading it back
-__device__ __forceinline__ void lds_add(double* p, double x) {
-  __hip_atomic_fetch_add(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
-__device__ __forceinline__ double lane_f64(double x, int lane) {
-  const uint64_t b = __builtin_bit_cast(uint64_t, x);
-  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)b, lane);
-  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
-  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
-
-// x + kCycles32 has ulp 2^-32 for |x| < 2^19 - 1: its low word is x modulo one
-// cycle, in 2^-32 cycles.
-constexpr double kCycles32 = 0x1.8p20;
-__device__ __forceinline__ uint32_t cycles32(double x) {
-  return (uint32_t)__builtin_bit_cast(uint64_t, x);
-}
-
-__device__ __forceinline__ pf16 mfma32(ph8 a, ph8 b, pf16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ ph8 neg8(ph8 x) {
-  pu4 u = __builtin_bit_cast(pu4, x);
-  u ^= 0x80008000u;
-  return __builtin_bit_cast(ph8, u);
-}
-
-// (a, b) rounded to nearest f16
-typedef float pf2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ ph2 pk(float a, float b) {
-  return __builtin_convertvector((pf2{a, b}), ph2);
-}
-
-// A product that is split into hi and lo: kept apart from the conversions, as
-// the compiler could fold it into the one that gives the operand hi and not into
-// the one that lo = x - hi is formed with, and at ties hi + lo would then be off
-// by an f16 ulp of x.
-__device__ __forceinline__ float formed(float x) {
-  __asm__("" : "+v"(x));
-  return x;
-}
 
 // Eight phasors of one step: (c, s), their p (or q) and amplitude.
 struct Phasors {
@@ -450,72 +297,6 @@ struct PairWave {
   }
 };
 
-// hi = (x rounded), lo = am x - hi, of eight values (x formed: no product)
-__device__ __forceinline__ void split8(const float (&x)[8], const float (&am)[8], ph8& hi,
-                                       ph8& lo) {
-#pragma unroll
-  for (int e = 0; e < 8; e += 2) {
-    const ph2 t = pk(x[e], x[e + 1]);
-    hi[e] = t[0];
-    hi[e + 1] = t[1];
-    const ph2 d = pk(__builtin_fmaf(am[e], x[e], -(float)t[0]),
-                     __builtin_fmaf(am[e + 1], x[e + 1], -(float)t[1]));
-    lo[e] = d[0];
-    lo[e + 1] = d[1];
-  }
-}
-
-__device__ __forceinline__ void split8(const float (&x)[8], float one, ph8& hi, ph8& lo) {
-#pragma unroll
-  for (int e = 0; e < 8; e += 2) {
-    const ph2 t = pk(x[e], x[e + 1]);
-    hi[e] = t[0];
-    hi[e + 1] = t[1];
-    const ph2 d = pk(__builtin_fmaf(x[e], one, -(float)t[0]),
-                     __builtin_fmaf(x[e + 1], one, -(float)t[1]));
-    lo[e] = d[0];
-    lo[e + 1] = d[1];
-  }
-}
-
-__device__ __forceinline__ ph8 half8(const float (&x)[8]) {
-  ph8 r;
-#pragma unroll
-  for (int e = 0; e < 8; e += 2) {
-    const ph2 t = pk(x[e], x[e + 1]);
-    r[e] = t[0];
-    r[e + 1] = t[1];
-  }
-  return r;
-}
-
-// eight values as f16
-__device__ __forceinline__ ph8 mul8(ph8 a, ph8 b) { return a * b; }
-
-// (Dr, Di) += complex product of the hi parts of A and B
-struct Cplx8 {
-  ph8 rh, rl, ih, il;
-};
-
-__device__ __forceinline__ void cmul_hi(const Cplx8& a, const Cplx8& b, pf16& Dr, pf16& Di) {
-  Dr = mfma32(a.rh, b.rh, Dr);
-  Di = mfma32(a.rh, b.ih, Di);
-  Dr = mfma32(a.ih, neg8(b.ih), Dr);
-  Di = mfma32(a.ih, b.rh, Di);
-}
-
-// and of hi by lo and lo by hi parts
-__device__ __forceinline__ void cmul_lo(const Cplx8& a, const Cplx8& b, pf16& Dr, pf16& Di) {
-  Dr = mfma32(a.rh, b.rl, Dr);
-  Di = mfma32(a.rh, b.il, Di);
-  Dr = mfma32(a.ih, neg8(b.il), Dr);
-  Di = mfma32(a.ih, b.rl, Di);
-  Dr = mfma32(a.rl, b.rh, Dr);
-  Di = mfma32(a.rl, b.ih, Di);
-  Dr = mfma32(a.il, neg8(b.ih), Dr);
-  Di = mfma32(a.il, b.rh, Di);
-}
-
 // registers 8 s .. 8 s + 7 of T as the second product's B operand
 template <bool FULL>
 __device__ __forceinline__ Cplx8 operand_of(const pf16& Tr, const pf16& Ti, int s, float one) {
@@ -535,9 +316,6 @@ __device__ __forceinline__ Cplx8 operand_of(const pf16& Tr, const pf16& Ti, int 
   }
   return o;
 }
-
-constexpr pf16 kZero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
-                          0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
 // PART 0: the far form (g_0 full, g_1 hi parts); PART 1, 2: the near form's g_0,
 // g_1 (full) and g_2, g_3 (hi parts).  Adds the products of a tile with `steps`
@@ -901,9 +679,6 @@ hipError_t launch_reduce_either(const double2* partial, const uint32_t* handled,
                                                  (uint32_t)M, y);
   return hipGetLastError();
 }
-
-// Two workgroups of four waves run on a CU (their LDS and VGPRs).
-constexpr size_t kPairSlots = 2 * 256;
 
 // One split where the target tiles fill the slots many times over; else the
 // count (at most 8 above one round) that leaves the last round fullest, each

@@ -112,7 +112,11 @@ holo_status holo_synchronize(holo_ctx *ctx);
  * same z, the FP64 kernel forms dz once per target; same bits; default 1),
  * "f64_rows" (0/1: with "f64_planar", when the sources also come in rows of
  * consecutive sources with one x, as lattices in x-slow order do, dx^2 is
- * formed once per target and row; same bits; default 1),
+ * formed once per target and row; same bits; default 1), "grid_pairs" (0/1:
+ * HOLO_FP32_SPLIT to targets on a uniform lattice, 256 or more, uses the
+ * lattice-to-lattice kernel where the sources are on a uniform lattice too,
+ * and the point-to-lattice kernel for 256 or more sources elsewhere, within
+ * their far-field bounds; default 1),
  * "grid" (0/1: HOLO_FP32_SPLIT on lattice sources uses the matrix-core
  * lattice kernel; default 1), "grid16" (0/1: on a uniform lattice that
  * kernel uses 16 x 16 tiles, padded to multiples of 16; default 1), "grid32"
