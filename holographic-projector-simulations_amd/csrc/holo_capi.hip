@@ -1454,7 +1454,7 @@ holo_status holo_transform_mc(holo_ctx* ctx, holo_precision precision, int sign,
   HOLO_TRY(ensure(ctx->ph, N * sizeof(double), ctx->device));
   // per-target FP32-split draws on product-grid sources gather only the
   // weight; the grid is recognised on the device, without a host round trip
-  const bool lattice = !fp64 && !(flags & HOLO_MC_SHARED) && holo::tuning().mc_lattice;
+  const bool lattice = !fp64 && !(flags & HOLO_MC_SHARED);
   holo::McLattice lat;
   if (lattice) {
     HOLO_TRY(ensure(ctx->mc_wc, N * sizeof(float2), ctx->device));
@@ -1463,6 +1463,7 @@ holo_status holo_transform_mc(holo_ctx* ctx, holo_precision precision, int sign,
     lat.info = static_cast<const uint32_t*>(ctx->mc_info.ptr);
     lat.wc = static_cast<const float2*>(ctx->mc_wc.ptr);
     lat.xy = static_cast<const double*>(ctx->mc_xy.ptr);
+    lat.use = holo::tuning().mc_lattice;
   }
   HOLO_HIP(holo::launch_mc_pack(fp64, da, dp, du, N, static_cast<double4*>(ctx->pos.ptr),
                                 static_cast<double*>(ctx->ph.ptr),

@@ -101,6 +101,9 @@ struct U4 {
   uint32_t x, y, z, w;
 };
 
+// LANES: for counters (uniform, per lane, uniform, uniform): from the fourth round on
+// both factors differ by lane and the two XORs of a word are one instruction.
+template <bool LANES = false>
 __device__ __forceinline__ U4 philox4x32_10(U4 c, uint32_t k0, uint32_t k1) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
@@ -113,9 +116,9 @@ __device__ __forceinline__ U4 philox4x32_10(U4 c, uint32_t k0, uint32_t k1) {
     const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0;
     const uint32_t hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
     U4 n;
-    n.x = hi1 ^ c.y ^ k0;
+    n.x = LANES && r >= 3 ? __builtin_amdgcn_bitop3_b32(hi1, c.y, k0, 0x96) : hi1 ^ c.y ^ k0;
     n.y = lo1;
-    n.z = hi0 ^ c.w ^ k1;
+    n.z = LANES && r >= 4 ? __builtin_amdgcn_bitop3_b32(hi0, c.w, k1, 0x96) : hi0 ^ c.w ^ k1;
     n.w = lo0;
     c = n;
   }

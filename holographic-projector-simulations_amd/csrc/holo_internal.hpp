@@ -308,14 +308,28 @@ struct McLattice {
   const uint32_t* info = nullptr;
   const float2* wc = nullptr;
   const double* xy = nullptr;
+  bool use = true;  // false: every source from its record, over the same ranges
 };
 
-// Per-target Monte Carlo runs as one launch per source range of about
-// kMcPassBytes of gathered data, which one XCD's 4 MB L2 holds beside the
-// streamed targets (on the 1024^2 lattice, K = 4096: 39.1 ms in one launch,
-// 23.0 / 22.9 / 25.9 / 32.9 ms in 2 / 3 / 4 / 6 ranges): the number of ranges.
-constexpr size_t kMcPassBytes = size_t(3) << 20;
-uint32_t mc_passes(size_t N, bool fp64);
+// Per-target Monte Carlo runs over source ranges whose gathered data one XCD's 4 MB
+// L2 holds (1024^2 targets, K = 1024, in us: 1024^2 lattice 8920 / 4210 / 4340 / 4860
+// in 1 / 2 / 3 / 4 ranges of its 8 MB of weights; jittered 14300 / 8010 / 7550 in
+// 3 / 5 / 8 of its 32 MB of records).
+// A grid of up to this many workgroups is resident at once: one launch takes its
+// ranges in turn (256^2 targets, lattice: 397 us, 456 in a launch per range), while
+// those of a larger grid drift apart (1024^2: 8140 us, 4260).
+constexpr unsigned kMcRound = 768;
+// From this many draws on (an eighth where kMcRound holds) lattices take the kernel
+// that stages their tables in LDS and other sources the general one, each an idle
+// launch or range for the other: 2^22 draws 630 -> 414 us, 2^26 427 -> 386 us on the
+// 1024^2 lattice; at 2^24 the idle launches take what the tables give.
+constexpr uint64_t kMcStageDraws = uint64_t(1) << 25;
+// Draws a target from which k_mc stages the tables too (131 x 72 sources, 98518
+// targets, K = 23: 27 us without, 28 us with; 100^2 to 256^2, K = 1024: 270 -> 173 us).
+constexpr uint32_t kMcStageK = 64;
+// From this many on the general kernel's ranges fit records instead of weights: 2^26
+// draws from 700^2 jittered sources 609 (2 ranges) -> 564 us (5), 2^24 294 -> 294 us.
+constexpr uint64_t kMcRecordDraws = uint64_t(1) << 26;
 
 hipError_t launch_mc(int sign, bool fp64, bool shared, bool obliquity, const double4* pos,
                      const double* ph, size_t N, const double* v, size_t M,

@@ -661,18 +661,25 @@ __device__ __forceinline__ U4 mc_draws(uint32_t k, uint32_t m, uint32_t slo, uin
   if constexpr (SHARED_IDX)
     return philox4x32_10(U4{k >> 1, m / kMcGroup, kMcSharedTag, kMcStream}, slo, shi);
   else
-    return philox4x32_10(U4{k >> 1, m, 0u, kMcStream}, slo, shi);
+    return philox4x32_10<true>(U4{k >> 1, m, 0u, kMcStream}, slo, shi);
 }
 
 // A drawn source n as (x, y, z, w): w = amp (FP64, the phase in ph[n]) or the
 // bit-cast FP32 weight (FP32-split).  On a product grid (FP32-split only) the
 // sources of the leading complete rows come from the row and column tables
-// and the weight array, the same values as the packed records.
+// and the weight array, the same values as the packed records: of a call's
+// sources all (kMcTables), none (kMcRecords) or some (kMcMixed, which chooses
+// each component's address by a select).
+enum McView { kMcRecords, kMcStaged, kMcTables, kMcMixed };
+constexpr uint32_t kMcTable = 2560;  // entries of the tables staged in LDS
+
 struct McSourceView {
   const double4* pos;
   McLattice lat;
-  uint32_t ny = 0, body = 0;
-  double inv_ny = 0.0;
+  uint32_t ny = 0, body = 0, magic = 0, row0 = 0;
+  bool whole = false;  // all sources are on the grid
+  double z = 0.0;
+  const double* table = nullptr;
   __device__ McSourceView(const double4* p, const McLattice& l, bool fp64, uint32_t N)
       : pos(p), lat(l) {
     uint32_t rows = 0;
@@ -682,23 +689,65 @@ struct McSourceView {
       if (!rows) ny = 0;
     }
     body = min(rows * ny, N);
-    inv_ny = ny ? 1.0 / (double)ny : 0.0;
+    whole = ny && body == N;
+    if (!lat.use || body < N / 2) body = 0;  // jittered sources start with a "row" of one
+    if (ny) {
+      magic = 0xffffffffu / ny;
+      z = lat.xy[kLatticeMaxRow];
+    }
   }
-  // branch-free: each component is one load from an address chosen by select
-  __device__ __forceinline__ double4 operator()(uint32_t n) const {
+  // Whether all sources are on the grid and the tables' part for any `width` of them
+  // fits into kMcTable entries.
+  __device__ __forceinline__ bool stages(uint32_t width) const {
+    return whole && ny <= kMcTable && ny + width / ny + 2 <= kMcTable;
+  }
+  // The tables' part for the sources [lo, hi) into tab, the columns first; the whole
+  // workgroup.
+  __device__ __forceinline__ void stage(uint32_t lo, uint32_t hi, double* tab) {
+    row0 = lo / ny;
+    const uint32_t entries = ny + (hi - 1) / ny + 1 - row0;
+    for (uint32_t k = threadIdx.x; k < entries; k += kBlock)
+      tab[k] = k < ny ? lat.xy[k] : lat.xy[kLatticeMaxRow + 1 + row0 + k - ny];
+    table = tab;
+    __syncthreads();
+  }
+  template <McView VIEW>
+  __device__ __forceinline__ double4 at(uint32_t n) const {
+    if constexpr (VIEW == kMcRecords) return pos[n];
+    // n / ny: magic is 2^32 / ny less at most 1, and n < 2^31, so the product's
+    // high word is the quotient or one less
+    uint32_t i = __umulhi(n, magic), j = n - i * ny;
+    const bool next = j >= ny;
+    i += next ? 1u : 0u;
+    j -= next ? ny : 0u;
+    const double* pw = reinterpret_cast<const double*>(lat.wc + n);
+    if constexpr (VIEW == kMcStaged)
+      return make_double4(table[ny - row0 + i], table[j], z, *pw);
+    const double* px = lat.xy + (kLatticeMaxRow + 1 + i);
+    const double* py = lat.xy + j;
+    if constexpr (VIEW == kMcTables) return make_double4(*px, *py, z, *pw);
     const bool tab = n < body;
-    uint32_t i = (uint32_t)((double)n * inv_ny);  // within one of n / ny
-    i -= (uint32_t)(i * ny > n);
-    i += (uint32_t)((i + 1) * ny <= n);
-    const uint32_t j = n - i * ny;
     const double* rec = &pos[n].x;
-    const double* px = tab ? lat.xy + kLatticeMaxRow + 1 + i : rec;
-    const double* py = tab ? lat.xy + j : rec + 1;
+    px = tab ? px : rec;
+    py = tab ? py : rec + 1;
     const double* pz = tab ? lat.xy + kLatticeMaxRow : rec + 2;
-    const double* pw = tab ? reinterpret_cast<const double*>(lat.wc + n) : rec + 3;
+    pw = tab ? pw : rec + 3;
     return make_double4(*px, *py, *pz, *pw);
   }
 };
+
+// f(view) with the sources' McView, which is uniform.
+template <bool FP64, typename F>
+__device__ __forceinline__ void with_view(const McSourceView& s, uint32_t N, F&& f) {
+  if (FP64 || s.body == 0)
+    f(std::integral_constant<McView, kMcRecords>{});
+  else if (s.table)
+    f(std::integral_constant<McView, kMcStaged>{});
+  else if (s.body == N)
+    f(std::integral_constant<McView, kMcTables>{});
+  else
+    f(std::integral_constant<McView, kMcMixed>{});
+}
 
 // Per-target estimator; thread i evaluates the target at v[i], whose index
 // (the Philox counter) is tmap[i], or i without a map.  Block row blockIdx.y
@@ -709,67 +758,77 @@ __global__ __launch_bounds__(kBlock) void k_mc(
     const double4* __restrict__ pos, const double* __restrict__ ph,
     uint32_t N, const double* __restrict__ v, uint32_t M, const uint32_t* __restrict__ tmap,
     uint32_t K, uint32_t kchunk, uint32_t seed_lo, uint32_t seed_hi, double Kw,
-    double inv_lambda, double scale, McLattice lat, double2* __restrict__ y) {
+    double inv_lambda, double scale, McLattice lat, int stage, int staged_only,
+    double2* __restrict__ y) {
+  __shared__ double s_tab[FP64 ? 1 : kMcTable];
+  McSourceView source(pos, lat, FP64, N);
+  if constexpr (!FP64) {
+    const bool staged = source.stages(N);  // uniform
+    if (staged_only && !staged) return;
+    if (stage && lat.use && staged) source.stage(0, N, s_tab);
+  }
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= M) return;
   const uint32_t kb = blockIdx.y * kchunk, ke = min(K, kb + kchunk);
   const uint32_t m = tmap ? tmap[i] : i;
   const double vx = v[3 * (size_t)i], vy = v[3 * (size_t)i + 1],
                vz = v[3 * (size_t)i + 2];
-  const McSourceView source(pos, lat, FP64, N);
   double ar = 0.0, ai = 0.0;
-  float fr = 0.f, fi = 0.f;
-  // 8 samples per step: 4 Philox blocks, then 8 independent gathers in flight
-  const uint32_t K8 = kb + ((ke - kb) & ~7u);
-  for (uint32_t k = kb; k < K8; k += 8) {
-    uint32_t idx[8];
+  with_view<FP64>(source, N, [&](auto view) {
+    float fr = 0.f, fi = 0.f;
+    // 8 samples per step: 4 Philox blocks, then 8 independent gathers in flight
+    const uint32_t K8 = kb + ((ke - kb) & ~7u);
+    for (uint32_t k = kb; k < K8; k += 8) {
+      uint32_t idx[8];
 #pragma unroll
-    for (int h = 0; h < 4; ++h) {
-      const U4 o = mc_draws<SHARED_IDX>(k + 2 * h, m, seed_lo, seed_hi);
-      idx[2 * h] = lemire_index(o.x, o.y, N);
-      idx[2 * h + 1] = lemire_index(o.z, o.w, N);
-    }
-    double4 p[8];
-    double phv[8];
+      for (int h = 0; h < 4; ++h) {
+        const U4 o = mc_draws<SHARED_IDX>(k + 2 * h, m, seed_lo, seed_hi);
+        idx[2 * h] = lemire_index(o.x, o.y, N);
+        idx[2 * h + 1] = lemire_index(o.z, o.w, N);
+      }
+      double4 p[8];
+      double phv[8];
 #pragma unroll
-    for (int h = 0; h < 8; ++h) {
-      p[h] = source(idx[h]);
-      if constexpr (FP64) phv[h] = ph[idx[h]];
-    }
+      for (int h = 0; h < 8; ++h) {
+        p[h] = source.at<view.value>(idx[h]);
+        if constexpr (FP64) phv[h] = ph[idx[h]];
+      }
+      __builtin_amdgcn_sched_barrier(0);  // all loads before the first pair
 #pragma unroll
-    for (int h = 0; h < 8; ++h) {
-      if constexpr (FP64) {
-        const PairF64 q =
-            pair_f64<SIGN, 0, OBL>(p[h].w, phv[h], p[h].x, p[h].y, p[h].z, vx, vy, vz, Kw);
-        accumulate_phasor<0>(q.r, q.arg, ar, ai);
-      } else {
-        mc_pair_f32s<SIGN, OBL>(p[h], vx, vy, vz, inv_lambda, fr, fi);
+      for (int h = 0; h < 8; ++h) {
+        if constexpr (FP64) {
+          const PairF64 q =
+              pair_f64<SIGN, 0, OBL>(p[h].w, phv[h], p[h].x, p[h].y, p[h].z, vx, vy, vz, Kw);
+          accumulate_phasor<0>(q.r, q.arg, ar, ai);
+        } else {
+          mc_pair_f32s<SIGN, OBL>(p[h], vx, vy, vz, inv_lambda, fr, fi);
+        }
+      }
+      if constexpr (!FP64) {
+        ar += fr;
+        ai += fi;
+        fr = 0.f;
+        fi = 0.f;
       }
     }
-    if constexpr (!FP64) {
-      ar += fr;
-      ai += fi;
-      fr = 0.f;
-      fi = 0.f;
-    }
-  }
-  for (uint32_t k = K8; k < ke; k += 2) {
-    const U4 o = mc_draws<SHARED_IDX>(k, m, seed_lo, seed_hi);
-    const uint32_t idx[2] = {lemire_index(o.x, o.y, N), lemire_index(o.z, o.w, N)};
+    for (uint32_t k = K8; k < ke; k += 2) {
+      const U4 o = mc_draws<SHARED_IDX>(k, m, seed_lo, seed_hi);
+      const uint32_t idx[2] = {lemire_index(o.x, o.y, N), lemire_index(o.z, o.w, N)};
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if (h == 1 && k + 1 >= ke) break;
-      const double4 p = source(idx[h]);
-      if constexpr (FP64) {
-        const PairF64 q = pair_f64<SIGN, 0, OBL>(p.w, ph[idx[h]], p.x, p.y, p.z, vx, vy, vz, Kw);
-        accumulate_phasor<0>(q.r, q.arg, ar, ai);
-      } else {
-        mc_pair_f32s<SIGN, OBL>(p, vx, vy, vz, inv_lambda, fr, fi);
+      for (int h = 0; h < 2; ++h) {
+        if (h == 1 && k + 1 >= ke) break;
+        const double4 p = source.at<view.value>(idx[h]);
+        if constexpr (FP64) {
+          const PairF64 q = pair_f64<SIGN, 0, OBL>(p.w, ph[idx[h]], p.x, p.y, p.z, vx, vy, vz, Kw);
+          accumulate_phasor<0>(q.r, q.arg, ar, ai);
+        } else {
+          mc_pair_f32s<SIGN, OBL>(p, vx, vy, vz, inv_lambda, fr, fi);
+        }
       }
     }
-  }
-  ar += fr;
-  ai += fi;
+    ar += fr;
+    ai += fi;
+  });
   y[(size_t)blockIdx.y * M + i] = make_double2(ar * scale, ai * scale);
 }
 
@@ -777,52 +836,60 @@ __global__ __launch_bounds__(kBlock) void k_mc(
 // random source; from a 1024^2 plane the gathered data (8 MB of weights on a
 // lattice, 32 MB of records otherwise) does not fit the 4 MB L2 of an XCD, and
 // the misses bound k_mc.  k_mc_pass takes only the draws whose source index
-// lies in [lo, hi), a range whose data fits one L2, and the host launches it
-// once per range: every launch regenerates its targets' Philox streams (the
-// indices are k_mc's), queues each lane's in-range draws in that lane's LDS
-// ring and evaluates them 8 at a time, every lane of the wave taking 8 once
-// each active lane holds 8; a ring that could overflow in the next round
-// forces a partial batch (lanes with fewer entries idle in it).  Each launch
-// adds its sums into y[m] (FP64): the first writes, the last scales by N / K.
-// The summation order of a target is fixed by its indices and the ranges.
+// lies in a range whose data fits one L2, range after range: each regenerates its
+// targets' Philox streams (the indices are k_mc's), queues each lane's in-range
+// draws in that lane's LDS ring and evaluates them 8 at a time, every lane of the
+// wave taking 8 once each active lane holds 8; a ring that could overflow in the
+// next round forces a partial batch (lanes with fewer entries idle in it).  A
+// launch takes the ranges [b0, b1) and adds their sums into y[m] (FP64): the first
+// writes, the last scales by N / K.  The summation order of a target is fixed by
+// its indices and the ranges.
+// What bounds it: the lines that the L2s deliver, one of 128 bytes for each draw's
+// weight (32.6 TB/s; 34 where everything hits), which is why the other two gathers,
+// from the row and column tables, are staged in LDS (STAGE: they fit kMcTable
+// entries, three workgroups to a CU): as L1 gathers they kept the address units
+// busy at 55 cycles each.  1024^2 lattice to 1024^2 targets, K = 1024: 5.3 -> 4.26 ms.
+// Idle slots read source lo, one line for all (their old entries: 4.78 ms).  Weights
+// loaded past the caches (nontemporal): 11.9 ms.  Records (jittered): 14.3 -> 7.6 ms.
 constexpr uint32_t kMcQueue = 32;  // ring slots per lane, a power of two
 
-template <int SIGN, bool FP64, bool OBL>
-__global__ __launch_bounds__(kBlock) void k_mc_pass(
-    const double4* __restrict__ pos, const double* __restrict__ ph, uint32_t N,
-    const double* __restrict__ v, uint32_t M, uint32_t K, uint32_t seed_lo, uint32_t seed_hi,
-    double Kw, double inv_lambda, McLattice lat, uint32_t lo, uint32_t hi, int first,
-    double scale, double2* __restrict__ y) {
-  __shared__ uint32_t s_q[kMcQueue][kBlock];  // [slot][lane]: one bank per lane
-  const uint32_t t = threadIdx.x, m = blockIdx.x * kBlock + t;
-  const bool active = m < M;
-  if (__ballot(active) == 0) return;  // the whole wave is past M (no barriers below)
-  const uint32_t mm = active ? m : M - 1;
-  const double vx = v[3 * (size_t)mm], vy = v[3 * (size_t)mm + 1], vz = v[3 * (size_t)mm + 2];
-  const McSourceView source(pos, lat, FP64, N);
-  double ar = 0.0, ai = 0.0;
+template <McView VIEW, int SIGN, bool FP64, bool OBL>
+__device__ __forceinline__ void mc_pass(const McSourceView& source, const double* __restrict__ ph,
+                                        uint32_t N, double vx, double vy, double vz, bool active,
+                                        uint32_t m, uint32_t K, uint32_t seed_lo,
+                                        uint32_t seed_hi, double Kw, double inv_lambda,
+                                        uint32_t lo, uint32_t hi, uint32_t* s_q, double& ar,
+                                        double& ai) {
+  // byte offsets into the ring [slot][lane]: one bank per lane
+  constexpr uint32_t kStep = kBlock * sizeof(uint32_t), kMask = (kMcQueue - 1) * kStep;
+  const uint32_t t = threadIdx.x * (uint32_t)sizeof(uint32_t);
+  const auto slot = [&](uint32_t at) __attribute__((always_inline)) -> uint32_t& {
+    return *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(s_q) + ((at & kMask) | t));
+  };
   uint32_t head = 0, tail = 0;
-  // the next `take` (<= 8) queued draws of this lane; idle slots read source
-  // lo and their terms are dropped by a select (never multiplied by zero: a
-  // target at that source would turn 0 * inf into NaN)
-  const auto batch = [&](uint32_t take) __attribute__((always_inline)) {
+  // the next 8 queued draws of every lane, or up to 8; idle lanes drop their terms by
+  // a select (never multiplied by zero: a target at source lo would turn 0 * inf
+  // into NaN)
+  const auto batch = [&](auto full) __attribute__((always_inline)) {
+    const uint32_t take = full.value ? 8 * kStep : min(8 * kStep, tail - head);
     uint32_t idx[8];
 #pragma unroll
-    for (int h = 0; h < 8; ++h) {
-      const uint32_t q = s_q[(head + h) & (kMcQueue - 1)][t];
-      idx[h] = (active && (uint32_t)h < take) ? q : lo;
+    for (uint32_t h = 0; h < 8; ++h) {
+      const uint32_t n = slot(head + h * kStep);
+      idx[h] = active && h * kStep < take ? n : lo;  // idle slots all read one line
     }
     double4 p[8];
     double phv[8];
 #pragma unroll
     for (int h = 0; h < 8; ++h) {
-      p[h] = source(idx[h]);
+      p[h] = source.template at<VIEW>(idx[h]);
       if constexpr (FP64) phv[h] = ph[idx[h]];
     }
-    float fr = 0.f, fi = 0.f;
+    __builtin_amdgcn_sched_barrier(0);  // all loads before the first pair
+    float fr[2] = {0.f, 0.f}, fi[2] = {0.f, 0.f};  // sums of four in FP32
 #pragma unroll
     for (int h = 0; h < 8; ++h) {
-      const bool use = (uint32_t)h < take;
+      const bool use = full.value || h * kStep < take;
       if constexpr (FP64) {
         const PairF64 q =
             pair_f64<SIGN, 0, OBL>(p[h].w, phv[h], p[h].x, p[h].y, p[h].z, vx, vy, vz, Kw);
@@ -831,45 +898,92 @@ __global__ __launch_bounds__(kBlock) void k_mc_pass(
         ar += use ? tr : 0.0;
         ai += use ? ti : 0.0;
       } else {
-        float tr = 0.f, ti = 0.f;
+        float tr = fr[h / 4], ti = fi[h / 4];
         mc_pair_f32s<SIGN, OBL>(p[h], vx, vy, vz, inv_lambda, tr, ti);
-        fr += use ? tr : 0.f;
-        fi += use ? ti : 0.f;
+        fr[h / 4] = use ? tr : fr[h / 4];
+        fi[h / 4] = use ? ti : fi[h / 4];
       }
     }
     if constexpr (!FP64) {
-      ar += fr;
-      ai += fi;
+      ar += (double)fr[0] + (double)fr[1];
+      ai += (double)fi[0] + (double)fi[1];
     }
     head += take;
   };
-  for (uint32_t k = 0; k < K; k += 8) {
-    uint32_t idx[8];
+  for (uint32_t k = 0;; k += 8) {
+    const bool more = k < K;
+    if (more) {
+      uint32_t idx[8];
 #pragma unroll
-    for (int h = 0; h < 4; ++h) {
-      const U4 o = mc_draws<false>(k + 2 * h, mm, seed_lo, seed_hi);
-      idx[2 * h] = lemire_index(o.x, o.y, N);
-      idx[2 * h + 1] = lemire_index(o.z, o.w, N);
-    }
-#pragma unroll
-    for (int h = 0; h < 8; ++h)
-      if (active && k + h < K && idx[h] - lo < hi - lo) {
-        s_q[tail & (kMcQueue - 1)][t] = idx[h];
-        ++tail;
+      for (int h = 0; h < 4; ++h) {
+        const U4 o = mc_draws<false>(k + 2 * h, m, seed_lo, seed_hi);
+        idx[2 * h] = lemire_index(o.x, o.y, N);
+        idx[2 * h + 1] = lemire_index(o.z, o.w, N);
       }
-    // full batches while every active lane holds 8 (idle lanes count as full)
-    while (__builtin_amdgcn_ballot_w64(active && tail - head < 8) == 0) batch(8);
-    // every ring holds at most kMcQueue - 8 entries before the next round
-    if (__builtin_amdgcn_ballot_w64(active && tail - head > kMcQueue - 8))
-      batch(min(8u, tail - head));
+      const uint32_t width = active ? hi - lo : 0u;
+#pragma unroll
+      for (int h = 0; h < 8; ++h)
+        if (k + h < K && idx[h] - lo < width) {
+          slot(tail) = idx[h];
+          tail += kStep;
+        }
+      // full batches while every active lane holds 8 (idle lanes count as full)
+      while (__builtin_amdgcn_ballot_w64(active && tail - head < 8 * kStep) == 0)
+        batch(std::true_type{});
+    }
+    // every ring holds at most kMcQueue - 8 entries before the next round, none
+    // after the last
+    while (__builtin_amdgcn_ballot_w64(
+               active && tail - head > (more ? (kMcQueue - 8) * kStep : 0u)) != 0)
+      batch(std::false_type{});
+    if (!more) break;
   }
-  while (__builtin_amdgcn_ballot_w64(active && tail != head)) batch(min(8u, tail - head));
+}
+
+template <bool STAGE, int SIGN, bool FP64, bool OBL>
+__global__ __launch_bounds__(kBlock) void k_mc_pass(
+    const double4* __restrict__ pos, const double* __restrict__ ph, uint32_t N,
+    const double* __restrict__ v, uint32_t M, uint32_t K, uint32_t seed_lo, uint32_t seed_hi,
+    double Kw, double inv_lambda, McLattice lat, uint32_t b0, uint32_t b1, uint32_t passes,
+    uint32_t widest, int staged, double scale, double2* __restrict__ y) {
+  __shared__ uint32_t s_q[kMcQueue * kBlock];
+  // (without the tables five workgroups' rings fill a CU's LDS)
+  double* s_tab = nullptr;
+  if constexpr (STAGE) {
+    __shared__ double tab[kMcTable];
+    s_tab = tab;
+  }
+  McSourceView source(pos, lat, FP64, N);
+  if (widest && source.stages(widest) != (staged != 0)) return;  // uniform
+  const uint32_t m = blockIdx.x * kBlock + threadIdx.x;
+  const bool active = m < M, idle = __ballot(active) == 0;  // idle: the whole wave is past M
+  const uint32_t mm = active ? m : M - 1;
+  const double vx = v[3 * (size_t)mm], vy = v[3 * (size_t)mm + 1], vz = v[3 * (size_t)mm + 2];
+  double ar = 0.0, ai = 0.0;
+  for (uint32_t b = b0; b < b1; ++b) {
+    const uint32_t lo = (uint32_t)((uint64_t)b * N / passes);
+    const uint32_t hi = (uint32_t)((uint64_t)(b + 1) * N / passes);
+    if constexpr (STAGE) {
+      __syncthreads();  // the previous range's reads are done
+      source.stage(lo, hi, s_tab);
+    }
+    if (idle) continue;
+    const auto run = [&](auto view) __attribute__((always_inline)) {
+      mc_pass<view.value, SIGN, FP64, OBL>(source, ph, N, vx, vy, vz, active, mm, K, seed_lo,
+                                           seed_hi, Kw, inv_lambda, lo, hi, s_q, ar, ai);
+    };
+    if constexpr (STAGE)
+      run(std::integral_constant<McView, kMcStaged>{});
+    else
+      with_view<FP64>(source, N, run);
+  }
   if (active) {
-    if (!first) {
+    if (b0) {
       const double2 old = y[m];
       ar += old.x;
       ai += old.y;
     }
+    if (b1 < passes) scale = 1.0;
     y[m] = make_double2(ar * scale, ai * scale);
   }
 }
@@ -935,14 +1049,12 @@ __global__ __launch_bounds__(kBlock) void k_mc_shared(
   }
 }
 
-uint32_t mc_passes(size_t N, bool fp64) {
+// Ranges of about `per_pass` bytes over `bytes` gathered (at most 8; option
+// "mc_passes" sets the number).
+static uint32_t mc_passes(size_t N, size_t bytes, size_t per_pass) {
   const int opt = tuning().mc_passes;
   if (opt > 0) return (uint32_t)std::min<size_t>((size_t)opt, std::max<size_t>(N, 1));
-  // the gathered bytes per source: the FP32 weight on a lattice (the records
-  // of other point sets are 4x larger and get 4x fuller ranges), or the FP64
-  // record and phase
-  const size_t bytes = N * (fp64 ? 40 : 8);
-  const size_t p = (bytes + kMcPassBytes - 1) / kMcPassBytes;
+  const size_t p = (bytes + per_pass - 1) / per_pass;
   return (uint32_t)std::min<size_t>(std::max<size_t>(p, 1), 8);
 }
 
@@ -956,25 +1068,57 @@ hipError_t launch_mc(int sign, bool fp64, bool shared, bool obliquity, const dou
   const double il = 1.0 / lambda;
   const unsigned blocks = shared ? (unsigned)((M + kMcGroup - 1) / kMcGroup)
                                  : (unsigned)((M + kBlock - 1) / kBlock);
-  const uint32_t passes = shared ? 1u : mc_passes(N, fp64);
+  const bool round = blocks <= kMcRound;
+  const uint64_t draws = (uint64_t)M * K;
+  // FP64 gathers 40 bytes per draw.  FP32-split sources gather 8 on a lattice; off it
+  // 32, which take ranges of their own where the draws pay for them.
+  const size_t mb = size_t(1) << 20;
+  uint32_t passes;
+  if (fp64)
+    passes = std::min(mc_passes(N, 40 * N, 3 * mb), round ? 3u : 8u);
+  else if (!round && draws >= kMcRecordDraws)
+    passes = mc_passes(N, 32 * N, 4 * mb);
+  else
+    passes = mc_passes(N, 8 * N, 3 * mb);
+  const bool apart = !fp64 && lat.info && passes > 1 &&
+                     draws >= (round ? kMcStageDraws / 8 : kMcStageDraws);
   with_sign(sign, [&](auto sg) {
     with_bool(fp64, [&](auto f64) {
       with_bool(obliquity, [&](auto obl) {
-        if (shared)
+        if (shared) {
           k_mc_shared<sg.value, (bool)f64.value, (bool)obl.value><<<blocks, kBlock, 0, stream>>>(
               pos, ph, (uint32_t)N, v, (uint32_t)M, K, slo, shi, K_wave, il, scale, y);
-        else if (passes <= 1)
-          k_mc<sg.value, (bool)f64.value, (bool)obl.value, false>
-              <<<blocks, kBlock, 0, stream>>>(pos, ph, (uint32_t)N, v, (uint32_t)M, nullptr, K,
-                                              K + (K & 1u), slo, shi, K_wave, il, scale, lat, y);
-        else
-          for (uint32_t b = 0; b < passes; ++b)
-            k_mc_pass<sg.value, (bool)f64.value, (bool)obl.value>
-                <<<blocks, kBlock, 0, stream>>>(
-                    pos, ph, (uint32_t)N, v, (uint32_t)M, K, slo, shi, K_wave, il, lat,
-                    (uint32_t)((uint64_t)b * N / passes),
-                    (uint32_t)((uint64_t)(b + 1) * N / passes), b == 0 ? 1 : 0,
-                    b + 1 == passes ? scale : 1.0, y);
+          return;
+        }
+        // widest: 0, or the width of the staged ranges, and the launch is for the
+        // sources that can (`staged`) or cannot be staged and exits on the others
+        const auto ranges = [&](auto stage, uint32_t passes, uint32_t widest, bool staged) {
+          if (passes <= 1)
+            k_mc<sg.value, (bool)f64.value, (bool)obl.value, false>
+                <<<blocks, kBlock, 0, stream>>>(pos, ph, (uint32_t)N, v, (uint32_t)M, nullptr, K,
+                                                K + (K & 1u), slo, shi, K_wave, il, scale, lat,
+                                                K >= kMcStageK ? 1 : 0, widest ? 1 : 0, y);
+          else
+            for (uint32_t b = 0; b < passes; b = round ? passes : b + 1)
+              k_mc_pass<(bool)stage.value, sg.value, (bool)f64.value, (bool)obl.value>
+                  <<<blocks, kBlock, 0, stream>>>(pos, ph, (uint32_t)N, v, (uint32_t)M, K, slo,
+                                                  shi, K_wave, il, lat, b,
+                                                  round ? passes : b + 1, passes, widest,
+                                                  staged ? 1 : 0, scale, y);
+        };
+        if constexpr (!(bool)f64.value) {
+          if (apart) {
+            const uint32_t staged = mc_passes(N, 8 * N, 4 * mb);
+            const uint32_t widest = (uint32_t)((N + staged - 1) / staged);
+            if (lat.use)
+              ranges(std::true_type{}, staged, widest, true);
+            else
+              ranges(std::false_type{}, staged, widest, true);
+            ranges(std::false_type{}, passes, widest, false);
+            return;
+          }
+        }
+        ranges(std::false_type{}, passes, 0u, false);
       });
     });
   });
@@ -1006,7 +1150,7 @@ hipError_t launch_mc_subset(int sign, bool shared, bool obliquity, const double4
             <<<dim3(blocks, S), kBlock, 0, stream>>>(pos, ph, (uint32_t)N, vsub,
                                                      (uint32_t)count, tmap, K, chunk, slo, shi,
                                                      K_wave, 1.0 / lambda, scale, McLattice{},
-                                                     out);
+                                                     0, 0, out);
       });
     });
   });
@@ -1112,7 +1256,7 @@ __global__ __launch_bounds__(kBlock) void k_mc_indices(
   if (j >= count) return;
   const uint32_t m = m0 + j;
   for (uint32_t k = 0; k < K; k += 2) {
-    const U4 o = philox4x32_10(U4{k >> 1, m, tag, kMcStream}, seed_lo, seed_hi);
+    const U4 o = philox4x32_10<true>(U4{k >> 1, m, tag, kMcStream}, seed_lo, seed_hi);
     idx[(size_t)j * K + k] = lemire_index(o.x, o.y, (uint32_t)N);
     if (k + 1 < K) idx[(size_t)j * K + k + 1] = lemire_index(o.z, o.w, (uint32_t)N);
   }

@@ -131,8 +131,7 @@ holo_status holo_synchronize(holo_ctx *ctx);
  * pairs take the x of their row and the y of their column from tables of
  * the lattice's rows and columns, dx^2 once per row, instead of each
  * source's position; same bits; default 1), "mc_passes"
- * (per-target Monte Carlo: source ranges, one launch each, 0 = automatic,
- * 1 = one launch), "mc_lattice" (0/1: per-target
+ * (per-target Monte Carlo: source ranges, taken in turn, 0 = automatic), "mc_lattice" (0/1: per-target
  * FP32-split Monte Carlo on product-grid sources reads positions from row
  * and column tables; same results; default 1).  Results do not depend on them beyond summation order and, for "grid",
  * "grid16", "grid32", "grid64" and "grid_pairs", the FP32-split rounding (all paths stay within
