@@ -37,7 +37,7 @@ HIP_FLAGS = [
     f"-I{INCLUDE}",
 ]
 LIB_SOURCES = ["holo_kernels.hip", "holo_grid.hip", "holo_pairs.hip",
-               "holo_points.hip", "holo_capi.hip"]
+               "holo_points.hip", "holo_lattice.hip", "holo_capi.hip"]
 
 
 def hipcc() -> str:

@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <numeric>
 #include <string>
@@ -75,7 +76,10 @@ holo_status ensure(DevBuf& b, size_t bytes, int device) {
 
 }  // namespace
 
+struct holo_plan;
+
 struct holo_ctx {
+  ~holo_ctx();
   int device = 0;
   hipStream_t stream = nullptr;
   bool own_stream = false;
@@ -87,6 +91,9 @@ struct holo_ctx {
   DevBuf pos64, ph64;            // FP64 Monte Carlo records for the error report
   // recorded on the previous stream when holo_set_stream switches streams
   hipEvent_t switched = nullptr;
+  // FP32-split calls without a plan: the buffers of the last one (about 120 bytes a
+  // source, at most kShotSources of them)
+  std::unique_ptr<holo_plan> shot;
 };
 
 struct holo_plan {
@@ -153,7 +160,18 @@ struct holo_plan {
       (void)hipSetDevice(cur);
     }
   }
+  // No sources and no tiles; the buffers stay.
+  void clear() {
+    N = row = n_tiles = 0;
+    uniform_z = tiles_built = false;
+    planar = true;
+    max_offset = 0.0;
+    grid_tiles = g16_tiles = g16_tail = g32_tiles = g64_tiles = 0;
+    pp = holo::PairPlan();
+  }
 };
+
+holo_ctx::~holo_ctx() = default;
 
 namespace {
 
@@ -542,8 +560,45 @@ struct HostGrid {
   double cx0_64 = INFINITY, cx1_64 = -INFINITY, cy0_64 = INFINITY, cy1_64 = -INFINITY;
   float rho64_y = 0;
   std::vector<double4> centre64;
-  std::vector<int32_t> tail;  // sources after the lattice (padded lattices)
+  size_t n16 = 0, n32 = 0, n64 = 0;  // tiles of each width
+  size_t n_tail = 0;  // sources after the lattice (padded lattices)
+  bool tail_same = true;  // all at one place
 };
+
+// The 16-row tiles of a lattice of g.nx x g.ny sources: counts, bounds and radii.
+void grid16_shape(double x0, double y0, double px, double py, HostGrid& g) {
+  g.px = px;
+  g.py = py;
+  g.rho16_x = std::nextafter((float)(7.5 * std::fabs(px)), INFINITY);
+  g.rho16_y = std::nextafter((float)(7.5 * std::fabs(py)), INFINITY);
+  // an odd number of tile columns (5 or more) takes one more, of padding only,
+  // so that they pair into 16 x 32 tiles (1000 columns: 64 instead of 63)
+  const size_t TI = (g.nx + 15) / 16, TJ = (g.ny + 15) / 16 + ((g.ny + 15) / 16 % 2 && g.ny > 64);
+  g.tj16 = TJ;
+  const auto ends = [](double o, double p, size_t n, double width, double& lo, double& hi) {
+    const double a = o + 0.5 * (width - 1) * p;
+    const double b = o + (width * (double)(n - 1) + 0.5 * (width - 1)) * p;
+    lo = std::min(a, b);
+    hi = std::max(a, b);
+  };
+  g.n16 = TI * TJ;
+  ends(x0, px, TI, 16, g.cx0_16, g.cx1_16);
+  ends(y0, py, TJ, 16, g.cy0_16, g.cy1_16);
+  if (TJ % 2) return;
+  g.rho32_y = std::nextafter((float)(15.5 * std::fabs(py)), INFINITY);
+  g.n32 = TI * TJ / 2;
+  g.cx0_32 = g.cx0_16;
+  g.cx1_32 = g.cx1_16;
+  ends(y0, py, TJ / 2, 32, g.cy0_32, g.cy1_32);
+  // quads of tiles 4T .. 4T + 3: 16 x 64 tiles centred at
+  // x_0 + (16I + 7.5) p_x, y_0 + (64J' + 31.5) p_y (no extra padding for them)
+  if (TJ % 4) return;
+  g.rho64_y = std::nextafter((float)(31.5 * std::fabs(py)), INFINITY);
+  g.n64 = TI * TJ / 4;
+  g.cx0_64 = g.cx0_16;
+  g.cx1_64 = g.cx1_16;
+  ends(y0, py, TJ / 4, 64, g.cy0_64, g.cy1_64);
+}
 
 // Sides that are not multiples of 16 are padded to the next multiple with
 // weight-0 slots (perm -1) at the lattice points beyond the edge.
@@ -557,65 +612,33 @@ void build_grid16(const double* u, HostGrid& g) {
     if (!(std::fabs(u[3 * i * ny] - (x0 + (double)i * px)) <= 1e-9 * std::fabs(px))) return;
   for (size_t j = 0; j < ny; ++j)
     if (!(std::fabs(u[3 * j + 1] - (y0 + (double)j * py)) <= 1e-9 * std::fabs(py))) return;
-  g.px = px;
-  g.py = py;
-  g.rho16_x = std::nextafter((float)(7.5 * std::fabs(px)), INFINITY);
-  g.rho16_y = std::nextafter((float)(7.5 * std::fabs(py)), INFINITY);
-  const float2 rho{g.rho16_x, g.rho16_y};
-  // an odd number of tile columns (5 or more) takes one more, of padding only,
-  // so that they pair into 16 x 32 tiles (1000 columns: 64 instead of 63)
-  const size_t TI = (nx + 15) / 16, TJ = (ny + 15) / 16 + ((ny + 15) / 16 % 2 && ny > 64);
-  g.centre16.reserve(TI * TJ);
-  g.perm16.reserve(256 * TI * TJ);
-  g.tj16 = TJ;
+  grid16_shape(x0, y0, px, py, g);
+  const size_t TJ = g.tj16, TI = g.n16 / TJ;
+  const auto centres = [&](std::vector<double4>& c, size_t n, size_t width, float rho_y) {
+    const float2 rho{g.rho16_x, rho_y};
+    const size_t cols = n / TI;
+    c.reserve(n);
+    for (size_t t = 0; t < n; ++t) {
+      const size_t I = t / cols, J = t % cols;
+      c.push_back(double4{x0 + ((double)(16 * I) + 7.5) * px,
+                          y0 + ((double)(width * J) + 0.5 * (double)(width - 1)) * py, g.z,
+                          __builtin_bit_cast(double, rho)});
+    }
+  };
+  centres(g.centre16, g.n16, 16, g.rho16_y);
+  centres(g.centre32, g.n32, 32, g.rho32_y);
+  centres(g.centre64, g.n64, 64, g.rho64_y);
+  g.perm16.reserve(256 * g.n16);
   g.axes16.resize(16 * (TI + TJ));
   for (size_t a = 0; a < 16 * TI; ++a)
     g.axes16[a] = a < nx ? u[3 * a * ny] : x0 + (double)a * px;
   for (size_t b = 0; b < 16 * TJ; ++b)
     g.axes16[16 * TI + b] = b < ny ? u[3 * b + 1] : y0 + (double)b * py;
   for (size_t I = 0; I < TI; ++I)
-    for (size_t J = 0; J < TJ; ++J) {
-      const double cx = x0 + ((double)(16 * I) + 7.5) * px;
-      const double cy = y0 + ((double)(16 * J) + 7.5) * py;
-      g.centre16.push_back(double4{cx, cy, g.z, __builtin_bit_cast(double, rho)});
-      g.cx0_16 = std::min(g.cx0_16, cx);
-      g.cx1_16 = std::max(g.cx1_16, cx);
-      g.cy0_16 = std::min(g.cy0_16, cy);
-      g.cy1_16 = std::max(g.cy1_16, cy);
+    for (size_t J = 0; J < TJ; ++J)
       for (size_t a = 16 * I; a < 16 * I + 16; ++a)
         for (size_t b = 16 * J; b < 16 * J + 16; ++b)
           g.perm16.push_back(a < nx && b < ny ? (int32_t)(a * ny + b) : -1);
-    }
-  if (TJ % 2) return;
-  g.rho32_y = std::nextafter((float)(15.5 * std::fabs(py)), INFINITY);
-  const float2 rho32{g.rho16_x, g.rho32_y};
-  g.centre32.reserve(TI * TJ / 2);
-  for (size_t I = 0; I < TI; ++I)
-    for (size_t J = 0; J < TJ / 2; ++J) {
-      const double cx = x0 + ((double)(16 * I) + 7.5) * px;
-      const double cy = y0 + ((double)(32 * J) + 15.5) * py;
-      g.centre32.push_back(double4{cx, cy, g.z, __builtin_bit_cast(double, rho32)});
-      g.cx0_32 = std::min(g.cx0_32, cx);
-      g.cx1_32 = std::max(g.cx1_32, cx);
-      g.cy0_32 = std::min(g.cy0_32, cy);
-      g.cy1_32 = std::max(g.cy1_32, cy);
-    }
-  // quads of tiles 4T .. 4T + 3: 16 x 64 tiles centred at
-  // x_0 + (16I + 7.5) p_x, y_0 + (64J' + 31.5) p_y (no extra padding for them)
-  if (TJ % 4) return;
-  g.rho64_y = std::nextafter((float)(31.5 * std::fabs(py)), INFINITY);
-  const float2 rho64{g.rho16_x, g.rho64_y};
-  g.centre64.reserve(TI * TJ / 4);
-  for (size_t I = 0; I < TI; ++I)
-    for (size_t J = 0; J < TJ / 4; ++J) {
-      const double cx = x0 + ((double)(16 * I) + 7.5) * px;
-      const double cy = y0 + ((double)(64 * J) + 31.5) * py;
-      g.centre64.push_back(double4{cx, cy, g.z, __builtin_bit_cast(double, rho64)});
-      g.cx0_64 = std::min(g.cx0_64, cx);
-      g.cx1_64 = std::max(g.cx1_64, cx);
-      g.cy0_64 = std::min(g.cy0_64, cy);
-      g.cy1_64 = std::max(g.cy1_64, cy);
-    }
 }
 
 bool build_grid(const double* u, size_t N, HostGrid& g) {
@@ -716,8 +739,13 @@ bool build_grid16_padded(const double* u, size_t N, HostGrid& g) {
   g.ny = ny;
   g.z = u[2];
   build_grid16(u, g);
-  if (g.centre16.empty()) return false;
-  for (size_t n = body; n < N; ++n) g.tail.push_back((int32_t)n);
+  if (!g.n16) return false;
+  g.n_tail = N - body;
+  for (size_t n = body; n < N; ++n) {
+    g.perm16.push_back((int32_t)n);
+    for (int d = 0; d < 3; ++d)
+      g.tail_same = g.tail_same && u[3 * n + d] == u[3 * body + d];
+  }
   return true;
 }
 
@@ -761,9 +789,12 @@ holo_status plan_build_tiles(holo_ctx* ctx, const holo_plan* p, const double* u_
   return HOLO_OK;
 }
 
-// The 16-row tiles of grid (and their tail), if any, onto the device.
-holo_status upload_grid16(holo_ctx* ctx, holo_plan* p, const HostGrid& grid, const double* u) {
-  const size_t n16 = grid.centre16.size(), nt = grid.tail.size();
+// The 16-row tiles of grid (and their tail), if any, onto the device: from the
+// host's arrays, or cut there when it has none.  x0, y0: source 0.
+holo_status upload_grid16(holo_ctx* ctx, holo_plan* p, const HostGrid& grid, double x0,
+                          double y0) {
+  const size_t n16 = grid.n16, nt = grid.n_tail, ti = n16 ? n16 / grid.tj16 : 0;
+  const bool upload = !grid.perm16.empty();
   if (!n16) return HOLO_OK;
   if (256 * n16 + nt > kMaxCount) return fail(HOLO_EINVAL, "too many tile slots");
   p->g16_tiles = n16;
@@ -783,22 +814,12 @@ holo_status upload_grid16(holo_ctx* ctx, holo_plan* p, const HostGrid& grid, con
   HOLO_TRY(ensure(p->g16_wq, 6 * 64 * n16 * sizeof(uint4), ctx->device));
   HOLO_TRY(ensure(p->g16_wqn, 4 * 64 * n16 * sizeof(uint4), ctx->device));
   HOLO_TRY(ensure(p->g16_ts, n16 * sizeof(float), ctx->device));
-  HOLO_HIP(hipMemcpyAsync(p->g16_centre.ptr, grid.centre16.data(), n16 * sizeof(double4),
-                          hipMemcpyHostToDevice, ctx->stream));
   p->g16_tj = grid.tj16;
   p->g16_nx = grid.nx;
   p->g16_ny = grid.ny;
-  HOLO_TRY(ensure(p->g16_axes, grid.axes16.size() * sizeof(double), ctx->device));
-  HOLO_HIP(hipMemcpyAsync(p->g16_axes.ptr, grid.axes16.data(),
-                          grid.axes16.size() * sizeof(double), hipMemcpyHostToDevice,
-                          ctx->stream));
-  HOLO_HIP(hipMemcpyAsync(p->g16_perm.ptr, grid.perm16.data(), 256 * n16 * sizeof(int32_t),
-                          hipMemcpyHostToDevice, ctx->stream));
-  if (nt)
-    HOLO_HIP(hipMemcpyAsync(static_cast<int32_t*>(p->g16_perm.ptr) + 256 * n16,
-                            grid.tail.data(), nt * sizeof(int32_t), hipMemcpyHostToDevice,
-                            ctx->stream));
-  const size_t n32 = grid.centre32.size();
+  const size_t axes = 16 * (ti + grid.tj16);
+  HOLO_TRY(ensure(p->g16_axes, axes * sizeof(double), ctx->device));
+  const size_t n32 = grid.n32;
   if (n32) {
     p->g32_tiles = n32;
     p->g32_cx0 = grid.cx0_32;
@@ -807,10 +828,8 @@ holo_status upload_grid16(holo_ctx* ctx, holo_plan* p, const HostGrid& grid, con
     p->g32_cy1 = grid.cy1_32;
     p->g32_rho_y = grid.rho32_y;
     HOLO_TRY(ensure(p->g32_centre, n32 * sizeof(double4), ctx->device));
-    HOLO_HIP(hipMemcpyAsync(p->g32_centre.ptr, grid.centre32.data(), n32 * sizeof(double4),
-                            hipMemcpyHostToDevice, ctx->stream));
   }
-  const size_t n64 = grid.centre64.size();
+  const size_t n64 = grid.n64;
   if (n64) {
     p->g64_tiles = n64;
     p->g64_cx0 = grid.cx0_64;
@@ -819,12 +838,46 @@ holo_status upload_grid16(holo_ctx* ctx, holo_plan* p, const HostGrid& grid, con
     p->g64_cy1 = grid.cy1_64;
     p->g64_rho_y = grid.rho64_y;
     HOLO_TRY(ensure(p->g64_centre, n64 * sizeof(double4), ctx->device));
-    HOLO_HIP(hipMemcpyAsync(p->g64_centre.ptr, grid.centre64.data(), n64 * sizeof(double4),
-                            hipMemcpyHostToDevice, ctx->stream));
+  }
+  if (upload) {
+    const auto copy = [&](DevBuf& to, const void* from, size_t bytes) {
+      return bytes ? hipMemcpyAsync(to.ptr, from, bytes, hipMemcpyHostToDevice, ctx->stream)
+                   : hipSuccess;
+    };
+    HOLO_HIP(copy(p->g16_centre, grid.centre16.data(), n16 * sizeof(double4)));
+    HOLO_HIP(copy(p->g32_centre, grid.centre32.data(), n32 * sizeof(double4)));
+    HOLO_HIP(copy(p->g64_centre, grid.centre64.data(), n64 * sizeof(double4)));
+    HOLO_HIP(copy(p->g16_perm, grid.perm16.data(), (256 * n16 + nt) * sizeof(int32_t)));
+    HOLO_HIP(copy(p->g16_axes, grid.axes16.data(), axes * sizeof(double)));
+  } else {
+    const auto rho = [&](float y) {
+      return __builtin_bit_cast(double, float2{grid.rho16_x, y});
+    };
+    holo::LatticeTiles t;
+    t.u = static_cast<const double*>(p->u.ptr);
+    t.nx = (uint32_t)grid.nx;
+    t.ny = (uint32_t)grid.ny;
+    t.ti = (uint32_t)ti;
+    t.tj = (uint32_t)grid.tj16;
+    t.n_tail = (uint32_t)nt;
+    t.x0 = x0;
+    t.y0 = y0;
+    t.z = grid.z;
+    t.px = grid.px;
+    t.py = grid.py;
+    t.rho16 = rho(grid.rho16_y);
+    t.rho32 = rho(grid.rho32_y);
+    t.rho64 = rho(grid.rho64_y);
+    t.perm = static_cast<int32_t*>(p->g16_perm.ptr);
+    t.centre16 = static_cast<double4*>(p->g16_centre.ptr);
+    t.centre32 = n32 ? static_cast<double4*>(p->g32_centre.ptr) : nullptr;
+    t.centre64 = n64 ? static_cast<double4*>(p->g64_centre.ptr) : nullptr;
+    t.axes = static_cast<double*>(p->g16_axes.ptr);
+    HOLO_HIP(holo::launch_lattice_tiles(t, ctx->stream));
   }
   holo::PairPlan& pp = p->pp;
-  pp.x0 = u[0];
-  pp.y0 = u[1];
+  pp.x0 = x0;
+  pp.y0 = y0;
   pp.z = grid.z;
   pp.px = grid.px;
   pp.py = grid.py;
@@ -833,10 +886,7 @@ holo_status upload_grid16(holo_ctx* ctx, holo_plan* p, const HostGrid& grid, con
   pp.tj = (uint32_t)((grid.ny + 63) / 64);
   const size_t np = (grid.nx + 31) / 32 * pp.tj;
   pp.n_tail = (uint32_t)nt;
-  pp.tail_same = true;
-  for (const int32_t n : grid.tail)
-    for (int d = 0; d < 3; ++d)
-      pp.tail_same = pp.tail_same && u[3 * (size_t)n + d] == u[3 * (size_t)grid.tail[0] + d];
+  pp.tail_same = grid.tail_same;
   HOLO_TRY(ensure(p->pr_wq, 1024 * np * sizeof(uint4), ctx->device));
   HOLO_TRY(ensure(p->pr_ts, np * sizeof(float), ctx->device));
   HOLO_TRY(ensure(p->pr_tail, std::max<size_t>(nt, 1) * sizeof(float2), ctx->device));
@@ -877,11 +927,11 @@ holo_status plan_upload_tiles(holo_ctx* ctx, holo_plan* p, const double* u_host)
                             hipMemcpyHostToDevice, ctx->stream));
     HOLO_HIP(hipMemcpyAsync(p->g_perm.ptr, grid.perm.data(), 64 * nt * sizeof(int32_t),
                             hipMemcpyHostToDevice, ctx->stream));
-    HOLO_TRY(upload_grid16(ctx, p, grid, u_host));
+    HOLO_TRY(upload_grid16(ctx, p, grid, u_host[0], u_host[1]));
   } else if (p->tile == 64 && build_grid16_padded(u_host, p->N, grid)) {
     p->grid_nx = grid.nx;
     p->grid_ny = grid.ny;
-    HOLO_TRY(upload_grid16(ctx, p, grid, u_host));
+    HOLO_TRY(upload_grid16(ctx, p, grid, u_host[0], u_host[1]));
   }
   // host vectors are freed on return: wait for the copies
   HOLO_HIP(hipStreamSynchronize(ctx->stream));
@@ -945,11 +995,60 @@ holo_status plan_build(holo_ctx* ctx, holo_plan* p, const double* u, size_t N,
   p->row = row_length(uh, N);
   HOLO_TRY(plan_upload_tiles(ctx, p, uh));
   // the uploads are ordered before a first call on another stream
-  HOLO_HIP(hipEventCreateWithFlags(&p->ran, hipEventDisableTiming));
+  if (!p->ran) HOLO_HIP(hipEventCreateWithFlags(&p->ran, hipEventDisableTiming));
   HOLO_HIP(hipEventRecord(p->ran, ctx->stream));
   p->ran_on = ctx->stream;
   return HOLO_OK;
 }
+
+// plan_build for one call with device positions on a uniform lattice that the 16-row
+// and lattice-to-lattice kernels take, found and cut on the device (*found; else
+// nothing is built).  512^2 sources to 512^2 targets: 2.13 ms with plan_build and a plan's
+// allocations in every call, 0.23 ms with this and the context's own plan.
+holo_status plan_build_lattice(holo_ctx* ctx, holo_plan* p, const double* u, size_t N,
+                               bool* found) {
+  *found = false;
+  const holo::Tuning& tu = holo::tuning();
+  if (N < 64 || !tu.grid || !tu.grid16) return HOLO_OK;
+  HOLO_TRY(ensure(ctx->pairs, 256 + holo::kPairFlags * sizeof(uint32_t), ctx->device));
+  holo::LatticeInfo* di = static_cast<holo::LatticeInfo*>(ctx->pairs.ptr);
+  static_assert(sizeof(holo::LatticeInfo) <= 128, "shares the buffer of PairTargets");
+  HOLO_HIP(holo::launch_find_lattice(u, N, di, ctx->stream));
+  holo::LatticeInfo f;
+  HOLO_HIP(hipMemcpyAsync(&f, di, sizeof(f), hipMemcpyDeviceToHost, ctx->stream));
+  HOLO_HIP(hipStreamSynchronize(ctx->stream));
+  const size_t ny = f.ny, nx = f.rows, body = nx * ny;
+  if (!f.uniform) return HOLO_OK;
+  // as build_grid, else as build_grid16_padded
+  const bool whole = body == N && nx % 8 == 0 && ny % 8 == 0;
+  if (!whole &&
+      (N < 256 || ny < 16 || ny == N || nx < 16 || N - body >= std::max(nx, ny)))
+    return HOLO_OK;
+  p->device = ctx->device;
+  p->N = N;
+  p->tile = 64;
+  p->uniform_z = f.uniform_z != 0;
+  p->row = ny >= 4 && f.in_rows ? ny : 0;
+  HOLO_TRY(ensure(p->u, 3 * N * sizeof(double), ctx->device));
+  HOLO_HIP(hipMemcpyAsync(p->u.ptr, u, 3 * N * sizeof(double), hipMemcpyDeviceToDevice,
+                          ctx->stream));
+  HostGrid g;
+  g.nx = nx;
+  g.ny = ny;
+  g.z = f.z;
+  grid16_shape(f.x0, f.y0, f.px, f.py, g);
+  g.n_tail = N - body;
+  g.tail_same = f.tail_same != 0;
+  HOLO_TRY(upload_grid16(ctx, p, g, f.x0, f.y0));
+  if (!p->ran) HOLO_HIP(hipEventCreateWithFlags(&p->ran, hipEventDisableTiming));
+  HOLO_HIP(hipEventRecord(p->ran, ctx->stream));
+  p->ran_on = ctx->stream;
+  *found = true;
+  return HOLO_OK;
+}
+
+// Up to this many the context keeps the buffers of a call without a plan (0.5 GB).
+constexpr size_t kShotSources = size_t(1) << 22;
 
 // Up to this many sources a call prepares the weights of both lattice paths in
 // one launch: a second launch costs 3 us (also when it has nothing to do), the
@@ -1386,13 +1485,20 @@ holo_status holo_transform_full(holo_ctx* ctx, holo_precision precision, int sig
                                           ctx->stream));
     }
   } else {
-    holo_plan plan;
-    HOLO_TRY(plan_build(ctx, &plan, u, N, 0, dev));
-    HOLO_TRY(plan_run(ctx, &plan, precision, sign, obl, lambda, holo::kPolar, da, dp, dv, M,
+    // a plan for this call, built anew in the buffers of the context's last one
+    std::unique_ptr<holo_plan> own;
+    if (N > kShotSources) own.reset(new holo_plan);
+    if (!own && !ctx->shot) ctx->shot.reset(new holo_plan);
+    holo_plan* plan = own ? own.get() : ctx->shot.get();
+    plan->clear();
+    bool found = false;
+    if (dev) HOLO_TRY(plan_build_lattice(ctx, plan, u, N, &found));
+    if (!found) HOLO_TRY(plan_build(ctx, plan, u, N, 0, dev));
+    HOLO_TRY(plan_run(ctx, plan, precision, sign, obl, lambda, holo::kPolar, da, dp, dv, M,
                       dy));
     HOLO_TRY(report_error(ctx, false, dv, M, dy, err_rel_l2, dev,
                           [&](const ErrScratch& e, size_t count) {
-                            return plan_fp64_at(ctx, &plan, sign, obl, lambda, holo::kPolar, da,
+                            return plan_fp64_at(ctx, plan, sign, obl, lambda, holo::kPolar, da,
                                                 dp, e, count);
                           }));
     HOLO_HIP(hipStreamSynchronize(ctx->stream));  // plan buffers die here
@@ -1712,7 +1818,7 @@ holo_status holo_lattice_layout(const double* u, size_t N, size_t* nx, size_t* n
   if (N && build_grid(u, N, g)) {
     t16 = !g.centre16.empty();
   } else if (N && build_grid16_padded(u, N, g)) {
-    t = g.tail.size();
+    t = g.n_tail;
     t16 = true;
   } else {
     g = HostGrid();

@@ -311,6 +311,27 @@ struct McLattice {
   bool use = true;  // false: every source from its record, over the same ranges
 };
 
+// A uniform lattice found by launch_find_lattice: rows of ny sources (0: no such
+// row), `rows` of them leading and complete, `uniform` their pitches.
+constexpr uint32_t kLatticeFindRow = 65536;
+struct LatticeInfo {
+  uint32_t ny, rows, uniform, uniform_z, in_rows, tail_same;
+  double x0, y0, z, px, py;
+};
+hipError_t launch_find_lattice(const double* u, size_t N, LatticeInfo* info, hipStream_t stream);
+// ti x tj tiles of 16 x 16; rho*: the packed half-sizes; centre32, centre64: may be NULL.
+struct LatticeTiles {
+  const double* u;
+  uint32_t nx, ny, ti, tj, n_tail;
+  double x0, y0, z, px, py, rho16, rho32, rho64;
+  int32_t* perm;
+  double4* centre16;
+  double4* centre32;
+  double4* centre64;
+  double* axes;
+};
+hipError_t launch_lattice_tiles(const LatticeTiles& a, hipStream_t stream);
+
 // Per-target Monte Carlo runs over source ranges whose gathered data one XCD's 4 MB
 // L2 holds (1024^2 targets, K = 1024, in us: 1024^2 lattice 8920 / 4210 / 4340 / 4860
 // in 1 / 2 / 3 / 4 ranges of its 8 MB of weights; jittered 14300 / 8010 / 7550 in
