@@ -349,7 +349,7 @@ size_t split_elems_f64(size_t M, size_t N) {
 
 size_t split_elems_f32(size_t M, size_t n_tiles) {
   const int R = holo::tuning().r_f32;
-  const int S = n_tiles ? holo::choose_splits(M, R == 1 || R == 4 ? R : 2, n_tiles, 64) : 1;
+  const int S = holo::tile_splits(M, R == 1 || R == 4 ? R : 2, n_tiles);
   return S > 1 ? (size_t)S * M : 0;
 }
 
@@ -1079,7 +1079,7 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
     // that the call is done.  (Options that pick a 16-row tile shape keep it.)
     const uint32_t* skip = nullptr;
     int Sp = 1;
-    const int S16 = holo::grid_splits(M, quads ? p->g64_tiles : (pairs ? p->g32_tiles : nt));
+    const int S16 = holo::grid_splits(M, quads ? p->g64_tiles : (pairs ? p->g32_tiles : nt), nkc);
     const holo::Tuning& tu = holo::tuning();
     holo::Grid16Prep prep;
     prep.wf = (int)wf;
@@ -1186,7 +1186,7 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
     gt.z = p->grid_z;
     gt.rho_x = p->grid_rho_x;
     gt.rho_y = p->grid_rho_y;
-    const int S = holo::grid_splits(M, nt);
+    const int S = holo::grid_splits(M, nt, 1);
     const size_t pe = S > 1 ? (size_t)S * M : 0;
     if (pe) HOLO_TRY(ensure(ctx->partial, pe * sizeof(double2), ctx->device));
     HOLO_HIP(holo::launch_superpose_grid(sign, obliquity, gt,

@@ -335,8 +335,11 @@ __global__ __launch_bounds__(kBlock) void k_superpose_grid(
   if (mo < M) out[(size_t)blockIdx.y * M + mo] = make_double2(sr, si);
 }
 
-int grid_splits(size_t M, size_t n_tiles) {
-  return n_tiles ? choose_splits(M, 1, n_tiles, 16) : 1;
+int grid_splits(size_t M, size_t n_tiles, int group) {
+  // below 32 tiles of 16 x 16 the reduction's launch costs what the splits give
+  if (n_tiles * group < 32) return 1;
+  return choose_splits(M, 1, n_tiles, M < kFillTargets ? (group == 4 ? 1 : 16 / group) : 16,
+                       kTileSplits);
 }
 
 hipError_t launch_superpose_grid(int sign, bool obliquity, const GridTiles& gt,
@@ -345,7 +348,7 @@ hipError_t launch_superpose_grid(int sign, bool obliquity, const GridTiles& gt,
                                  double lambda, double2* y, double2* partial,
                                  size_t partial_cap, hipStream_t stream) {
   if (M == 0) return hipSuccess;
-  int S = grid_splits(M, gt.n_tiles);
+  int S = grid_splits(M, gt.n_tiles, 1);
   while (S > 1 && (size_t)S * M > partial_cap) --S;
   const uint32_t chunk = gt.n_tiles ? (gt.n_tiles + S - 1) / S : 0;
   const dim3 grid((unsigned)((M + kBlock - 1) / kBlock), (unsigned)S);
@@ -1065,7 +1068,7 @@ hipError_t launch_superpose_grid16(int sign, bool obliquity, int nkc, const Grid
   if (nkc == 4 && (pairs.n_tiles != 2 * gt.n_tiles || !pairs.centre))
     return hipErrorInvalidValue;
   if (gt.n_tail && (!gt.tail_perm || !gt.tail_wc)) return hipErrorInvalidValue;
-  int S = grid_splits(M, gt.n_tiles);
+  int S = grid_splits(M, gt.n_tiles, nkc);
   while (S > 1 && (size_t)S * M > partial_cap) --S;
   const uint32_t chunk = gt.n_tiles ? (gt.n_tiles + S - 1) / S : 0;
   const dim3 grid((unsigned)((M + kBlock - 1) / kBlock), (unsigned)S);
@@ -1108,8 +1111,7 @@ hipError_t launch_superpose_grid16(int sign, bool obliquity, int nkc, const Grid
   });
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  if (skip) return launch_reduce_either(partial, skip, Sp, S, M, y, stream);
-  return launch_reduce_partials(S, M, partial, y, stream);
+  return launch_reduce_partials(S, M, partial, y, stream, skip, Sp);
 }
 
 }  // namespace holo

@@ -112,6 +112,15 @@ inline void with_r(int R, F&& f) {
 int choose_splits(size_t M, int R, size_t units, size_t min_units_per_split,
                   size_t max_splits = 64);
 
+// Source splits of the tiled kernel (tiles of at most 64 sources) and, grid_splits,
+// of the lattice kernels (tiles of 16 x 16 group): down to a tile each while M targets
+// (a lane each) leave the chip idle, runs of at least 64 and 16 tiles above.  Pairs
+// too near for the GEMM forms, 256^2 sources, in us with runs at every size and now:
+// jittered to 16^2, 64^2 and 128^2 targets 900, 1130, 1380 and 125, 300, 800; lattice
+// to the same 734, 986, 767 and 106, 203, 558; 64^2 jittered to 64^2 1189 and 52.
+constexpr size_t kTileSplits = 128, kFillTargets = size_t(1) << 18;
+int tile_splits(size_t M, int R, size_t n_tiles);
+
 // Targets per lane and source splits of an FP64 launch.
 struct F64Shape {
   int R, S;
@@ -147,9 +156,11 @@ hipError_t launch_superpose_f64_auto(int sign, WeightForm wf, bool obliquity,
                                      size_t N, const double* v, size_t M, double K, double2* y,
                                      double2* partial, size_t partial_cap, hipStream_t stream);
 
-// y[m] = sum_s partial[s*M + m] in fixed order (nothing to do for S <= 1).
+// y[m] = sum_s partial[s*M + m] in fixed order (nothing to do for S <= 1).  With
+// `handled` (device): over Sp splits when it is set, else S.
 hipError_t launch_reduce_partials(int S, size_t M, const double2* partial, double2* y,
-                                  hipStream_t stream);
+                                  hipStream_t stream, const uint32_t* handled = nullptr,
+                                  int Sp = 1);
 
 // FP32-split: weights wc (float2 per slot, polar: launch_tile_weights with
 // polar_out), tiles as above.  skip, Sp: as launch_superpose_grid16, for the
@@ -217,7 +228,7 @@ hipError_t launch_superpose_grid16(int sign, bool obliquity, int nkc, const Grid
                                    size_t partial_cap, hipStream_t stream,
                                    const uint32_t* skip = nullptr, int Sp = 1);
 // Source splits the lattice kernel uses for M targets over n_tiles tiles.
-int grid_splits(size_t M, size_t n_tiles);
+int grid_splits(size_t M, size_t n_tiles, int group);
 
 // Lattice-to-lattice kernel (holo_pairs.hip): the sources of a uniform lattice
 // x0 + i px, y0 + j py, z (n = i ny + j, i < nx, j < ny), cut into 32 x 64 tiles
@@ -276,11 +287,6 @@ hipError_t launch_superpose_points(int sign, bool obliquity, const PointPlan& pp
                                    const double* w0, const double* w1, const double* v, size_t M,
                                    double lambda, int S, PairTargets* pt, uint32_t* flags,
                                    uint32_t* handled, double2* out, hipStream_t stream);
-
-// y = the sum of partial's Sp splits when *handled, else of its Sg splits
-// (nothing where that is one: y holds the result).
-hipError_t launch_reduce_either(const double2* partial, const uint32_t* handled, int Sp, int Sg,
-                                size_t M, double2* y, hipStream_t stream);
 
 // wc[slot] = a e^{i phi} (polar input) or w (cartesian input) of source
 // perm[slot] as (re, im); with polar_out as (|w|, arg w / 2 pi in [-1/2, 1/2)).

@@ -52,6 +52,11 @@ int choose_splits(size_t M, int R, size_t units, size_t min_units, size_t max_sp
   return (int)std::max<size_t>(S, 1);
 }
 
+int tile_splits(size_t M, int R, size_t n_tiles) {
+  if (!n_tiles) return 1;
+  return choose_splits(M, R, n_tiles, M < kFillTargets * R ? 1 : 64, kTileSplits);
+}
+
 // 1024 sources on 4096 targets: 367 us as 4 workgroups, 15 us by this rule; 7680 on
 // 30000: 499 and 270 us; 65536 on 262144: 15.7 ms (16 splits) and 15.1 - 15.7 ms.
 // Launch shape of the FP64 kernel: the targets per lane R (at most r_f64) and source
@@ -285,10 +290,17 @@ __global__ __launch_bounds__(kBlock) void k_superpose_f64_auto(
                                                           out, s_tab);
 }
 
+// The splits to sum (`handled`: launch_reduce_partials).
+__device__ __forceinline__ uint32_t splits_of(const uint32_t* handled, uint32_t Sp, uint32_t S) {
+  return handled && *handled ? Sp : S;
+}
+
 // One thread per target, the splits in order, eight loads in flight.
 __global__ __launch_bounds__(kBlock) void k_reduce_partials(
-    const double2* __restrict__ partial, uint32_t S, uint32_t M,
-    double2* __restrict__ y) {
+    const double2* __restrict__ partial, const uint32_t* __restrict__ handled, uint32_t Sp,
+    uint32_t Sg, uint32_t M, double2* __restrict__ y) {
+  const uint32_t S = splits_of(handled, Sp, Sg);
+  if (S <= 1) return;  // that split wrote y
   const uint32_t m = blockIdx.x * kBlock + threadIdx.x;
   if (m < M) y[m] = sum_splits(partial + m, S, M);
 }
@@ -296,8 +308,11 @@ __global__ __launch_bounds__(kBlock) void k_reduce_partials(
 // Fewer targets than fill the GPU: 32 targets by 8 ranges of splits per workgroup,
 // each range summed in order, then the ranges.
 __global__ __launch_bounds__(kBlock) void k_reduce_partials_few(
-    const double2* __restrict__ partial, uint32_t S, uint32_t M, double2* __restrict__ y) {
+    const double2* __restrict__ partial, const uint32_t* __restrict__ handled, uint32_t Sp,
+    uint32_t Sg, uint32_t M, double2* __restrict__ y) {
   __shared__ double2 s_part[8][32];
+  const uint32_t S = splits_of(handled, Sp, Sg);
+  if (S <= 1) return;
   const uint32_t t = threadIdx.x & 31, q = threadIdx.x >> 5;
   const uint32_t m = blockIdx.x * 32 + t;
   const uint32_t a = q * S / 8, b = (q + 1) * S / 8;
@@ -318,9 +333,11 @@ __global__ __launch_bounds__(kBlock) void k_reduce_partials_few(
 // ... in order, then a fixed tree over the lanes, so the order is set by S
 // alone.
 __global__ __launch_bounds__(kBlock) void k_reduce_partials_wide(
-    const double2* __restrict__ partial, uint32_t S, uint32_t M,
-    double2* __restrict__ y) {
+    const double2* __restrict__ partial, const uint32_t* __restrict__ handled, uint32_t Sp,
+    uint32_t Sg, uint32_t M, double2* __restrict__ y) {
   __shared__ double s_re[kBlock], s_im[kBlock];
+  const uint32_t S = splits_of(handled, Sp, Sg);
+  if (S <= 1) return;
   const uint32_t m = blockIdx.x, t = threadIdx.x;
   double re = 0.0, im = 0.0;
   for (uint32_t s = t; s < S; s += kBlock) {
@@ -345,22 +362,21 @@ __global__ __launch_bounds__(kBlock) void k_reduce_partials_wide(
 // targets, 64 splits: 17.9 us; by ranges 5.5 us).
 constexpr size_t kReduceFew = 131072;
 
+// The form is chosen by S, so that a call's bits do not depend on a path that was
+// tried before (Sp splits, when *handled).
 hipError_t launch_reduce_partials(int S, size_t M, const double2* partial, double2* y,
-                                  hipStream_t stream) {
-  if (S <= 1 || M == 0) return hipSuccess;
-  if (M <= 4096 && S >= 64) {
-    k_reduce_partials_wide<<<(unsigned)M, kBlock, 0, stream>>>(partial, (uint32_t)S,
-                                                               (uint32_t)M, y);
-    return hipGetLastError();
-  }
-  if (M <= kReduceFew && S >= 8) {
-    k_reduce_partials_few<<<(unsigned)((M + 31) / 32), kBlock, 0, stream>>>(
-        partial, (uint32_t)S, (uint32_t)M, y);
-    return hipGetLastError();
-  }
-  const unsigned blocks = (unsigned)((M + kBlock - 1) / kBlock);
-  k_reduce_partials<<<blocks, kBlock, 0, stream>>>(partial, (uint32_t)S,
-                                                   (uint32_t)M, y);
+                                  hipStream_t stream, const uint32_t* handled, int Sp) {
+  if (!handled) Sp = S;
+  if (std::max(S, Sp) <= 1 || M == 0) return hipSuccess;
+  const size_t by = S > 1 ? S : Sp;
+  const uint32_t s = (uint32_t)S, sp = (uint32_t)Sp, m = (uint32_t)M;
+  if (M <= 4096 && by >= 64)
+    k_reduce_partials_wide<<<m, kBlock, 0, stream>>>(partial, handled, sp, s, m, y);
+  else if (M <= kReduceFew && by >= 8)
+    k_reduce_partials_few<<<(m + 31) / 32, kBlock, 0, stream>>>(partial, handled, sp, s, m, y);
+  else
+    k_reduce_partials<<<(unsigned)((M + kBlock - 1) / kBlock), kBlock, 0, stream>>>(
+        partial, handled, sp, s, m, y);
   return hipGetLastError();
 }
 
@@ -596,7 +612,7 @@ hipError_t launch_superpose_f32s(int sign, bool obliquity, const TileSet& ts,
   if (M == 0) return hipSuccess;
   int R = tuning().r_f32;
   if (R != 1 && R != 2 && R != 4) R = 2;
-  int S = ts.n_tiles ? choose_splits(M, R, ts.n_tiles, 64) : 1;
+  int S = tile_splits(M, R, ts.n_tiles);
   while (S > 1 && (size_t)S * M > partial_cap) --S;
   const uint32_t chunk = ts.n_tiles ? (ts.n_tiles + S - 1) / S : 0;
   const dim3 grid((unsigned)((M + (size_t)kBlock * R - 1) / ((size_t)kBlock * R)),
@@ -619,8 +635,7 @@ hipError_t launch_superpose_f32s(int sign, bool obliquity, const TileSet& ts,
   if (!ok) return hipErrorInvalidValue;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  if (skip) return launch_reduce_either(partial, skip, Sp, S, M, y, stream);
-  return launch_reduce_partials(S, M, partial, y, stream);
+  return launch_reduce_partials(S, M, partial, y, stream, skip, Sp);
 }
 
 __global__ __launch_bounds__(kBlock) void k_tile_weights(

@@ -659,27 +659,6 @@ k_superpose_pairs(PairSources sr, const PairTargets* __restrict__ ptp,
     pair_items<false, SIGN, OBL>(pw, sr, pt, S, M, inv_lambda, out);
 }
 
-// y = the sum of the splits of whichever path ran: Sp of this kernel's (its
-// single split wrote y itself), else Sg of the 16-row kernels'.
-__global__ __launch_bounds__(kBlock) void k_reduce_either(const double2* __restrict__ partial,
-                                                          const uint32_t* __restrict__ handled,
-                                                          uint32_t Sp, uint32_t Sg, uint32_t M,
-                                                          double2* __restrict__ y) {
-  const uint32_t S = *handled ? Sp : Sg;
-  if (S <= 1) return;
-  const uint32_t m = blockIdx.x * kBlock + threadIdx.x;
-  if (m < M) y[m] = sum_splits(partial + m, S, M);
-}
-
-hipError_t launch_reduce_either(const double2* partial, const uint32_t* handled, int Sp, int Sg,
-                                size_t M, double2* y, hipStream_t stream) {
-  if (std::max(Sp, Sg) <= 1 || M == 0) return hipSuccess;
-  const unsigned blocks = (unsigned)((M + kBlock - 1) / kBlock);
-  k_reduce_either<<<blocks, kBlock, 0, stream>>>(partial, handled, (uint32_t)Sp, (uint32_t)Sg,
-                                                 (uint32_t)M, y);
-  return hipGetLastError();
-}
-
 // One split where the target tiles fill the slots many times over; else the
 // count (at most 8 above one round) that leaves the last round fullest, each
 // wave with a source tile of its own.
