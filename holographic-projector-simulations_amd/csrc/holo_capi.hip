@@ -1580,9 +1580,13 @@ holo_status holo_transform_mc(holo_ctx* ctx, holo_precision precision, int sign,
                                            static_cast<double*>(ctx->mc_xy.ptr), ctx->stream));
   const double Kw = (2 * M_PI) / lambda;
   const bool shared = flags & HOLO_MC_SHARED, obl = flags & HOLO_OBLIQUITY;
+  uint32_t chunk;
+  const size_t S = holo::mc_splits(M, K, fp64, shared, &chunk);
+  if (S > 1) HOLO_TRY(ensure(ctx->partial, S * M * sizeof(double2), ctx->device));
   HOLO_HIP(holo::launch_mc(sign, fp64, shared, obl, static_cast<const double4*>(ctx->pos.ptr),
                            static_cast<const double*>(ctx->ph.ptr), N, dv, M, K, seed, Kw,
-                           lambda, lat, reinterpret_cast<double2*>(dy), ctx->stream));
+                           lambda, lat, reinterpret_cast<double2*>(dy),
+                           static_cast<double2*>(ctx->partial.ptr), ctx->stream));
   // the FP64 estimator with the same indices at the report's targets
   HOLO_TRY(report_error(ctx, fp64, dv, M, dy, err_rel_l2, dev,
                         [&](const ErrScratch& e, size_t count) {

@@ -344,7 +344,8 @@ hipError_t launch_lattice_tiles(const LatticeTiles& a, hipStream_t stream);
 // 3 / 5 / 8 of its 32 MB of records).
 // A grid of up to this many workgroups is resident at once: one launch takes its
 // ranges in turn (256^2 targets, lattice: 397 us, 456 in a launch per range), while
-// those of a larger grid drift apart (1024^2: 8140 us, 4260).
+// those of a larger grid drift apart (1024^2: 8140 us, 4260).  FP64: a third of that
+// (700^2 lattice to 300^2, 352 workgroups: 1790 us, 1600 in a launch per range).
 constexpr unsigned kMcRound = 768;
 // From this many draws on (an eighth where kMcRound holds) lattices take the kernel
 // that stages their tables in LDS and other sources the general one, each an idle
@@ -361,7 +362,14 @@ constexpr uint64_t kMcRecordDraws = uint64_t(1) << 26;
 hipError_t launch_mc(int sign, bool fp64, bool shared, bool obliquity, const double4* pos,
                      const double* ph, size_t N, const double* v, size_t M,
                      uint32_t K, uint64_t seed, double K_wave, double lambda,
-                     const McLattice& lat, double2* y, hipStream_t stream);
+                     const McLattice& lat, double2* y, double2* partial, hipStream_t stream);
+// Splits S of the draws, of `chunk` each, up to kMcRound workgroups (shared subsets,
+// eight to a CU: twice that); S > 1 needs S M partial values.  64^2 targets, K = 1024,
+// 1024^2 lattice: 415 -> 97 us (one split and now), FP64 1.42 -> 0.18 ms; shared
+// subsets 580 -> 60 us, FP64 1.09 ms -> 90 us; below 128 draws (shared: 64) to a split
+// the tables and the reduction cost what it gives.
+constexpr size_t kMcMinDraws = 128;
+uint32_t mc_splits(size_t M, uint32_t K, bool fp64, bool shared, uint32_t* chunk);
 
 // The FP64 estimator at `count` targets vsub whose indices (Philox counters)
 // are tmap[i]: per target, or (shared) of the target's group; pos/ph packed

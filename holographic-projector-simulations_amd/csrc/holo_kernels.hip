@@ -871,7 +871,7 @@ constexpr uint32_t kMcQueue = 32;  // ring slots per lane, a power of two
 template <McView VIEW, int SIGN, bool FP64, bool OBL>
 __device__ __forceinline__ void mc_pass(const McSourceView& source, const double* __restrict__ ph,
                                         uint32_t N, double vx, double vy, double vz, bool active,
-                                        uint32_t m, uint32_t K, uint32_t seed_lo,
+                                        uint32_t m, uint32_t kb, uint32_t K, uint32_t seed_lo,
                                         uint32_t seed_hi, double Kw, double inv_lambda,
                                         uint32_t lo, uint32_t hi, uint32_t* s_q, double& ar,
                                         double& ai) {
@@ -925,7 +925,7 @@ __device__ __forceinline__ void mc_pass(const McSourceView& source, const double
     }
     head += take;
   };
-  for (uint32_t k = 0;; k += 8) {
+  for (uint32_t k = kb;; k += 8) {
     const bool more = k < K;
     if (more) {
       uint32_t idx[8];
@@ -958,8 +958,9 @@ __device__ __forceinline__ void mc_pass(const McSourceView& source, const double
 template <bool STAGE, int SIGN, bool FP64, bool OBL>
 __global__ __launch_bounds__(kBlock) void k_mc_pass(
     const double4* __restrict__ pos, const double* __restrict__ ph, uint32_t N,
-    const double* __restrict__ v, uint32_t M, uint32_t K, uint32_t seed_lo, uint32_t seed_hi,
-    double Kw, double inv_lambda, McLattice lat, uint32_t b0, uint32_t b1, uint32_t passes,
+    const double* __restrict__ v, uint32_t M, uint32_t K, uint32_t kchunk, uint32_t seed_lo,
+    uint32_t seed_hi, double Kw, double inv_lambda, McLattice lat, uint32_t b0, uint32_t b1,
+    uint32_t passes,
     uint32_t widest, int staged, double scale, double2* __restrict__ y) {
   __shared__ uint32_t s_q[kMcQueue * kBlock];
   // (without the tables five workgroups' rings fill a CU's LDS)
@@ -974,6 +975,8 @@ __global__ __launch_bounds__(kBlock) void k_mc_pass(
   const bool active = m < M, idle = __ballot(active) == 0;  // idle: the whole wave is past M
   const uint32_t mm = active ? m : M - 1;
   const double vx = v[3 * (size_t)mm], vy = v[3 * (size_t)mm + 1], vz = v[3 * (size_t)mm + 2];
+  const uint32_t kb = blockIdx.y * kchunk, ke = min(K, kb + kchunk);
+  y += (size_t)blockIdx.y * M;
   double ar = 0.0, ai = 0.0;
   for (uint32_t b = b0; b < b1; ++b) {
     const uint32_t lo = (uint32_t)((uint64_t)b * N / passes);
@@ -984,7 +987,7 @@ __global__ __launch_bounds__(kBlock) void k_mc_pass(
     }
     if (idle) continue;
     const auto run = [&](auto view) __attribute__((always_inline)) {
-      mc_pass<view.value, SIGN, FP64, OBL>(source, ph, N, vx, vy, vz, active, mm, K, seed_lo,
+      mc_pass<view.value, SIGN, FP64, OBL>(source, ph, N, vx, vy, vz, active, mm, kb, ke, seed_lo,
                                            seed_hi, Kw, inv_lambda, lo, hi, s_q, ar, ai);
     };
     if constexpr (STAGE)
@@ -1008,10 +1011,12 @@ __global__ __launch_bounds__(kBlock) void k_mc_pass(
 template <int SIGN, bool FP64, bool OBL>
 __global__ __launch_bounds__(kBlock) void k_mc_shared(
     const double4* __restrict__ pos, const double* __restrict__ ph,
-    uint32_t N, const double* __restrict__ v, uint32_t M, uint32_t K,
+    uint32_t N, const double* __restrict__ v, uint32_t M, uint32_t K, uint32_t kchunk,
     uint32_t seed_lo, uint32_t seed_hi, double Kw, double inv_lambda,
     double scale, double2* __restrict__ y) {
   constexpr int R = kMcGroup / kBlock;
+  const uint32_t kb = blockIdx.y * kchunk, ke = min(K, kb + kchunk);  // kchunk: of 64
+  y += (size_t)blockIdx.y * M;
   const uint32_t g = blockIdx.x;
   double vx[R], vy[R], vz[R], ar[R], ai[R];
   float fr[R], fi[R];
@@ -1025,12 +1030,12 @@ __global__ __launch_bounds__(kBlock) void k_mc_shared(
     ar[r] = ai[r] = 0.0;
     fr[r] = fi[r] = 0.f;
   }
-  for (uint32_t k = 0; k < K; k += 2) {
+  for (uint32_t k = kb; k < ke; k += 2) {
     const U4 o = philox4x32_10(U4{k >> 1, g, kMcSharedTag, kMcStream}, seed_lo, seed_hi);
     const uint32_t idx[2] = {lemire_index(o.x, o.y, N), lemire_index(o.z, o.w, N)};
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      if (h == 1 && k + 1 >= K) break;
+      if (h == 1 && k + 1 >= ke) break;
       const double4 p = pos[idx[h]];
       if constexpr (FP64) {
         const double phv = ph[idx[h]];
@@ -1047,7 +1052,7 @@ __global__ __launch_bounds__(kBlock) void k_mc_shared(
       }
     }
     if constexpr (!FP64) {
-      if ((k & 62) == 62 || k + 2 >= K) {  // flush FP32 partials every 64 draws
+      if ((k & 62) == 62 || k + 2 >= ke) {  // flush FP32 partials every 64 draws
 #pragma unroll
         for (int r = 0; r < R; ++r) {
           ar[r] += fr[r];
@@ -1073,17 +1078,36 @@ static uint32_t mc_passes(size_t N, size_t bytes, size_t per_pass) {
   return (uint32_t)std::min<size_t>(std::max<size_t>(p, 1), 8);
 }
 
+static bool mc_round(size_t blocks, bool fp64) {
+  return blocks <= (fp64 ? kMcRound / 3 : kMcRound);
+}
+
+uint32_t mc_splits(size_t M, uint32_t K, bool fp64, bool shared, uint32_t* chunk) {
+  const size_t group = shared ? kMcGroup : (size_t)kBlock, blocks = (M + group - 1) / group;
+  const size_t fill = shared ? 2 * kMcRound : kMcRound, least = shared ? 64 : kMcMinDraws;
+  size_t S = std::min<size_t>({fill / blocks, K / least, 64});
+  if (!shared && !mc_round(blocks, fp64)) S = 1;  // ranges add to y launch by launch
+  S = std::max<size_t>(S, 1);
+  const size_t c = (K + S - 1) / S, step = shared ? 64 : 8;
+  *chunk = (uint32_t)std::min<size_t>((c + step - 1) / step * step, (UINT32_MAX / step) * step);
+  return (uint32_t)((K + (size_t)*chunk - 1) / *chunk);
+}
+
 hipError_t launch_mc(int sign, bool fp64, bool shared, bool obliquity, const double4* pos,
                      const double* ph, size_t N, const double* v, size_t M,
                      uint32_t K, uint64_t seed, double K_wave, double lambda,
-                     const McLattice& lat, double2* y, hipStream_t stream) {
+                     const McLattice& lat, double2* y, double2* partial, hipStream_t stream) {
   if (!M) return hipSuccess;
   const double scale = (double)N / (double)K;
   const uint32_t slo = (uint32_t)seed, shi = (uint32_t)(seed >> 32);
   const double il = 1.0 / lambda;
   const unsigned blocks = shared ? (unsigned)((M + kMcGroup - 1) / kMcGroup)
                                  : (unsigned)((M + kBlock - 1) / kBlock);
-  const bool round = blocks <= kMcRound;
+  uint32_t chunk;
+  const uint32_t S = mc_splits(M, K, fp64, shared, &chunk);
+  double2* out = S > 1 ? partial : y;
+  const dim3 grid(blocks, S);
+  const bool round = mc_round(blocks, fp64);
   const uint64_t draws = (uint64_t)M * K;
   // FP64 gathers 40 bytes per draw.  FP32-split sources gather 8 on a lattice; off it
   // 32, which take ranges of their own where the draws pay for them.
@@ -1101,25 +1125,24 @@ hipError_t launch_mc(int sign, bool fp64, bool shared, bool obliquity, const dou
     with_bool(fp64, [&](auto f64) {
       with_bool(obliquity, [&](auto obl) {
         if (shared) {
-          k_mc_shared<sg.value, (bool)f64.value, (bool)obl.value><<<blocks, kBlock, 0, stream>>>(
-              pos, ph, (uint32_t)N, v, (uint32_t)M, K, slo, shi, K_wave, il, scale, y);
+          k_mc_shared<sg.value, (bool)f64.value, (bool)obl.value><<<grid, kBlock, 0, stream>>>(
+              pos, ph, (uint32_t)N, v, (uint32_t)M, K, chunk, slo, shi, K_wave, il, scale, out);
           return;
         }
         // widest: 0, or the width of the staged ranges, and the launch is for the
         // sources that can (`staged`) or cannot be staged and exits on the others
         const auto ranges = [&](auto stage, uint32_t passes, uint32_t widest, bool staged) {
           if (passes <= 1)
-            k_mc<sg.value, (bool)f64.value, (bool)obl.value, false>
-                <<<blocks, kBlock, 0, stream>>>(pos, ph, (uint32_t)N, v, (uint32_t)M, nullptr, K,
-                                                K + (K & 1u), slo, shi, K_wave, il, scale, lat,
-                                                K >= kMcStageK ? 1 : 0, widest ? 1 : 0, y);
+            k_mc<sg.value, (bool)f64.value, (bool)obl.value, false><<<grid, kBlock, 0, stream>>>(
+                pos, ph, (uint32_t)N, v, (uint32_t)M, nullptr, K, chunk, slo, shi, K_wave, il,
+                scale, lat, chunk >= kMcStageK ? 1 : 0, widest ? 1 : 0, out);
           else
             for (uint32_t b = 0; b < passes; b = round ? passes : b + 1)
               k_mc_pass<(bool)stage.value, sg.value, (bool)f64.value, (bool)obl.value>
-                  <<<blocks, kBlock, 0, stream>>>(pos, ph, (uint32_t)N, v, (uint32_t)M, K, slo,
-                                                  shi, K_wave, il, lat, b,
-                                                  round ? passes : b + 1, passes, widest,
-                                                  staged ? 1 : 0, scale, y);
+                  <<<grid, kBlock, 0, stream>>>(pos, ph, (uint32_t)N, v, (uint32_t)M, K, chunk,
+                                                slo, shi, K_wave, il, lat, b,
+                                                round ? passes : b + 1, passes, widest,
+                                                staged ? 1 : 0, scale, out);
         };
         if constexpr (!(bool)f64.value) {
           if (apart) {
@@ -1137,7 +1160,9 @@ hipError_t launch_mc(int sign, bool fp64, bool shared, bool obliquity, const dou
       });
     });
   });
-  return hipGetLastError();
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return launch_reduce_partials((int)S, M, partial, y, stream);
 }
 
 hipError_t launch_mc_subset(int sign, bool shared, bool obliquity, const double4* pos,
