@@ -364,7 +364,7 @@ hipError_t launch_mc(int sign, bool fp64, bool shared, bool obliquity, const dou
                      uint32_t K, uint64_t seed, double K_wave, double lambda,
                      const McLattice& lat, double2* y, double2* partial, hipStream_t stream);
 // Splits S of the draws, of `chunk` each, up to kMcRound workgroups (shared subsets,
-// eight to a CU: twice that); S > 1 needs S M partial values.  64^2 targets, K = 1024,
+// eight to a CU: 2048, which at 1024^2 targets takes 897 us for 1006); S > 1 needs S M partial values.  64^2 targets, K = 1024,
 // 1024^2 lattice: 415 -> 97 us (one split and now), FP64 1.42 -> 0.18 ms; shared
 // subsets 580 -> 60 us, FP64 1.09 ms -> 90 us; below 128 draws (shared: 64) to a split
 // the tables and the reduction cost what it gives.

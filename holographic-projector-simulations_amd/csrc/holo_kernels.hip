@@ -1084,7 +1084,7 @@ static bool mc_round(size_t blocks, bool fp64) {
 
 uint32_t mc_splits(size_t M, uint32_t K, bool fp64, bool shared, uint32_t* chunk) {
   const size_t group = shared ? kMcGroup : (size_t)kBlock, blocks = (M + group - 1) / group;
-  const size_t fill = shared ? 2 * kMcRound : kMcRound, least = shared ? 64 : kMcMinDraws;
+  const size_t fill = shared ? 2048 : kMcRound, least = shared ? 64 : kMcMinDraws;
   size_t S = std::min<size_t>({fill / blocks, K / least, 64});
   if (!shared && !mc_round(blocks, fp64)) S = 1;  // ranges add to y launch by launch
   S = std::max<size_t>(S, 1);

@@ -54,8 +54,8 @@
 // phasors: X of target row j and Y of target column j.  Real and imaginary
 // parts are separate operands: T_re = Wr Yr + Wi (-Yi), T_im = Wr Yi + Wi Yr.
 //
-// What bounds it: VALU issue, about 74 % busy (650 instructions per 2^20 pairs, half
-// of them for the phasors), beside matrix cores at 42 %; two waves per SIMD (242
+// What bounds it: VALU issue, 77 % busy (650 instructions per 2^20 pairs, half
+// of them for the phasors), beside matrix cores at 37 %; two waves per SIMD (242
 // VGPRs).  Per call, 1024^2 -> 1024^2: 2.0 ms at 0.35 m (5.4e14 pairs/s) where the
 // 16 x 64 tiles of k_superpose_grid16 take 57.8 ms, 4.9 ms at 0.2 m (93 ms), 6.5 ms
 // at 0.1 m (140 ms); 64^2 -> 64^2: 28 us (34 us).  With 32 x 32 source tiles the far
