@@ -784,7 +784,7 @@ __global__ __launch_bounds__(kBlock) void k_mc(
   }
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= M) return;
-  const uint32_t kb = blockIdx.y * kchunk, ke = min(K, kb + kchunk);
+  const uint32_t kb = blockIdx.y * kchunk, ke = kb + min(K - kb, kchunk);
   const uint32_t m = tmap ? tmap[i] : i;
   const double vx = v[3 * (size_t)i], vy = v[3 * (size_t)i + 1],
                vz = v[3 * (size_t)i + 2];
@@ -975,7 +975,7 @@ __global__ __launch_bounds__(kBlock) void k_mc_pass(
   const bool active = m < M, idle = __ballot(active) == 0;  // idle: the whole wave is past M
   const uint32_t mm = active ? m : M - 1;
   const double vx = v[3 * (size_t)mm], vy = v[3 * (size_t)mm + 1], vz = v[3 * (size_t)mm + 2];
-  const uint32_t kb = blockIdx.y * kchunk, ke = min(K, kb + kchunk);
+  const uint32_t kb = blockIdx.y * kchunk, ke = kb + min(K - kb, kchunk);
   y += (size_t)blockIdx.y * M;
   double ar = 0.0, ai = 0.0;
   for (uint32_t b = b0; b < b1; ++b) {
@@ -1015,7 +1015,7 @@ __global__ __launch_bounds__(kBlock) void k_mc_shared(
     uint32_t seed_lo, uint32_t seed_hi, double Kw, double inv_lambda,
     double scale, double2* __restrict__ y) {
   constexpr int R = kMcGroup / kBlock;
-  const uint32_t kb = blockIdx.y * kchunk, ke = min(K, kb + kchunk);  // kchunk: of 64
+  const uint32_t kb = blockIdx.y * kchunk, ke = kb + min(K - kb, kchunk);  // kchunk: of 64
   y += (size_t)blockIdx.y * M;
   const uint32_t g = blockIdx.x;
   double vx[R], vy[R], vz[R], ar[R], ai[R];
