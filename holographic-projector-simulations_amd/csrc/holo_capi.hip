@@ -1215,6 +1215,7 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
       pp.u = static_cast<const double*>(p->u.ptr);
       pp.perm = static_cast<const int32_t*>(p->perm.ptr);
       pp.wc = static_cast<float2*>(p->wc.ptr);
+      pp.n = (uint32_t)p->N;
       pp.n_slots = (uint32_t)slots;
       for (int d = 0; d < 3; ++d) {
         pp.lo[d] = p->lo[d];

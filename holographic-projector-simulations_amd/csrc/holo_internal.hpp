@@ -272,14 +272,14 @@ hipError_t launch_superpose_pairs(int sign, bool obliquity, const PairPlan& pp, 
                                   double lambda, int S, PairTargets* pt, uint32_t* flags,
                                   uint32_t* handled, double2* out, const Grid16Prep* grid16,
                                   hipStream_t stream);
-// Point-to-lattice kernel (holo_points.hip): n_slots slots of sources u[perm[slot]]
+// Point-to-lattice kernel (holo_points.hip): n_slots slots of the n sources u[perm[slot]]
 // (perm < 0: none) within [lo, hi]; wc: n_slots float2, the slots' polar weights,
 // written by each launch.
 struct PointPlan {
   const double* u = nullptr;
   const int32_t* perm = nullptr;
   float2* wc = nullptr;
-  uint32_t n_slots = 0;
+  uint32_t n = 0, n_slots = 0;
   double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
 };
 int point_splits(size_t M, size_t n_slots);

@@ -76,27 +76,29 @@ __device__ uint32_t block_first(uint32_t lim, uint32_t* s_min, F&& hit) {
 // with target 0's x again: the generator fills up with copies of point 0), then
 // checks its share of the targets against x_0 + i p_x, y_0 + j p_y, z_0 to 1e-9 of
 // a pitch (a product of one x per row and one y per column to the bit), and the
-// rest against target 0.  flags[b] = 1 when its share passes; workgroup 0 writes
+// rest against target 0.  flags[b] = 1 when its share passes, and `ok` (the caller's
+// checks) holds on every lane; workgroup 0 writes
 // *pt, with the mode that form(pt, cx0, cx1, cy0, cy1) gives for the lattice of 32 x
 // 32 tiles with the first and last centres (cx0, cy0), (cx1, cy1).
 template <typename F>
 __device__ void probe_targets(const double* __restrict__ v, uint32_t M, uint32_t b,
                               uint32_t n_probe, PairTargets* pt, uint32_t* flags, uint32_t* s_min,
-                              F&& form) {
+                              bool ok, F&& form) {
   const double x0 = v[0], y0 = v[1], z0 = v[2];
   const uint32_t lim = min(M, kPairMaxRow);
   const uint32_t ny = block_first(lim, s_min, [&](uint32_t k) { return v[3 * (size_t)k] != x0; });
   uint32_t nx = ny < lim && ny >= 16 ? M / ny : 0u;
   if (nx >= 16)
     nx = block_first(nx, s_min, [&](uint32_t k) { return v[3 * (size_t)k * ny] == x0; });
-  bool ok = nx >= 16;
   double px = 0.0, py = 0.0;
-  if (ok) {
+  if (nx < 16) {
+    ok = false;
+  } else {
     const uint32_t body = nx * ny;
     px = (v[3 * (size_t)(nx - 1) * ny] - x0) / (double)(nx - 1);
     py = (v[3 * (size_t)(ny - 1) + 1] - y0) / (double)(ny - 1);
     const double tx = 1e-9 * fabs(px), ty = 1e-9 * fabs(py);
-    ok = tx > 0.0 && ty > 0.0 && __builtin_isfinite(px) && __builtin_isfinite(py);
+    ok = ok && tx > 0.0 && ty > 0.0 && __builtin_isfinite(px) && __builtin_isfinite(py);
     for (uint32_t m = b * kBlock + threadIdx.x; m < M; m += n_probe * kBlock) {
       const double x = v[3 * (size_t)m], y = v[3 * (size_t)m + 1], z = v[3 * (size_t)m + 2];
       if (m < body) {

@@ -224,7 +224,7 @@ __global__ __launch_bounds__(kBlock) void k_pair_prep(PairPrep a, Grid16Prep g) 
     --b;
   }
   if (b < a.n_probe)
-    probe_targets(a.v, a.M, b, a.n_probe, a.pt, a.flags, reinterpret_cast<uint32_t*>(s_buf),
+    probe_targets(a.v, a.M, b, a.n_probe, a.pt, a.flags, reinterpret_cast<uint32_t*>(s_buf), true,
                   [&](const PairTargets& t, double cx0, double cx1, double cy0, double cy1) {
                     return pair_mode(a, t, cx0, cx1, cy0, cy1);
                   });

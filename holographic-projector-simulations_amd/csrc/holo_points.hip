@@ -316,8 +316,23 @@ k_superpose_points(PointPlan pp, const PairTargets* __restrict__ ptp,
     point_items<false, SIGN, OBL>(pw, pp, pt, S, M, inv_lambda, out);
 }
 
+// Whether this workgroup's share (b of n_probe) of the weights is finite in FP32.
+__device__ bool weights_finite(const PointPlan& pp, int wf, const double* __restrict__ w0,
+                               const double* __restrict__ w1, uint32_t b, uint32_t n_probe) {
+  bool ok = true;
+  for (uint32_t n = b * kBlock + threadIdx.x; n < pp.n; n += n_probe * kBlock) {
+    const double x = wf == kPolar ? w0[n] : w0[2 * (size_t)n];
+    const double y = wf == kPolar ? w1[n] : w0[2 * (size_t)n + 1];
+    ok = ok && __builtin_isfinite((float)x) &&
+         __builtin_isfinite(wf == kPolar ? y : (double)(float)y);
+  }
+  return ok;
+}
+
 // The polar weights of the slots (launch_tile_weights), and in the workgroups after
-// those the targets' lattice.
+// those the targets' lattice.  A call with a weight that is not finite keeps the tiled
+// kernel, whose infinities and NaN are those of the FP32 products: the integer phases
+// here would turn a NaN into a number, and an f16 pair an infinity into NaN.
 __global__ __launch_bounds__(kBlock) void k_point_prep(PointPlan pp, int wf,
                                                        const double* __restrict__ w0,
                                                        const double* __restrict__ w1,
@@ -332,7 +347,8 @@ __global__ __launch_bounds__(kBlock) void k_point_prep(PointPlan pp, int wf,
     if (s < pp.n_slots) pp.wc[s] = slot_weight_polar(wf, w0, w1, pp.perm[s]);
     return;
   }
-  probe_targets(v, M, blockIdx.x - wb, n_probe, pt, flags, s_min,
+  const uint32_t b = blockIdx.x - wb;
+  probe_targets(v, M, b, n_probe, pt, flags, s_min, weights_finite(pp, wf, w0, w1, b, n_probe),
                 [&](const PairTargets& t, double cx0, double cx1, double cy0, double cy1) {
                   const auto far = [](double a0, double a1, double b0, double b1) {
                     return fmax(fabs(fmax(a0, a1) - b0), fabs(b1 - fmin(a0, a1)));
