@@ -1486,6 +1486,7 @@ holo_status holo_transform_full(holo_ctx* ctx, holo_precision precision, int sig
                                           ctx->stream));
     }
   } else {
+    if (!u) return fail(HOLO_EINVAL, "null source positions");
     // a plan for this call, built anew in the buffers of the context's last one
     std::unique_ptr<holo_plan> own;
     if (N > kShotSources) own.reset(new holo_plan);
