@@ -18,6 +18,7 @@
 
 #include "holo_device.hpp"
 #include "holo_internal.hpp"
+#include "holo_mc.hpp"
 
 namespace holo {
 
@@ -784,7 +785,7 @@ __global__ __launch_bounds__(kBlock) void k_mc(
   }
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= M) return;
-  const uint32_t kb = blockIdx.y * kchunk, ke = kb + min(K - kb, kchunk);
+  McDraws d = mc_split(K, kchunk, blockIdx.y);
   const uint32_t m = tmap ? tmap[i] : i;
   const double vx = v[3 * (size_t)i], vy = v[3 * (size_t)i + 1],
                vz = v[3 * (size_t)i + 2];
@@ -792,12 +793,11 @@ __global__ __launch_bounds__(kBlock) void k_mc(
   with_view<FP64>(source, N, [&](auto view) {
     float fr = 0.f, fi = 0.f;
     // 8 samples per step: 4 Philox blocks, then 8 independent gathers in flight
-    const uint32_t K8 = kb + ((ke - kb) & ~7u);
-    for (uint32_t k = kb; k < K8; k += 8) {
+    for (; d.left >= 8; d.take(8)) {
       uint32_t idx[8];
 #pragma unroll
       for (int h = 0; h < 4; ++h) {
-        const U4 o = mc_draws<SHARED_IDX>(k + 2 * h, m, seed_lo, seed_hi);
+        const U4 o = mc_draws<SHARED_IDX>(d.k + 2 * h, m, seed_lo, seed_hi);
         idx[2 * h] = lemire_index(o.x, o.y, N);
         idx[2 * h + 1] = lemire_index(o.z, o.w, N);
       }
@@ -826,12 +826,12 @@ __global__ __launch_bounds__(kBlock) void k_mc(
         fi = 0.f;
       }
     }
-    for (uint32_t k = K8; k < ke; k += 2) {
-      const U4 o = mc_draws<SHARED_IDX>(k, m, seed_lo, seed_hi);
+    for (; d.left; d.take(2)) {
+      const U4 o = mc_draws<SHARED_IDX>(d.k, m, seed_lo, seed_hi);
       const uint32_t idx[2] = {lemire_index(o.x, o.y, N), lemire_index(o.z, o.w, N)};
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        if (h == 1 && k + 1 >= ke) break;
+        if (h == 1 && d.left == 1) break;
         const double4 p = source.at<view.value>(idx[h]);
         if constexpr (FP64) {
           const PairF64 q = pair_f64<SIGN, 0, OBL>(p.w, ph[idx[h]], p.x, p.y, p.z, vx, vy, vz, Kw);
@@ -871,8 +871,8 @@ constexpr uint32_t kMcQueue = 32;  // ring slots per lane, a power of two
 template <McView VIEW, int SIGN, bool FP64, bool OBL>
 __device__ __forceinline__ void mc_pass(const McSourceView& source, const double* __restrict__ ph,
                                         uint32_t N, double vx, double vy, double vz, bool active,
-                                        uint32_t m, uint32_t kb, uint32_t K, uint32_t seed_lo,
-                                        uint32_t seed_hi, double Kw, double inv_lambda,
+                                        uint32_t m, McDraws d, uint32_t seed_lo, uint32_t seed_hi,
+                                        double Kw, double inv_lambda,
                                         uint32_t lo, uint32_t hi, uint32_t* s_q, double& ar,
                                         double& ai) {
   // byte offsets into the ring [slot][lane]: one bank per lane
@@ -925,20 +925,20 @@ __device__ __forceinline__ void mc_pass(const McSourceView& source, const double
     }
     head += take;
   };
-  for (uint32_t k = kb;; k += 8) {
-    const bool more = k < K;
+  for (;; d.take(8)) {
+    const bool more = d.left != 0;
     if (more) {
       uint32_t idx[8];
 #pragma unroll
       for (int h = 0; h < 4; ++h) {
-        const U4 o = mc_draws<false>(k + 2 * h, m, seed_lo, seed_hi);
+        const U4 o = mc_draws<false>(d.k + 2 * h, m, seed_lo, seed_hi);
         idx[2 * h] = lemire_index(o.x, o.y, N);
         idx[2 * h + 1] = lemire_index(o.z, o.w, N);
       }
       const uint32_t width = active ? hi - lo : 0u;
 #pragma unroll
-      for (int h = 0; h < 8; ++h)
-        if (k + h < K && idx[h] - lo < width) {
+      for (uint32_t h = 0; h < 8; ++h)
+        if (h < d.left && idx[h] - lo < width) {
           slot(tail) = idx[h];
           tail += kStep;
         }
@@ -975,7 +975,7 @@ __global__ __launch_bounds__(kBlock) void k_mc_pass(
   const bool active = m < M, idle = __ballot(active) == 0;  // idle: the whole wave is past M
   const uint32_t mm = active ? m : M - 1;
   const double vx = v[3 * (size_t)mm], vy = v[3 * (size_t)mm + 1], vz = v[3 * (size_t)mm + 2];
-  const uint32_t kb = blockIdx.y * kchunk, ke = kb + min(K - kb, kchunk);
+  const McDraws draws = mc_split(K, kchunk, blockIdx.y);
   y += (size_t)blockIdx.y * M;
   double ar = 0.0, ai = 0.0;
   for (uint32_t b = b0; b < b1; ++b) {
@@ -987,7 +987,7 @@ __global__ __launch_bounds__(kBlock) void k_mc_pass(
     }
     if (idle) continue;
     const auto run = [&](auto view) __attribute__((always_inline)) {
-      mc_pass<view.value, SIGN, FP64, OBL>(source, ph, N, vx, vy, vz, active, mm, kb, ke, seed_lo,
+      mc_pass<view.value, SIGN, FP64, OBL>(source, ph, N, vx, vy, vz, active, mm, draws, seed_lo,
                                            seed_hi, Kw, inv_lambda, lo, hi, s_q, ar, ai);
     };
     if constexpr (STAGE)
@@ -1015,7 +1015,7 @@ __global__ __launch_bounds__(kBlock) void k_mc_shared(
     uint32_t seed_lo, uint32_t seed_hi, double Kw, double inv_lambda,
     double scale, double2* __restrict__ y) {
   constexpr int R = kMcGroup / kBlock;
-  const uint32_t kb = blockIdx.y * kchunk, ke = kb + min(K - kb, kchunk);  // kchunk: of 64
+  McDraws d = mc_split(K, kchunk, blockIdx.y);  // kchunk: of 64
   y += (size_t)blockIdx.y * M;
   const uint32_t g = blockIdx.x;
   double vx[R], vy[R], vz[R], ar[R], ai[R];
@@ -1030,12 +1030,12 @@ __global__ __launch_bounds__(kBlock) void k_mc_shared(
     ar[r] = ai[r] = 0.0;
     fr[r] = fi[r] = 0.f;
   }
-  for (uint32_t k = kb; k < ke; k += 2) {
-    const U4 o = philox4x32_10(U4{k >> 1, g, kMcSharedTag, kMcStream}, seed_lo, seed_hi);
+  for (; d.left; d.take(2)) {
+    const U4 o = philox4x32_10(U4{d.k >> 1, g, kMcSharedTag, kMcStream}, seed_lo, seed_hi);
     const uint32_t idx[2] = {lemire_index(o.x, o.y, N), lemire_index(o.z, o.w, N)};
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      if (h == 1 && k + 1 >= ke) break;
+      if (h == 1 && d.left == 1) break;
       const double4 p = pos[idx[h]];
       if constexpr (FP64) {
         const double phv = ph[idx[h]];
@@ -1052,7 +1052,7 @@ __global__ __launch_bounds__(kBlock) void k_mc_shared(
       }
     }
     if constexpr (!FP64) {
-      if ((k & 62) == 62 || k + 2 >= ke) {  // flush FP32 partials every 64 draws
+      if ((d.k & 62) == 62 || d.left <= 2) {  // flush FP32 partials every 64 draws
 #pragma unroll
         for (int r = 0; r < R; ++r) {
           ar[r] += fr[r];
@@ -1087,10 +1087,7 @@ uint32_t mc_splits(size_t M, uint32_t K, bool fp64, bool shared, uint32_t* chunk
   const size_t fill = shared ? 2048 : kMcRound, least = shared ? 64 : kMcMinDraws;
   size_t S = std::min<size_t>({fill / blocks, K / least, 64});
   if (!shared && !mc_round(blocks, fp64)) S = 1;  // ranges add to y launch by launch
-  S = std::max<size_t>(S, 1);
-  const size_t c = (K + S - 1) / S, step = shared ? 64 : 8;
-  *chunk = (uint32_t)std::min<size_t>((c + step - 1) / step * step, (UINT32_MAX / step) * step);
-  return (uint32_t)((K + (size_t)*chunk - 1) / *chunk);
+  return mc_chunk(K, S, shared ? 64 : 8, chunk);
 }
 
 hipError_t launch_mc(int sign, bool fp64, bool shared, bool obliquity, const double4* pos,
@@ -1176,12 +1173,10 @@ hipError_t launch_mc_subset(int sign, bool shared, bool obliquity, const double4
   const unsigned blocks = (unsigned)((count + kBlock - 1) / kBlock);
   // a few hundred targets: the draws are split into chunks of at least 64
   // (a multiple of 8) over enough blocks to fill the GPU, summed in order
-  uint32_t S = (uint32_t)std::min<size_t>({(K + 63) / 64, kFewTargetSplits,
-                                          partial_cap / count});
-  S = std::max(S, 1u);
-  uint32_t chunk = (K + S - 1) / S;
-  chunk = (chunk + 7u) & ~7u;
-  S = (K + chunk - 1) / chunk;
+  uint32_t chunk;
+  const uint32_t S = mc_chunk(
+      K, std::min<size_t>({((size_t)K + 63) / 64, kFewTargetSplits, partial_cap / count}), 8,
+      &chunk);
   double2* out = S > 1 ? partial : y;
   with_sign(sign, [&](auto sg) {
     with_bool(shared, [&](auto sh) {
@@ -1295,10 +1290,11 @@ __global__ __launch_bounds__(kBlock) void k_mc_indices(
   const uint32_t j = blockIdx.x * kBlock + threadIdx.x;
   if (j >= count) return;
   const uint32_t m = m0 + j;
-  for (uint32_t k = 0; k < K; k += 2) {
+  for (McDraws d{0u, K}; d.left; d.take(2)) {
+    const uint32_t k = d.k;
     const U4 o = philox4x32_10<true>(U4{k >> 1, m, tag, kMcStream}, seed_lo, seed_hi);
     idx[(size_t)j * K + k] = lemire_index(o.x, o.y, (uint32_t)N);
-    if (k + 1 < K) idx[(size_t)j * K + k + 1] = lemire_index(o.z, o.w, (uint32_t)N);
+    if (d.left > 1) idx[(size_t)j * K + k + 1] = lemire_index(o.z, o.w, (uint32_t)N);
   }
 }
 
