@@ -336,8 +336,9 @@ __global__ __launch_bounds__(kBlock) void k_superpose_grid(
 }
 
 int grid_splits(size_t M, size_t n_tiles, int group) {
-  // below 32 tiles of 16 x 16 the reduction's launch costs what the splits give
-  if (n_tiles * group < 32) return 1;
+  // below 32 tiles of 16 x 16 the reduction's launch costs what the splits give (a
+  // caller's own count holds)
+  if (n_tiles == 0 || (tuning().splits <= 0 && n_tiles * group < 32)) return 1;
   return choose_splits(M, 1, n_tiles, M < kFillTargets ? (group == 4 ? 1 : 16 / group) : 16,
                        kTileSplits);
 }
