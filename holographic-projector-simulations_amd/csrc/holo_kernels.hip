@@ -1069,13 +1069,13 @@ __global__ __launch_bounds__(kBlock) void k_mc_shared(
   }
 }
 
-// Ranges of about `per_pass` bytes over `bytes` gathered (at most 8; option
+// Ranges of about `per_pass` bytes over `bytes` gathered, at most `most` (option
 // "mc_passes" sets the number).
-static uint32_t mc_passes(size_t N, size_t bytes, size_t per_pass) {
+static uint32_t mc_passes(size_t N, size_t bytes, size_t per_pass, size_t most = 8) {
   const int opt = tuning().mc_passes;
   if (opt > 0) return (uint32_t)std::min<size_t>((size_t)opt, std::max<size_t>(N, 1));
   const size_t p = (bytes + per_pass - 1) / per_pass;
-  return (uint32_t)std::min<size_t>(std::max<size_t>(p, 1), 8);
+  return (uint32_t)std::min<size_t>(std::max<size_t>(p, 1), most);
 }
 
 static bool mc_round(size_t blocks, bool fp64) {
@@ -1111,7 +1111,7 @@ hipError_t launch_mc(int sign, bool fp64, bool shared, bool obliquity, const dou
   const size_t mb = size_t(1) << 20;
   uint32_t passes;
   if (fp64)
-    passes = std::min(mc_passes(N, 40 * N, 3 * mb), round ? 3u : 8u);
+    passes = mc_passes(N, 40 * N, 3 * mb, round ? 3 : 8);
   else if (!round && draws >= kMcRecordDraws)
     passes = mc_passes(N, 32 * N, 4 * mb);
   else

@@ -44,3 +44,19 @@ def test_splits(pkg, ctx, oracle, case, z, M):
         assert rel_l2(y[splits][sub], ref) <= 1e-6
     if z == 0.3:
         assert not np.array_equal(y[1], y[3 if case == "18 tiles" else 4])
+
+
+# FP64: fewer ranges by default where one round of workgroups holds the call (M = 300)
+@pytest.mark.parametrize("M", [300, 70000])
+def test_mc_passes_fp64(pkg, ctx, oracle, M):
+    u, v, K = lattice(64, 60, 8e-6, 8e-6), scattered(M, 0.3), 200
+    amp, phase = weights(2, len(u))
+    sub = np.arange(0, M, max(1, M // 200))
+    ref = oracle.transform_mc(1, LAM, amp, phase, u, v, K, 5, targets=sub)
+    y = {}
+    for passes in (3, 8, 13, 64):
+        pkg.set_option("mc_passes", passes)
+        y[passes] = ctx.transform_mc(amp, phase, u, v, K, 5, 1, LAM, pkg.FP64)
+        assert rel_l2(y[passes][sub], ref) <= 1e-12
+    for a, b in ((3, 8), (8, 13), (13, 64)):
+        assert not np.array_equal(y[a], y[b])
