@@ -50,6 +50,14 @@ struct DevBuf {
   void* ptr = nullptr;
   size_t bytes = 0;
   int device = 0;
+  bool graph = false;  // a captured graph uses it
+  DevBuf() = default;
+  DevBuf(DevBuf&& o) noexcept : ptr(o.ptr), bytes(o.bytes), device(o.device), graph(o.graph) {
+    o.ptr = nullptr;
+    o.bytes = 0;
+    o.graph = false;
+  }
+  DevBuf(const DevBuf&) = delete;
   ~DevBuf() { release(); }
   void release() {
     if (ptr) {
@@ -86,11 +94,12 @@ struct holo_ctx {
   // staging buffers for host-pointer calls and scratch
   DevBuf amp, phase, u, v, y, w, partial, small, b, pos, ph;
   DevBuf mc_wc, mc_xy, mc_info;  // product-grid Monte Carlo (McLattice)
-  DevBuf pairs;                  // lattice-to-lattice kernel: target lattice, flags, outcome
   DevBuf errb;                   // error report: subset, FP64 values, partials
   DevBuf pos64, ph64;            // FP64 Monte Carlo records for the error report
   // recorded on the previous stream when holo_set_stream switches streams
   hipEvent_t switched = nullptr;
+  bool capturing = false;        // the stream, as the call found it
+  std::vector<DevBuf> retired;   // outgrown scratch that a captured graph still uses
   // FP32-split calls without a plan: the buffers of the last one (about 120 bytes a
   // source, at most kShotSources of them)
   std::unique_ptr<holo_plan> shot;
@@ -99,7 +108,7 @@ struct holo_ctx {
 struct holo_plan {
   int device = 0;
   size_t N = 0;
-  DevBuf u;  // AoS xyz, 3N doubles
+  DevBuf u;  // AoS xyz, 3N doubles, then the words that plan_look gives
   bool uniform_z = false;  // every source has the z of source 0
   size_t row = 0;          // sources in rows of `row` with one x (0: not)
   // FP32-split tiling
@@ -209,7 +218,36 @@ holo_status noalloc_scratch(int device, void** out) {
 holo_status use_device(holo_ctx* ctx) {
   if (!ctx) return fail(HOLO_EINVAL, "null context");
   HOLO_HIP(hipSetDevice(ctx->device));
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
+    (void)hipGetLastError();  // (the null stream beside another stream's capture)
+    st = hipStreamCaptureStatusNone;
+  }
+  ctx->capturing = st != hipStreamCaptureStatusNone;
   return HOLO_OK;
+}
+
+// Context scratch of at least `bytes`.  Nothing is allocated while the stream is being
+// captured, and what a captured graph uses is kept when a later call outgrows it.
+holo_status ensure(holo_ctx* ctx, DevBuf& b, size_t bytes) {
+  const bool fits = bytes <= b.bytes && b.ptr;
+  if (ctx->capturing) {
+    if (!fits)
+      return fail(HOLO_EDEVICE, "scratch cannot be allocated during a capture: make the call "
+                                "once before it");
+    b.graph = true;
+    return HOLO_OK;
+  }
+  if (!fits && b.graph) ctx->retired.push_back(std::move(b));
+  return ensure(b, bytes, ctx->device);
+}
+
+// Room for `want` split partials: *cap = want, or what there is during a capture (a
+// launch then takes fewer splits).
+holo_status partial_room(holo_ctx* ctx, size_t want, size_t* cap) {
+  *cap = want;
+  if (ctx->capturing) *cap = std::min(want, ctx->partial.bytes / sizeof(double2));
+  return *cap ? ensure(ctx, ctx->partial, *cap * sizeof(double2)) : HOLO_OK;
 }
 
 holo_status check_common(holo_ctx* ctx, int precision, int sign, double lambda,
@@ -244,7 +282,7 @@ holo_status stage_in(holo_ctx* ctx, DevBuf& buf, const T* src, size_t count,
     *out = src;
     return HOLO_OK;
   }
-  HOLO_TRY(ensure(buf, count * sizeof(T), ctx->device));
+  HOLO_TRY(ensure(ctx, buf, count * sizeof(T)));
   HOLO_HIP(hipMemcpyAsync(buf.ptr, src, count * sizeof(T), hipMemcpyHostToDevice,
                           ctx->stream));
   *out = static_cast<const T*>(buf.ptr);
@@ -259,7 +297,7 @@ holo_status out_buf(holo_ctx* ctx, DevBuf& buf, T* dst, size_t count, bool dev,
     *out = dst;
     return HOLO_OK;
   }
-  HOLO_TRY(ensure(buf, std::max<size_t>(count, 1) * sizeof(T), ctx->device));
+  HOLO_TRY(ensure(ctx, buf, std::max<size_t>(count, 1) * sizeof(T)));
   *out = static_cast<T*>(buf.ptr);
   return HOLO_OK;
 }
@@ -298,7 +336,7 @@ holo_status err_scratch(holo_ctx* ctx, ErrScratch* e) {
                o_ref = o_vsub + align256(3 * n * sizeof(double)),
                o_part = o_ref + align256(n * sizeof(double2)),
                total = o_part + np * sizeof(double2);
-  HOLO_TRY(ensure(ctx->errb, total, ctx->device));
+  HOLO_TRY(ensure(ctx, ctx->errb, total));
   char* b = static_cast<char*>(ctx->errb.ptr);
   e->err = reinterpret_cast<double*>(b);
   e->energy = reinterpret_cast<double*>(b + o_energy);
@@ -966,6 +1004,21 @@ size_t row_length(const double* u, size_t N) {
   return L;
 }
 
+// The buffer of N positions, and behind them the words of the lattice searches and of
+// the kernels that look at a call's targets: PairTargets or LatticeInfo at 0, the
+// outcome at 128, a flag per workgroup at 256.  They are the plan's, like its weights,
+// so that a call needs no scratch of its own for them.
+constexpr size_t kLookBytes = 256 + holo::kPairFlags * sizeof(uint32_t);
+static_assert(sizeof(holo::LatticeInfo) <= 128 && sizeof(holo::PairTargets) <= 128, "plan_look");
+
+holo_status plan_positions(holo_ctx* ctx, holo_plan* p, size_t N) {
+  return ensure(p->u, align256(3 * N * sizeof(double)) + kLookBytes, ctx->device);
+}
+
+char* plan_look(const holo_plan* p, size_t N) {
+  return static_cast<char*>(p->u.ptr) + align256(3 * N * sizeof(double));
+}
+
 holo_status plan_build(holo_ctx* ctx, holo_plan* p, const double* u, size_t N,
                        unsigned tile, bool dev) {
   p->device = ctx->device;
@@ -976,7 +1029,7 @@ holo_status plan_build(holo_ctx* ctx, holo_plan* p, const double* u, size_t N,
   if (N && !u) return fail(HOLO_EINVAL, "null source positions");
   std::vector<double> host;
   const double* uh = u;
-  HOLO_TRY(ensure(p->u, std::max<size_t>(3 * N, 1) * sizeof(double), ctx->device));
+  HOLO_TRY(plan_positions(ctx, p, N));
   if (N) {
     if (dev) {
       host.resize(3 * N);
@@ -1010,9 +1063,8 @@ holo_status plan_build_lattice(holo_ctx* ctx, holo_plan* p, const double* u, siz
   *found = false;
   const holo::Tuning& tu = holo::tuning();
   if (N < 64 || !tu.grid || !tu.grid16) return HOLO_OK;
-  HOLO_TRY(ensure(ctx->pairs, 256 + holo::kPairFlags * sizeof(uint32_t), ctx->device));
-  holo::LatticeInfo* di = static_cast<holo::LatticeInfo*>(ctx->pairs.ptr);
-  static_assert(sizeof(holo::LatticeInfo) <= 128, "shares the buffer of PairTargets");
+  HOLO_TRY(plan_positions(ctx, p, N));
+  holo::LatticeInfo* di = reinterpret_cast<holo::LatticeInfo*>(plan_look(p, N));
   HOLO_HIP(holo::launch_find_lattice(u, N, di, ctx->stream));
   holo::LatticeInfo f;
   HOLO_HIP(hipMemcpyAsync(&f, di, sizeof(f), hipMemcpyDeviceToHost, ctx->stream));
@@ -1029,7 +1081,6 @@ holo_status plan_build_lattice(holo_ctx* ctx, holo_plan* p, const double* u, siz
   p->tile = 64;
   p->uniform_z = f.uniform_z != 0;
   p->row = ny >= 4 && f.in_rows ? ny : 0;
-  HOLO_TRY(ensure(p->u, 3 * N * sizeof(double), ctx->device));
   HOLO_HIP(hipMemcpyAsync(p->u.ptr, u, 3 * N * sizeof(double), hipMemcpyDeviceToDevice,
                           ctx->stream));
   HostGrid g;
@@ -1060,9 +1111,10 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
                           bool obliquity, double lambda, holo::WeightForm wf,
                           const double* w0, const double* w1, const double* v, size_t M,
                           double* y) {
+  const auto elems = [M](int S) { return S > 1 ? (size_t)S * M : 0; };  // S splits' partials
   if (precision == HOLO_FP64) {
-    const size_t pe = split_elems_f64(M, p->N);
-    if (pe) HOLO_TRY(ensure(ctx->partial, pe * sizeof(double2), ctx->device));
+    size_t pe;
+    HOLO_TRY(partial_room(ctx, split_elems_f64(M, p->N), &pe));
     const double K = (2 * M_PI) / lambda;  // TWO_PI_OVER_LAMBDA, cuda/macros.h:29-31
     HOLO_HIP(holo::launch_superpose_f64(sign, wf, obliquity, p->uniform_z, p->row, w0, w1,
                                         static_cast<const double*>(p->u.ptr),
@@ -1080,6 +1132,7 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
     const uint32_t* skip = nullptr;
     int Sp = 1;
     const int S16 = holo::grid_splits(M, quads ? p->g64_tiles : (pairs ? p->g32_tiles : nt), nkc);
+    size_t pe;
     const holo::Tuning& tu = holo::tuning();
     holo::Grid16Prep prep;
     prep.wf = (int)wf;
@@ -1096,10 +1149,9 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
     bool prepared = false;
     if (tu.grid_pairs && tu.grid32 && tu.grid64 && p->pp.n_tiles && M >= holo::kPairMinTargets) {
       Sp = holo::pair_splits(M, p->pp.n_tiles);
-      const size_t pe = std::max(Sp, S16) > 1 ? (size_t)std::max(Sp, S16) * M : 0;
-      if (pe) HOLO_TRY(ensure(ctx->partial, pe * sizeof(double2), ctx->device));
-      HOLO_TRY(ensure(ctx->pairs, 256 + holo::kPairFlags * sizeof(uint32_t), ctx->device));
-      char* b = static_cast<char*>(ctx->pairs.ptr);
+      HOLO_TRY(partial_room(ctx, elems(std::max(Sp, S16)), &pe));
+      Sp = (int)std::min<size_t>(Sp, std::max<size_t>(pe / M, 1));
+      char* b = plan_look(p, p->N);
       uint32_t* handled = reinterpret_cast<uint32_t*>(b + 128);
       HOLO_HIP(holo::launch_superpose_pairs(
           sign, obliquity, p->pp, wf, w0, w1, v, M, lambda, Sp,
@@ -1154,8 +1206,7 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
       gt.cy1 = p->g64_cy1;
       gt.rho_y = p->g64_rho_y;
     }
-    const size_t pe = S16 > 1 ? (size_t)S16 * M : 0;
-    if (pe) HOLO_TRY(ensure(ctx->partial, pe * sizeof(double2), ctx->device));
+    HOLO_TRY(partial_room(ctx, elems(S16), &pe));
     HOLO_HIP(holo::launch_superpose_grid16(sign, obliquity, nkc, gt, g32, g16,
                                            static_cast<const float2*>(p->g16_wc.ptr),
                                            static_cast<const uint4*>(p->g16_wq.ptr),
@@ -1186,9 +1237,8 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
     gt.z = p->grid_z;
     gt.rho_x = p->grid_rho_x;
     gt.rho_y = p->grid_rho_y;
-    const int S = holo::grid_splits(M, nt, 1);
-    const size_t pe = S > 1 ? (size_t)S * M : 0;
-    if (pe) HOLO_TRY(ensure(ctx->partial, pe * sizeof(double2), ctx->device));
+    size_t pe;
+    HOLO_TRY(partial_room(ctx, elems(holo::grid_splits(M, nt, 1)), &pe));
     HOLO_HIP(holo::launch_superpose_grid(sign, obliquity, gt,
                                          static_cast<const float2*>(p->g_wc.ptr),
                                          static_cast<const uint4*>(p->g_wh.ptr),
@@ -1203,7 +1253,8 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
       if (!p->tiles_built) HOLO_TRY(plan_build_tiles(ctx, p, nullptr));
     }
     const size_t slots = p->n_tiles * p->tile;
-    const size_t pe = split_elems_f32(M, p->n_tiles);
+    const size_t want = split_elems_f32(M, p->n_tiles);
+    size_t pe;
     // Targets on a lattice take the point-to-lattice kernel (default tiles; `skip`
     // as for the 16-row kernels above)
     const holo::Tuning& tu = holo::tuning();
@@ -1222,11 +1273,9 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
         pp.hi[d] = p->hi[d];
       }
       Sp = holo::point_splits(M, slots);
-      const size_t pp_elems = Sp > 1 ? (size_t)Sp * M : 0;
-      if (std::max(pe, pp_elems))
-        HOLO_TRY(ensure(ctx->partial, std::max(pe, pp_elems) * sizeof(double2), ctx->device));
-      HOLO_TRY(ensure(ctx->pairs, 256 + holo::kPairFlags * sizeof(uint32_t), ctx->device));
-      char* b = static_cast<char*>(ctx->pairs.ptr);
+      HOLO_TRY(partial_room(ctx, std::max(want, elems(Sp)), &pe));
+      Sp = (int)std::min<size_t>(Sp, std::max<size_t>(pe / M, 1));
+      char* b = plan_look(p, p->N);
       uint32_t* handled = reinterpret_cast<uint32_t*>(b + 128);
       HOLO_HIP(holo::launch_superpose_points(
           sign, obliquity, pp, wf, w0, w1, v, M, lambda, Sp,
@@ -1247,7 +1296,7 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
     ts.n_tiles = (uint32_t)p->n_tiles;
     ts.tile = p->tile;
     ts.planar = p->planar;
-    if (pe) HOLO_TRY(ensure(ctx->partial, pe * sizeof(double2), ctx->device));
+    HOLO_TRY(partial_room(ctx, want, &pe));
     HOLO_HIP(holo::launch_superpose_f32s(sign, obliquity, ts,
                                          static_cast<const float2*>(p->wc.ptr), v, M,
                                          lambda, reinterpret_cast<double2*>(y),
@@ -1469,8 +1518,8 @@ holo_status holo_transform_full(holo_ctx* ctx, holo_precision precision, int sig
     HOLO_TRY(report_zero(ctx, err_rel_l2, dev));
     const double* du;
     HOLO_TRY(stage_in(ctx, ctx->u, u, 3 * N, dev, &du));
-    const size_t pe = split_elems_f64(M, N);
-    if (pe) HOLO_TRY(ensure(ctx->partial, pe * sizeof(double2), ctx->device));
+    size_t pe;
+    HOLO_TRY(partial_room(ctx, split_elems_f64(M, N), &pe));
     const double K = (2 * M_PI) / lambda;  // TWO_PI_OVER_LAMBDA, cuda/macros.h:29-31
     if (dev && !holo::tuning().f64_libm) {
       // device positions: their layout is found on the device
@@ -1558,16 +1607,16 @@ holo_status holo_transform_mc(holo_ctx* ctx, holo_precision precision, int sign,
   HOLO_TRY(stage_in(ctx, ctx->u, u, 3 * N, dev, &du));
   HOLO_TRY(stage_in(ctx, ctx->v, v, 3 * M, dev, &dv));
   const bool fp64 = precision == HOLO_FP64;
-  HOLO_TRY(ensure(ctx->pos, N * sizeof(double4), ctx->device));
-  HOLO_TRY(ensure(ctx->ph, N * sizeof(double), ctx->device));
+  HOLO_TRY(ensure(ctx, ctx->pos, N * sizeof(double4)));
+  HOLO_TRY(ensure(ctx, ctx->ph, N * sizeof(double)));
   // per-target FP32-split draws on product-grid sources gather only the
   // weight; the grid is recognised on the device, without a host round trip
   const bool lattice = !fp64 && !(flags & HOLO_MC_SHARED);
   holo::McLattice lat;
   if (lattice) {
-    HOLO_TRY(ensure(ctx->mc_wc, N * sizeof(float2), ctx->device));
-    HOLO_TRY(ensure(ctx->mc_xy, (holo::kLatticeMaxRow + 1 + N) * sizeof(double), ctx->device));
-    HOLO_TRY(ensure(ctx->mc_info, 2 * sizeof(uint32_t), ctx->device));
+    HOLO_TRY(ensure(ctx, ctx->mc_wc, N * sizeof(float2)));
+    HOLO_TRY(ensure(ctx, ctx->mc_xy, (holo::kLatticeMaxRow + 1 + N) * sizeof(double)));
+    HOLO_TRY(ensure(ctx, ctx->mc_info, 2 * sizeof(uint32_t)));
     lat.info = static_cast<const uint32_t*>(ctx->mc_info.ptr);
     lat.wc = static_cast<const float2*>(ctx->mc_wc.ptr);
     lat.xy = static_cast<const double*>(ctx->mc_xy.ptr);
@@ -1583,17 +1632,18 @@ holo_status holo_transform_mc(holo_ctx* ctx, holo_precision precision, int sign,
   const double Kw = (2 * M_PI) / lambda;
   const bool shared = flags & HOLO_MC_SHARED, obl = flags & HOLO_OBLIQUITY;
   uint32_t chunk;
-  const size_t S = holo::mc_splits(M, K, fp64, shared, &chunk);
-  if (S > 1) HOLO_TRY(ensure(ctx->partial, S * M * sizeof(double2), ctx->device));
+  const size_t S = holo::mc_splits(M, K, fp64, shared, SIZE_MAX, &chunk);
+  size_t pe;
+  HOLO_TRY(partial_room(ctx, S > 1 ? S * M : 0, &pe));
   HOLO_HIP(holo::launch_mc(sign, fp64, shared, obl, static_cast<const double4*>(ctx->pos.ptr),
                            static_cast<const double*>(ctx->ph.ptr), N, dv, M, K, seed, Kw,
                            lambda, lat, reinterpret_cast<double2*>(dy),
-                           static_cast<double2*>(ctx->partial.ptr), ctx->stream));
+                           static_cast<double2*>(ctx->partial.ptr), pe, ctx->stream));
   // the FP64 estimator with the same indices at the report's targets
   HOLO_TRY(report_error(ctx, fp64, dv, M, dy, err_rel_l2, dev,
                         [&](const ErrScratch& e, size_t count) {
-                          HOLO_TRY(ensure(ctx->pos64, N * sizeof(double4), ctx->device));
-                          HOLO_TRY(ensure(ctx->ph64, N * sizeof(double), ctx->device));
+                          HOLO_TRY(ensure(ctx, ctx->pos64, N * sizeof(double4)));
+                          HOLO_TRY(ensure(ctx, ctx->ph64, N * sizeof(double)));
                           double4* p64 = static_cast<double4*>(ctx->pos64.ptr);
                           double* ph64 = static_cast<double*>(ctx->ph64.ptr);
                           HOLO_HIP(holo::launch_mc_pack(true, da, dp, du, N, p64, ph64, nullptr,
@@ -1638,7 +1688,7 @@ holo_status holo_normalize_polar(holo_ctx* ctx, const double* y, size_t M, doubl
   double *da, *dp;
   HOLO_TRY(out_buf(ctx, ctx->amp, amp, M, dev, &da));
   HOLO_TRY(out_buf(ctx, ctx->phase, phase, M, dev, &dp));
-  HOLO_TRY(ensure(ctx->small, 2048 * sizeof(double), ctx->device));
+  HOLO_TRY(ensure(ctx, ctx->small, 2048 * sizeof(double)));
   double* scratch = static_cast<double*>(ctx->small.ptr);
   double* dmax = (dev && max_amp) ? max_amp : scratch + 1024;
   HOLO_HIP(holo::launch_normalize_polar(reinterpret_cast<const double2*>(dy), M, da, dp, dmax,
@@ -1766,7 +1816,7 @@ holo_status holo_plan_adjoint(holo_ctx* ctx, const holo_plan* plan_targets,
   double *dga, *dgt;
   HOLO_TRY(out_buf(ctx, ctx->pos, grad_amp, N, dev, &dga));
   HOLO_TRY(out_buf(ctx, ctx->ph, grad_theta, N, dev, &dgt));
-  HOLO_TRY(ensure(ctx->b, 2 * N * sizeof(double), ctx->device));
+  HOLO_TRY(ensure(ctx, ctx->b, 2 * N * sizeof(double)));
   double* db = static_cast<double*>(ctx->b.ptr);
   const bool obl = flags & HOLO_OBLIQUITY;
   if (M == 0) {

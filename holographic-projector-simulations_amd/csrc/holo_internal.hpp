@@ -362,14 +362,15 @@ constexpr uint64_t kMcRecordDraws = uint64_t(1) << 26;
 hipError_t launch_mc(int sign, bool fp64, bool shared, bool obliquity, const double4* pos,
                      const double* ph, size_t N, const double* v, size_t M,
                      uint32_t K, uint64_t seed, double K_wave, double lambda,
-                     const McLattice& lat, double2* y, double2* partial, hipStream_t stream);
+                     const McLattice& lat, double2* y, double2* partial,
+                     size_t partial_cap, hipStream_t stream);
 // Splits S of the draws, of `chunk` each, up to kMcRound workgroups (shared subsets,
-// eight to a CU: 2048, which at 1024^2 targets takes 897 us for 1006); S > 1 needs S M partial values.  64^2 targets, K = 1024,
+// eight to a CU: 2048, which at 1024^2 targets takes 897 us for 1006); S > 1 needs S M partial values, of which there are `cap`.  64^2 targets, K = 1024,
 // 1024^2 lattice: 415 -> 97 us (one split and now), FP64 1.42 -> 0.18 ms; shared
 // subsets 580 -> 60 us, FP64 1.09 ms -> 90 us; below 128 draws (shared: 64) to a split
 // the tables and the reduction cost what it gives.
 constexpr size_t kMcMinDraws = 128;
-uint32_t mc_splits(size_t M, uint32_t K, bool fp64, bool shared, uint32_t* chunk);
+uint32_t mc_splits(size_t M, uint32_t K, bool fp64, bool shared, size_t cap, uint32_t* chunk);
 
 // The FP64 estimator at `count` targets vsub whose indices (Philox counters)
 // are tmap[i]: per target, or (shared) of the target's group; pos/ph packed

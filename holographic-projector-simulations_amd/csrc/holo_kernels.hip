@@ -1082,18 +1082,21 @@ static bool mc_round(size_t blocks, bool fp64) {
   return blocks <= (fp64 ? kMcRound / 3 : kMcRound);
 }
 
-uint32_t mc_splits(size_t M, uint32_t K, bool fp64, bool shared, uint32_t* chunk) {
+uint32_t mc_splits(size_t M, uint32_t K, bool fp64, bool shared, size_t cap,
+                   uint32_t* chunk) {
   const size_t group = shared ? kMcGroup : (size_t)kBlock, blocks = (M + group - 1) / group;
   const size_t fill = shared ? 2048 : kMcRound, least = shared ? 64 : kMcMinDraws;
   size_t S = std::min<size_t>({fill / blocks, K / least, 64});
   if (!shared && !mc_round(blocks, fp64)) S = 1;  // ranges add to y launch by launch
+  S = std::min(S, cap / M);
   return mc_chunk(K, S, shared ? 64 : 8, chunk);
 }
 
 hipError_t launch_mc(int sign, bool fp64, bool shared, bool obliquity, const double4* pos,
                      const double* ph, size_t N, const double* v, size_t M,
                      uint32_t K, uint64_t seed, double K_wave, double lambda,
-                     const McLattice& lat, double2* y, double2* partial, hipStream_t stream) {
+                     const McLattice& lat, double2* y, double2* partial,
+                     size_t partial_cap, hipStream_t stream) {
   if (!M) return hipSuccess;
   const double scale = (double)N / (double)K;
   const uint32_t slo = (uint32_t)seed, shi = (uint32_t)(seed >> 32);
@@ -1101,7 +1104,7 @@ hipError_t launch_mc(int sign, bool fp64, bool shared, bool obliquity, const dou
   const unsigned blocks = shared ? (unsigned)((M + kMcGroup - 1) / kMcGroup)
                                  : (unsigned)((M + kBlock - 1) / kBlock);
   uint32_t chunk;
-  const uint32_t S = mc_splits(M, K, fp64, shared, &chunk);
+  const uint32_t S = mc_splits(M, K, fp64, shared, partial_cap, &chunk);
   double2* out = S > 1 ? partial : y;
   const dim3 grid(blocks, S);
   const bool round = mc_round(blocks, fp64);

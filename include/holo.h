@@ -26,6 +26,13 @@
  *  - N and M must be below 2^31.  A source and a target at the same point
  *    (d = 0) yield a non-finite term, as in the reference.
  *  - One context per host thread; calls on one context are not reentrant.
+ *  - HIP graph capture: plan calls and FP64 transforms with device pointers may
+ *    be captured on the context's stream.  Nothing is allocated meanwhile: a
+ *    call takes as many source splits as the context's scratch holds (make the
+ *    call once before the capture for as many as it would take otherwise), and
+ *    one that cannot do without more scratch (Monte Carlo, adjoint, an error
+ *    report) returns HOLO_EDEVICE without queueing work.  Scratch that a graph
+ *    was captured with stays until the context is destroyed.
  *  - Error report (err_rel_l2, nullable, of every call that returns a field
  *    or gradients): for HOLO_FP32_SPLIT the call also evaluates the FP64
  *    formulation r64 at count = min(M, 256) targets of its result r (M
