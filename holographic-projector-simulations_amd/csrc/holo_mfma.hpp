@@ -15,7 +15,8 @@ typedef _Float16 ph2 __attribute__((ext_vector_type(2)));
 typedef _Float16 ph8 __attribute__((ext_vector_type(8)));
 typedef uint32_t pu4 __attribute__((ext_vector_type(4)));
 
-// PairTargets::mode: a form, with kPairWide the source tiles of 64 columns
+// PairTargets::mode: a form, or (lattice to lattice) kPairNear, which holds for every
+// tile pair, with kPairWide for the source tiles of 64 columns
 constexpr uint32_t kPairFar = 1, kPairNear = 2, kPairWide = 4;
 constexpr float kPairMid = 15.5f;  // a 32 x 32 tile's centre
 constexpr uint32_t kPairMaxRow = 16384;  // longest row of targets looked for
@@ -24,29 +25,40 @@ constexpr int kPairWaves = kBlock / 64;
 constexpr size_t kPairSlots = 2 * 256;
 constexpr float kFourPi = 12.566370614359172f;
 
-// The bounds of every dropped term over all tile pairs: rxm, rym the largest
-// lateral distances between tile centres, hx, hy the largest |rho|, dz the
-// distance of the planes (the smallest D).  kPairFar, kPairNear or 0.
-// cross = |C| of the first order at its largest, held to far_max and near_max.
-// NaN gives 0.
-__device__ __forceinline__ uint32_t pair_form(float rxm, float rym, float hx, float hy, float dz,
-                                              float inv_lambda, bool obl, float far_max,
-                                              float near_max) {
-  const float id = 1.f / dz, id2 = id * id, ia = id * inv_lambda;  // D = dz at least
-  const float Pm = 2.f * rxm * hx + hx * hx, Qm = 2.f * rym * hy + hy * hy;
+// The dropped terms of a tile pair at their largest: rx, ry the lateral distances
+// between the tile centres (or the largest of several pairs), hx, hy the largest
+// |rho|, id = 1 / D (or of the smallest D).  cross = |C| of the first order.
+struct PairTerms {
+  bool in_range;
+  float cross, cubic, cube, sq, q4;
+};
+
+__device__ __forceinline__ PairTerms pair_terms(float rx, float ry, float hx, float hy, float id,
+                                                float inv_lambda) {
+  const float id2 = id * id, ia = id * inv_lambda;
+  const float Pm = 2.f * rx * hx + hx * hx, Qm = 2.f * ry * hy + hy * hy;
   const float big = fmaxf(Pm, Qm), sum = Pm + Qm;
-  const float cross = 1.5707964f * ia * id2 * Pm * Qm;
   const float c3 = 0.0625f * ia * id2 * id2;
-  const float cubic = 18.849556f * c3 * Pm * Qm * sum;  // rad, the c3 part of C
-  const float sq = sum * id2;
+  PairTerms t;
   // alpha P, which cycles32 has to hold, and c2 P^2, in 2^-32 cycles an int32
-  if (!(0.5f * ia * sum <= 0x1p17f && 0.125f * ia * id2 * big * big <= 0.25f)) return 0u;
-  if (cross <= far_max && cubic <= 1e-6f && c3 * big * big * big <= 1e-8f &&
-      (obl ? 1.f : 0.5f) * sq * sq <= 1e-7f)
-    return kPairFar;
-  const float q4 = 0.0390625f * sum * sum * sum * sum * ia * id2 * id2 * id2;
-  if (cross <= near_max && cubic <= 4e-4f && q4 <= 1e-8f && sq * sq * sq <= 1e-7f) return kPairNear;
-  return 0u;
+  t.in_range = 0.5f * ia * sum <= 0x1p17f && 0.125f * ia * id2 * big * big <= 0.25f;
+  t.cross = 1.5707964f * ia * id2 * Pm * Qm;
+  t.cubic = 18.849556f * c3 * Pm * Qm * sum;  // rad, the c3 part of C
+  t.cube = c3 * big * big * big;
+  t.sq = sum * id2;
+  t.q4 = 0.0390625f * sum * sum * sum * sum * ia * id2 * id2 * id2;
+  return t;
+}
+
+// Whether the forms hold with cross up to `most`.  NaN gives false.
+__device__ __forceinline__ bool pair_far(const PairTerms& t, bool obl, float most) {
+  return t.in_range && t.cross <= most && t.cubic <= 1e-6f && t.cube <= 1e-8f &&
+         (obl ? 1.f : 0.5f) * t.sq * t.sq <= 1e-7f;
+}
+
+__device__ __forceinline__ bool pair_near(const PairTerms& t, float most) {
+  return t.in_range && t.cross <= most && t.cubic <= 4e-4f && t.q4 <= 1e-8f &&
+         t.sq * t.sq * t.sq <= 1e-7f;
 }
 
 // first k in [1, lim) for which hit(k) holds, else lim; the whole workgroup
@@ -151,6 +163,10 @@ __device__ __forceinline__ double lane_f64(double x, int lane) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
+__device__ __forceinline__ float lane_f32(float x, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+}
+
 // x + kCycles32 has ulp 2^-32 for |x| < 2^19 - 1: its low word is x modulo one
 // cycle, in 2^-32 cycles.
 constexpr double kCycles32 = 0x1.8p20;
@@ -237,12 +253,17 @@ __device__ __forceinline__ void cmul_hi(const Cplx8& a, const Cplx8& b, pf16& Dr
   Di = mfma32(a.ih, b.rh, Di);
 }
 
-// and of hi by lo and lo by hi parts
-__device__ __forceinline__ void cmul_lo(const Cplx8& a, const Cplx8& b, pf16& Dr, pf16& Di) {
+// of hi by lo parts
+__device__ __forceinline__ void cmul_hl(const Cplx8& a, const Cplx8& b, pf16& Dr, pf16& Di) {
   Dr = mfma32(a.rh, b.rl, Dr);
   Di = mfma32(a.rh, b.il, Di);
   Dr = mfma32(a.ih, neg8(b.il), Dr);
   Di = mfma32(a.ih, b.rl, Di);
+}
+
+// and of hi by lo and lo by hi parts
+__device__ __forceinline__ void cmul_lo(const Cplx8& a, const Cplx8& b, pf16& Dr, pf16& Di) {
+  cmul_hl(a, b, Dr, Di);
   Dr = mfma32(a.rl, b.rh, Dr);
   Di = mfma32(a.rl, b.ih, Di);
   Dr = mfma32(a.il, neg8(b.ih), Dr);

@@ -23,14 +23,18 @@
 //                  g_3 = -q^2 (sigma gP + i sigma q / 6),
 //     gP = s 6 pi c3 / (4 pi w^3), gQ = gP / (4 pi), k11 the amplitude's cross
 //     term, and the rows and columns carry c3 P^3 and the quadratic amplitude.
+// Every tile pair takes the far form within its bounds and the near form elsewhere.
 // Where the bounds ask for it the source tiles are 32 x 32 (halves of the others).
-// k_pair_prep picks the form from bounds over all tile pairs (pair_form), or
-// neither, and then the 16-row kernels run as if this kernel did not exist.
+// k_pair_prep picks the width from the near form's bounds over all tile pairs
+// (pair_mode), or neither, and then the 16-row kernels run as if this kernel did not
+// exist.  (One form for a whole call, far up to cross = 2.4e-3 and near up to 0.12, left
+// 2.0e-6 of the field for one lit source in a tile's corner; now 5.8e-7.)
 //
 // Operands are f16 pairs x = hi + lo (both rounded to nearest), and a full
 // product is hi hi + hi lo + lo hi, in FP32: only lo lo (2^-22, of either sign)
 // is left out.  g_0 and the near form's g_1 are full products; the far form's g_1
-// (below 2.4e-3 of the sum) and g_2, g_3 (below 7e-3) take the hi parts.  X
+// (below 1e-3 of the sum) and g_2, g_3 (below 1.8e-3) take the phasors' and weights' hi
+// parts and both of T's, which are sums (T's hi parts alone: 3 to 4 % less time).  X
 // carries A over the planes' 1 / |dz|.  The matrix cores' FP32 sums are rounded to
 // one side: in T that is turned by X's phases, but in the second product it would
 // add up over the tiles (1.6e-7 of the field over 1024 tiles; 5e-7 when one
@@ -54,12 +58,12 @@
 // phasors: X of target row j and Y of target column j.  Real and imaginary
 // parts are separate operands: T_re = Wr Yr + Wi (-Yi), T_im = Wr Yi + Wi Yr.
 //
-// What bounds it: VALU issue, 77 % busy (650 instructions per 2^20 pairs, half
-// of them for the phasors), beside matrix cores at 37 %; two waves per SIMD (242
-// VGPRs).  Per call, 1024^2 -> 1024^2: 2.0 ms at 0.35 m (5.4e14 pairs/s) where the
-// 16 x 64 tiles of k_superpose_grid16 take 57.8 ms, 4.9 ms at 0.2 m (93 ms), 6.5 ms
-// at 0.1 m (140 ms); 64^2 -> 64^2: 28 us (34 us).  With 32 x 32 source tiles the far
-// form took 2.75 ms at 1024^2.
+// What bounds it: VALU issue (650 instructions per 2^20 pairs in the far form before T's lo parts, half
+// of them for the phasors), beside the matrix cores; two waves per SIMD (253
+// VGPRs).  Per call, 1024^2 -> 1024^2 at 0.35 m: 2.37 ms, 3 % of the tile pairs near (one
+// form for all: 2.05 ms), where the 16 x 64 tiles of k_superpose_grid16 take 57.8 ms;
+// 512^2 -> 512^2 at 0.1 m 0.32 ms, 75 % near (8.2 ms); 64^2 -> 64^2: 28 us (34 us).  With
+// 32 x 32 source tiles the far form took 1.35 times as long at 1024^2.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -176,36 +180,50 @@ __device__ void pair_tail_weights(const PairPrep& a, double* s_red) {
   if (threadIdx.x == 0) a.tail_wc[0] = make_float2((float)s_red[0], (float)s_red[kBlock]);
 }
 
-// The form and source tile width for targets with the first and last tile centres
-// (cx0, cy0), (cx1, cy1).  rho has a triangular distribution, so the mean square of
-// an order-n term over a tile pair is below 0.07 (n = 2), 0.022 (n = 4) of its
-// largest: 1.9e-7 for the far form's cross^2 / 2 at 2.4e-3, 2e-7 for the near form's
-// cross^4 / 24 at 0.12, in the tile pairs that are furthest off axis.
+// The largest cross a tile pair takes each form with.  The far form drops C^2 / 2 and
+// the near form C^4 / 24; lowering the constant to 1 - m^2 / 4, m the pair's largest
+// |C|, leaves at most m^2 / 4 (2.5e-7), and 1 / 2 to 1 / 2 - m^2 / 24 in the C^2 term at
+// most m^4 / 96 (1.4e-7).  These hold for one lit source in the worst corner of its
+// tile; over dense weights C's triangular distribution leaves less.  The f16 parts that
+// the small products drop are of the same size: 1e-3 2^-12 and 0.06^2 / 2 2^-12.
+constexpr float kCrossFar = 1e-3f, kCrossNear = 0.06f;
+
+// The source tile width for targets with the first and last tile centres (cx0, cy0),
+// (cx1, cy1): the wide tiles where the near form holds for every pair of them, but the
+// narrow ones where those are all far and the wide ones mostly are not (judged midway
+// between the lattices).
 __device__ uint32_t pair_mode(const PairPrep& a, const PairTargets& t, double cx0, double cx1,
                               double cy0, double cy1) {
   const auto far = [](double a0, double a1, double b0, double b1) {
     return fmax(fmax(fabs(a0 - b0), fabs(a0 - b1)), fmax(fabs(a1 - b0), fabs(a1 - b1)));
   };
+  const auto mid = [](double a0, double a1, double b0, double b1) {
+    return 0.5 * fabs(a0 + a1 - b0 - b1);
+  };
   // source tile centres: rows, and columns of wide and of narrow tiles
   const double sx0 = a.sx + (double)kPairMid * a.spx;
   const double sx1 = sx0 + (double)(((a.nx + 31) / 32 - 1) * 32) * a.spx;
-  uint32_t mode = 0u;
-  const float rxm = (float)far(cx0, cx1, sx0, sx1);
   const float hx = (float)((double)kPairMid * (fabs(t.px) + fabs(a.spx)));
-  const float dz = (float)fabs(t.z - a.sz), il = (float)a.inv_lambda;
-  for (int wide = 1; wide >= 0; --wide) {
-    const double mid = wide ? 31.5 : (double)kPairMid;
+  const double dz = fabs(t.z - a.sz);
+  const float il = (float)a.inv_lambda;
+  bool near[2], all_far[2], mid_far[2];
+  for (int wide = 0; wide < 2; ++wide) {
+    const double half = wide ? 31.5 : (double)kPairMid;
     const uint32_t cols = wide ? 64 : 32;
-    const double sy0 = a.sy + mid * a.spy;
+    const double sy0 = a.sy + half * a.spy;
     const double sy1 = sy0 + (double)(((a.ny + cols - 1) / cols - 1) * cols) * a.spy;
-    const float rym = (float)far(cy0, cy1, sy0, sy1);
-    const float hy = (float)((double)kPairMid * fabs(t.py) + mid * fabs(a.spy));
-    const uint32_t f = pair_form(rxm, rym, hx, hy, dz, il, a.obl != 0, 2.4e-3f, 0.12f);
-    // a wide far form beats everything, and a narrow far form a wide near one
-    if (f && (!mode || (f == kPairFar && mode != (kPairFar | kPairWide))))
-      mode = f | (wide ? kPairWide : 0u);
+    const float hy = (float)((double)kPairMid * fabs(t.py) + half * fabs(a.spy));
+    const PairTerms d = pair_terms((float)far(cx0, cx1, sx0, sx1), (float)far(cy0, cy1, sy0, sy1),
+                                   hx, hy, 1.f / (float)dz, il);
+    near[wide] = pair_near(d, kCrossNear);
+    all_far[wide] = pair_far(d, a.obl != 0, kCrossFar);
+    const double mx = mid(cx0, cx1, sx0, sx1), my = mid(cy0, cy1, sy0, sy1);
+    mid_far[wide] = pair_far(pair_terms((float)mx, (float)my, hx, hy,
+                                        1.f / (float)sqrt(mx * mx + my * my + dz * dz), il),
+                             a.obl != 0, kCrossFar);
   }
-  return mode;
+  if (near[1] && (mid_far[1] || !all_far[0])) return kPairNear | kPairWide;
+  return near[0] ? kPairNear : 0u;
 }
 
 __global__ __launch_bounds__(kBlock) void k_pair_prep(PairPrep a, Grid16Prep g) {
@@ -260,6 +278,7 @@ struct PairWave {
   float a0X, a1X, a2X;        // X's amplitude in p: A |dz| (1 + k1 P + k2 P^2)
   float a1Y, a2Y;             // Y's: 1 + k1 Q + k2 Q^2
   float c3X, c3Y, k11, gP, gQ;  // near form (c3X, c3Y in 2^-32 cycles)
+  float half;                   // near form: the C^2 term's coefficient
   float one;                  // 1, unknown to the compiler: x - hi as one mixed FMA
 
   // phasors of step s along AXIS (0: x, 1: y)
@@ -298,7 +317,6 @@ struct PairWave {
 };
 
 // registers 8 s .. 8 s + 7 of T as the second product's B operand
-template <bool FULL>
 __device__ __forceinline__ Cplx8 operand_of(const pf16& Tr, const pf16& Ti, int s, float one) {
   Cplx8 o;
   float r[8], i[8];
@@ -307,13 +325,8 @@ __device__ __forceinline__ Cplx8 operand_of(const pf16& Tr, const pf16& Ti, int 
     r[e] = Tr[8 * s + e];
     i[e] = Ti[8 * s + e];
   }
-  if constexpr (FULL) {
-    split8(r, one, o.rh, o.rl);
-    split8(i, one, o.ih, o.il);
-  } else {
-    o.rh = half8(r);
-    o.ih = half8(i);
-  }
+  split8(r, one, o.rh, o.rl);
+  split8(i, one, o.ih, o.il);
   return o;
 }
 
@@ -358,7 +371,7 @@ __device__ __forceinline__ void pair_products(const PairWave<SIGN, OBL>& pw, con
           gi = q * __builtin_fmaf(pw.gQ, q, kSig);
         } else {
           const float q2 = q * q;
-          const float hr = -q2 * __builtin_fmaf(kSig * pw.gQ, q, 0.5f), hi = pw.gP * q;
+          const float hr = -q2 * __builtin_fmaf(kSig * pw.gQ, q, pw.half), hi = pw.gP * q;
           ar[e] = hr * yr - hi * yi;
           ai[e] = hr * yi + hi * yr;
           gr = -kSig * pw.gP * q2;
@@ -435,16 +448,19 @@ __device__ __forceinline__ void pair_products(const PairWave<SIGN, OBL>& pw, con
         b.ih = half8(bi);
       }
     }
-    const Cplx8 tb = operand_of<PART == 1>(Br, Bi, s, pw.one);
+    const Cplx8 tb = operand_of(Br, Bi, s, pw.one);
     if constexpr (PART == 0) {
+      cmul_hl(b, tb, Lr, Li);
       cmul_hi(b, tb, Lr, Li);
     } else {
       if constexpr (PART == 1) cmul_lo(b, tb, Dr, Di);
+      if constexpr (PART == 2) cmul_hl(b, tb, Dr, Di);
       cmul_hi(b, tb, Dr, Di);
     }
-    const Cplx8 ta = operand_of<PART != 2>(Ar, Ai, s, pw.one);
+    const Cplx8 ta = operand_of(Ar, Ai, s, pw.one);
     if constexpr (PART == 0) cmul_lo(a, ta, Lr, Li);
     if constexpr (PART == 1) cmul_lo(a, ta, Dr, Di);
+    if constexpr (PART == 2) cmul_hl(a, ta, Dr, Di);
     cmul_hi(a, ta, Dr, Di);
   }
   if constexpr (PART == 0) {
@@ -469,7 +485,7 @@ struct PairSources {
 // shared out over the workgroup's waves, whose sums are added at the end, so that
 // a call of few tiles still occupies four SIMDs a tile and most calls have one
 // split, which writes the result itself.
-template <bool NEAR, int SIGN, bool OBL>
+template <int SIGN, bool OBL>
 __device__ __forceinline__ void pair_items(PairWave<SIGN, OBL>& pw, const PairSources& sr,
                                            const PairTargets& pt, uint32_t S, uint32_t M,
                                            double inv_lambda, double2* __restrict__ out) {
@@ -490,30 +506,37 @@ __device__ __forceinline__ void pair_items(PairWave<SIGN, OBL>& pw, const PairSo
   // source tiles of this mode, tj per row; a wide tile may lack its second half,
   // whose weights are then 0
   const uint32_t stj = wide ? sr.tj : (sr.ny + 31) / 32;
-  const uint32_t nst = sr.n_tiles / sr.tj * stj, chunk = (nst + parts - 1) / parts;
+  const uint32_t nst = sr.n_tiles / sr.tj * stj, chunk = (nst + parts - 1) / parts * kPairWaves;
   const double bX = -2.0 * (ti * pt.px * sr.px), bY = -2.0 * (ti * pt.py * sr.py);
   // slot 0's source, from the centre, along x and y
   const double hKX = 4.0 * (double)h - (double)kPairMid, hKY = 4.0 * (double)h - midY;
   const double rz = pt.z - sr.z;
   const float arz = (float)fabs(rz);
   const double irz = 1.0 / fabs(rz);  // X's amplitude is relative to it
+  const float hx = (float)((double)kPairMid * (fabs(pt.px) + fabs(sr.px)));
+  const float hy = (float)((double)kPairMid * fabs(pt.py) + midY * fabs(sr.py));
   for (uint32_t item = blockIdx.x; item < items; item += gridDim.x) {
     const uint32_t split = item % S, tile = item / S;
     const uint32_t I = tile / TJ, J = tile - I * TJ;
     const double tcx = pt.x0 + ((double)(32 * I) + (double)kPairMid) * pt.px;
     const double tcy = pt.y0 + ((double)(32 * J) + (double)kPairMid) * pt.py;
-    const uint32_t s0 = min(nst, (split * kPairWaves + wv) * chunk), s1 = min(nst, s0 + chunk);
+    // this wave's source tiles: s0 + wv, + 4, .. of the split's (the ones that take the
+    // near form lie side by side: with a run of tiles for each wave one wave had them
+    // all, and 1024^2 to 1024^2 took 2.5 ms)
+    const uint32_t s0 = min(nst, split * chunk), s1 = min(nst, s0 + chunk);
+    const uint32_t n = s1 > s0 + wv ? (s1 - s0 - wv + kPairWaves - 1) / kPairWaves : 0u;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       lds.re[wv][r][lane] = 0.0;
       lds.im[wv][r][lane] = 0.0;
     }
-    for (uint32_t base = s0; base < s1; base += 64) {
+    for (uint32_t base = 0; base < n; base += 64) {
       // the FP64 constants of up to 64 source tiles, one per lane
       double hrx, hry, hal, hf;
-      float hid;
+      float hid, hcr;
+      uint64_t far;
       {
-        const uint32_t t = min(base + lane, s1 - 1);
+        const uint32_t t = s0 + wv + kPairWaves * min(base + lane, n - 1);
         const uint32_t si = t / stj, sj = t - si * stj;
         hrx = tcx - (sr.x0 + ((double)(32 * si) + (double)kPairMid) * sr.px);
         hry = tcy - (sr.y0 + ((double)((wide ? 64 : 32) * sj) + midY) * sr.py);
@@ -522,14 +545,17 @@ __device__ __forceinline__ void pair_items(PairWave<SIGN, OBL>& pw, const PairSo
         hal = 0.5 * id * inv_lambda;
         hf = frac_cycle(d * inv_lambda);
         hid = (float)id;
+        const PairTerms d2 = pair_terms(fabsf((float)hrx), fabsf((float)hry), hx, hy, hid,
+                                        (float)inv_lambda);
+        hcr = d2.cross;
+        far = __builtin_amdgcn_ballot_w64(pair_far(d2, OBL, kCrossFar));
       }
-      const uint32_t cnt = min(64u, s1 - base);
+      const uint32_t cnt = min(64u, n - base);
       for (uint32_t k = 0; k < cnt; ++k) {
-        const uint32_t t = base + k;
+        const uint32_t t = s0 + wv + kPairWaves * (base + k);
         const double rx = lane_f64(hrx, (int)k), ry = lane_f64(hry, (int)k);
         const double al = lane_f64(hal, (int)k), f = lane_f64(hf, (int)k);
-        const float id = __builtin_bit_cast(
-            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, hid), (int)k));
+        const float id = lane_f32(hid, (int)k), cross = lane_f32(hcr, (int)k);
         const float id2 = id * id, alf = (float)al;
         // p = w P with w^2 = |c2| = alpha / (4 D^2), q = 4 pi w Q
         const float w = 0.5f * id * __builtin_amdgcn_sqrtf(alf);
@@ -566,12 +592,14 @@ __device__ __forceinline__ void pair_items(PairWave<SIGN, OBL>& pw, const PairSo
         const uint32_t steps = wide ? 4u : 2u;
         const float tst = sr.tscale[ti2];
         const float iY = (1.f / kFourPi) * iw;  // 1 / wY
+        const bool near = !(far >> k & 1);  // uniform
         pw.a0X = OBL ? (arz * id) * (arz * id) : arz * id;
+        if (!near) pw.a0X -= 0.25f * cross * cross * pw.a0X;
         pw.a1X = pw.a0X * ((OBL ? -1.f : -0.5f) * id2 * iw);
         pw.a1Y = (OBL ? -1.f : -0.5f) * id2 * iY;
-        // odd tiles enter the matrix cores with the opposite sign
-        pw.FtX += t << 31;
-        const float unit = t & 1 ? -tst : tst;
+        // every other tile enters the matrix cores with the opposite sign
+        pw.FtX += k << 31;
+        const float unit = k & 1 ? -tst : tst;
         const auto add = [&](auto part) __attribute__((always_inline)) {
           pf16 Dr = kZero16, Di = kZero16;
           pair_products<decltype(part)::value>(pw, wt, steps, Dr, Di);
@@ -581,7 +609,7 @@ __device__ __forceinline__ void pair_items(PairWave<SIGN, OBL>& pw, const PairSo
             lds_add(&lds.im[wv][r][lane], (double)(unit * Di[r]));
           }
         };
-        if constexpr (!NEAR) {
+        if (!near) {
           add(IC<0>{});
         } else {
           constexpr float k2 = OBL ? 1.f : 0.375f, k11 = OBL ? 1.f : 0.5f;
@@ -593,6 +621,7 @@ __device__ __forceinline__ void pair_items(PairWave<SIGN, OBL>& pw, const PairSo
           pw.k11 = k11 * (id2 * iw) * (id2 * iY);
           pw.gP = (float)SIGN * 9.424778f * id2 * iY;              // s 6 pi c3 / (w^2 wY)
           pw.gQ = (float)SIGN * 9.424778f / kFourPi * id2 * iY;   // s 6 pi c3 / (w wY^2)
+          pw.half = __builtin_fmaf(-1.f / 24.f, cross * cross, 0.5f);
           add(IC<1>{});
           // the same phasors again: kept from the first part, and with its results,
           // they would not fit the registers
@@ -653,10 +682,7 @@ k_superpose_pairs(PairSources sr, const PairTargets* __restrict__ ptp,
                          (threadIdx.x & 63) >> 5, threadIdx.x & 31};
   pw.one = 1.f;
   __asm__("" : "+v"(pw.one));
-  if (pt.mode & kPairNear)
-    pair_items<true, SIGN, OBL>(pw, sr, pt, S, M, inv_lambda, out);
-  else
-    pair_items<false, SIGN, OBL>(pw, sr, pt, S, M, inv_lambda, out);
+  pair_items<SIGN, OBL>(pw, sr, pt, S, M, inv_lambda, out);
 }
 
 // One split where the target tiles fill the slots many times over; else the

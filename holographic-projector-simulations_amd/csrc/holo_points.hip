@@ -354,12 +354,15 @@ __global__ __launch_bounds__(kBlock) void k_point_prep(PointPlan pp, int wf,
                     return fmax(fabs(fmax(a0, a1) - b0), fabs(b1 - fmin(a0, a1)));
                   };
                   const double gap = plane_gap(t.z, pp);
-                  return pair_form((float)far(cx0, cx1, pp.lo[0], pp.hi[0]),
-                                   (float)far(cy0, cy1, pp.lo[1], pp.hi[1]),
-                                   (float)((double)kPairMid * fabs(t.px)),
-                                   (float)((double)kPairMid * fabs(t.py)),
-                                   (float)gap, (float)inv_lambda, obl != 0, 1.2e-3f,
-                                   0.07f);
+                  const PairTerms d =
+                      pair_terms((float)far(cx0, cx1, pp.lo[0], pp.hi[0]),
+                                 (float)far(cy0, cy1, pp.lo[1], pp.hi[1]),
+                                 (float)((double)kPairMid * fabs(t.px)),
+                                 (float)((double)kPairMid * fabs(t.py)), 1.f / (float)gap,
+                                 (float)inv_lambda);
+                  return pair_far(d, obl != 0, 1.2e-3f) ? kPairFar
+                         : pair_near(d, 0.07f)          ? kPairNear
+                                                        : 0u;
                 });
 }
 
