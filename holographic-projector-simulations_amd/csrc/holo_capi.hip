@@ -1054,6 +1054,12 @@ holo_status plan_build(holo_ctx* ctx, holo_plan* p, const double* u, size_t N,
   return HOLO_OK;
 }
 
+// Smallest call that looks for a lattice on the device.  The search and its answer
+// take 28 us where there is none (64 jittered sources 118 us with and 91 without, 1024
+// 162 and 133; with a plan's allocations in every call 95 and 311, 256 128 us), and save 18 us where
+// there is one (64 sources 70 and 88 us, 1024 71 and 98).
+constexpr size_t kFindSources = 384;
+
 // plan_build for one call with device positions on a uniform lattice that the 16-row
 // and lattice-to-lattice kernels take, found and cut on the device (*found; else
 // nothing is built).  512^2 sources to 512^2 targets: 2.13 ms with plan_build and a plan's
@@ -1062,7 +1068,7 @@ holo_status plan_build_lattice(holo_ctx* ctx, holo_plan* p, const double* u, siz
                                bool* found) {
   *found = false;
   const holo::Tuning& tu = holo::tuning();
-  if (N < 64 || !tu.grid || !tu.grid16) return HOLO_OK;
+  if (N < kFindSources || !tu.grid || !tu.grid16) return HOLO_OK;
   HOLO_TRY(plan_positions(ctx, p, N));
   holo::LatticeInfo* di = reinterpret_cast<holo::LatticeInfo*>(plan_look(p, N));
   HOLO_HIP(holo::launch_find_lattice(u, N, di, ctx->stream));
