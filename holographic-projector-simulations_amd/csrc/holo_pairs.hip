@@ -75,15 +75,16 @@
 namespace holo {
 
 constexpr int kPairTile = 32;  // rows and columns of a target tile, rows of a source tile
-// MFMA operands of one 32 x 64 source tile's weights by one workgroup, and the
+// MFMA operands of one 32 x 64 source tile's weights by four workgroups, and the
 // target lattice by the n_probe workgroups after them (tail sources' weights by
-// one before those); the rest, if any, prepare the 16-row kernels' weights.
+// one before those); the rest, if any, prepare the 16-row kernels' weights.  What bounds
+// it is the FP64 sin and cos that a lane forms one after the other: with eight in each
+// (one workgroup a tile) a call of 16^2 or 64^2 sources spent 6.6 or 7.5 us here, 5.2 and 4.8 now.
 //
 // Weights: wq[(16 t + 4 s + 2 c + l) * 64 + lane] (8 f16) holds, for step s < 4
 // (columns 16 s ..), component c (re, im) and part l (hi, lo), row delta_x =
 // lane % 32 of tile t over its scale tscale[t] (the power of two above its
-// largest component); slots beyond the lattice are 0.  Wave v of the workgroup
-// forms step v.
+// largest modulus, or component of complex weights); slots beyond the lattice are 0.
 //
 // Targets: probe_targets.
 struct PairPrep {
@@ -101,23 +102,31 @@ struct PairPrep {
   uint32_t* flags;
 };
 
-__device__ __forceinline__ float2 pair_weight(const PairPrep& a, uint32_t n) {
-  return slot_weight(a.wf, a.w0, a.w1, (int32_t)n);
-}
-
-__device__ void pair_tile_weights(const PairPrep& a, uint32_t t, float* s_max) {
+// Columns 16 step .. 16 step + 15 of tile t: two sources' weights a lane, laid out
+// through LDS (s_w: 32 x 17 float2).
+__device__ void pair_tile_weights(const PairPrep& a, uint32_t t, uint32_t step, float* s_max,
+                                  float2* s_w) {
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const uint32_t I = t / a.tj, J = t - I * a.tj;
-  const uint32_t i = kPairTile * I + (lane & 31);
-  const uint32_t j0 = 2 * kPairTile * J + 16 * wv + 4 * (lane >> 5);
-  float2 w[8];
+  const auto source = [&](uint32_t row, uint32_t col) {
+    const uint32_t i = kPairTile * I + row, j = 2 * kPairTile * J + col;
+    return i < a.nx && j < a.ny ? (int32_t)(i * a.ny + j) : -1;
+  };
+  // the bound of the whole tile's components: the moduli's (polar) or their own
   float mx = 0.f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const uint32_t j = j0 + 8 * (e >> 2) + (e & 3);
-    w[e] = make_float2(0.f, 0.f);
-    if (i < a.nx && j < a.ny) w[e] = pair_weight(a, i * a.ny + j);
-    mx = fmaxf(mx, fmaxf(fabsf(w[e].x), fabsf(w[e].y)));
+  for (uint32_t e = 0; e < 8; ++e) {
+    const int32_t n = source(4 * e + wv, lane);
+    if (n < 0) continue;
+    if (a.wf == kPolar)
+      mx = fmaxf(mx, fabsf((float)a.w0[n]));
+    else
+      mx = fmaxf(mx, fmaxf(fabsf((float)a.w0[2 * (size_t)n]), fabsf((float)a.w0[2 * (size_t)n + 1])));
+  }
+#pragma unroll
+  for (uint32_t e = 0; e < 2; ++e) {
+    const uint32_t row = 16 * e + (threadIdx.x >> 4), col = threadIdx.x & 15;
+    s_w[17 * row + col] = slot_weight(a.wf, a.w0, a.w1, source(row, 16 * step + col));
   }
   for (int off = 32; off; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
   if (lane == 0) s_max[wv] = mx;
@@ -127,23 +136,20 @@ __device__ void pair_tile_weights(const PairPrep& a, uint32_t t, float* s_max) {
   if (mx > 0.f && __builtin_isfinite(mx)) frexpf(mx, &e2);
   e2 = e2 < -126 ? -126 : (e2 > 127 ? 127 : e2);
   const float is = ldexpf(1.f, -e2);
-  ph8 op[4];  // re hi, re lo, im hi, im lo
+  // wave 2 c + l: component c, part l
+  const float2* w = s_w + 17 * (lane & 31) + 4 * (lane >> 5);
+  ph8 op;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const float c[2] = {w[e].x * is, w[e].y * is};
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      // 11 significant bits by integer rounding: exact in f16, and lo exact
-      const float h = __builtin_bit_cast(
-          float, (__builtin_bit_cast(uint32_t, c[k]) + 0x1000u) & 0xffffe000u);
-      op[2 * k][e] = (_Float16)h;
-      op[2 * k + 1][e] = (_Float16)(c[k] - h);
-    }
+    const float2 x = w[8 * (e >> 2) + (e & 3)];
+    const float c = (wv & 2 ? x.y : x.x) * is;
+    // 11 significant bits by integer rounding: exact in f16, and lo exact
+    const float h = __builtin_bit_cast(
+        float, (__builtin_bit_cast(uint32_t, c) + 0x1000u) & 0xffffe000u);
+    op[e] = (_Float16)(wv & 1 ? c - h : h);
   }
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    a.wq[((size_t)16 * t + 4 * wv + q) * 64 + lane] = __builtin_bit_cast(pu4, op[q]);
-  if (threadIdx.x == 0) a.tscale[t] = ldexpf(1.f, e2);
+  a.wq[((size_t)16 * t + 4 * step + wv) * 64 + lane] = __builtin_bit_cast(pu4, op);
+  if (step == 0 && threadIdx.x == 0) a.tscale[t] = ldexpf(1.f, e2);
 }
 
 // FP32 weights of the sources after the lattice; when they all sit at one
@@ -151,7 +157,7 @@ __device__ void pair_tile_weights(const PairPrep& a, uint32_t t, float* s_max) {
 __device__ void pair_tail_weights(const PairPrep& a, double* s_red) {
   const uint32_t body = a.nx * a.ny;
   if (!a.tail_same) {
-    for (uint32_t k = threadIdx.x; k < a.n_tail; k += kBlock) a.tail_wc[k] = pair_weight(a, body + k);
+    for (uint32_t k = threadIdx.x; k < a.n_tail; k += kBlock) a.tail_wc[k] = slot_weight(a.wf, a.w0, a.w1, (int32_t)(body + k));
     return;
   }
   double re = 0.0, im = 0.0;
@@ -227,13 +233,15 @@ __device__ uint32_t pair_mode(const PairPrep& a, const PairTargets& t, double cx
 }
 
 __global__ __launch_bounds__(kBlock) void k_pair_prep(PairPrep a, Grid16Prep g) {
-  __shared__ double s_buf[2 * kBlock];
+  __shared__ double s_buf[2 * kBlock + 64];
+  static_assert(sizeof(s_buf) >= 32 * 17 * sizeof(float2) + kPairWaves * sizeof(float), "s_w, s_max");
   uint32_t b = blockIdx.x;
-  if (b < a.n_tiles) {
-    pair_tile_weights(a, b, reinterpret_cast<float*>(s_buf));
+  if (b < 4 * a.n_tiles) {
+    float2* s_w = reinterpret_cast<float2*>(s_buf);
+    pair_tile_weights(a, b >> 2, b & 3, reinterpret_cast<float*>(s_w + 32 * 17), s_w);
     return;
   }
-  b -= a.n_tiles;
+  b -= 4 * a.n_tiles;
   if (a.n_tail) {
     if (b == 0) {
       pair_tail_weights(a, s_buf);
@@ -741,7 +749,7 @@ hipError_t launch_superpose_pairs(int sign, bool obliquity, const PairPlan& pp, 
   a.pt = pt;
   a.flags = flags;
   const Grid16Prep g = grid16 ? *grid16 : Grid16Prep{};
-  const unsigned blocks = pp.n_tiles + (pp.n_tail ? 1u : 0u) + n_probe +
+  const unsigned blocks = 4 * pp.n_tiles + (pp.n_tail ? 1u : 0u) + n_probe +
                           (grid16 ? grid16_weight_blocks(g) : 0u);
   k_pair_prep<<<blocks, kBlock, 0, stream>>>(a, g);
   hipError_t e = hipGetLastError();

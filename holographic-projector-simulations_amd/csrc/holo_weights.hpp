@@ -57,22 +57,20 @@ __device__ __forceinline__ void grid16_weights(const Grid16Prep& a, uint32_t blo
     return;
   }
   __shared__ float s_max[kGridWaves];
+  __shared__ float2 s_w[kGridWaves][256];
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const uint32_t t = block * kGridWaves + wv;
   const uint32_t i = lane & 15, g = lane >> 4, ap = i >> 1, co = i & 1;
-  float2 w[2][4];
   float mx = 0.f;
   if (t < a.n_tiles) {  // uniform per wave
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const size_t at = (size_t)t * 256 + 16 * (8 * rb + ap) + 4 * g + q;
-        w[rb][q] = slot_weight(a.wf, a.w0, a.w1, a.perm[at]);
-        // lanes i = 2 ap and 2 ap + 1 hold the same weight
-        if (co == 0) a.wc[at] = w[rb][q];
-        mx = fmaxf(mx, fmaxf(fabsf(w[rb][q].x), fabsf(w[rb][q].y)));
-      }
+    for (uint32_t q = 0; q < 4; ++q) {
+      const size_t at = (size_t)t * 256 + 64 * q + lane;
+      const float2 x = slot_weight(a.wf, a.w0, a.w1, a.perm[at]);
+      a.wc[at] = x;
+      s_w[wv][64 * q + lane] = x;
+      mx = fmaxf(mx, fmaxf(fabsf(x.x), fabsf(x.y)));
+    }
   }
   for (int off = 32; off; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
   if (lane == 0) s_max[wv] = mx;
@@ -84,6 +82,11 @@ __device__ __forceinline__ void grid16_weights(const Grid16Prep& a, uint32_t blo
   if (mx > 0.f && __builtin_isfinite(mx)) frexpf(mx, &e);
   e = e < -126 ? -126 : (e > 127 ? 127 : e);
   const float is = ldexpf(1.f, -e);
+  float2 w[2][4];
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w[rb][q] = s_w[wv][16 * (8 * rb + ap) + 4 * g + q];
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
     const float kr = (float)(8 * rb + ap) - 7.5f;
