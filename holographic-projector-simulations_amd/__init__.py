@@ -86,6 +86,7 @@ def lib() -> ctypes.CDLL:
     L.holo_destroy.restype = None
     L.holo_set_stream.argtypes = [vp, vp]
     L.holo_synchronize.argtypes = [vp]
+    L.holo_trim.argtypes = [vp]
     L.holo_set_option.argtypes = [ctypes.c_char_p, ctypes.c_long]
     L.holo_get_option.argtypes = [ctypes.c_char_p]
     L.holo_get_option.restype = ctypes.c_long
@@ -121,7 +122,7 @@ def lib() -> ctypes.CDLL:
     L.holo_host_sincos.restype = None
     L.holo_host_sqrt_inv.argtypes = [d, dp, dp]
     L.holo_host_sqrt_inv.restype = None
-    for name in ("holo_create", "holo_set_stream", "holo_synchronize", "holo_set_option",
+    for name in ("holo_create", "holo_set_stream", "holo_synchronize", "holo_trim", "holo_set_option",
                  "holo_transform_full", "holo_transform_full_noalloc", "holo_transform_mc",
                  "holo_mc_indices",
                  "holo_normalize_polar", "holo_plan_create", "holo_plan_info", "holo_plan_lattice",
@@ -244,6 +245,10 @@ class Context:
 
     def synchronize(self) -> None:
         check(lib().holo_synchronize(self._h))
+
+    def trim(self) -> None:
+        """Wait for the context's work and free its device scratch."""
+        check(lib().holo_trim(self._h))
 
     def _torch_stream(self):
         import torch

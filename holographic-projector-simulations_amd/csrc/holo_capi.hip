@@ -1428,6 +1428,18 @@ holo_status holo_synchronize(holo_ctx* ctx) {
   return HOLO_OK;
 }
 
+holo_status holo_trim(holo_ctx* ctx) {
+  HOLO_TRY(use_device(ctx));
+  if (ctx->capturing) return fail(HOLO_EINVAL, "the context's stream is being captured");
+  HOLO_HIP(hipStreamSynchronize(ctx->stream));
+  ctx->shot.reset();
+  for (DevBuf* b : {&ctx->amp, &ctx->phase, &ctx->u, &ctx->v, &ctx->y, &ctx->w, &ctx->partial,
+                    &ctx->small, &ctx->b, &ctx->pos, &ctx->ph, &ctx->mc_wc, &ctx->mc_xy,
+                    &ctx->mc_info, &ctx->errb, &ctx->pos64, &ctx->ph64})
+    if (!b->graph) b->release();
+  return HOLO_OK;
+}
+
 holo_status holo_set_option(const char* name, long value) {
   if (!name) return fail(HOLO_EINVAL, "null option name");
   holo::Tuning& t = holo::tuning();

@@ -31,8 +31,8 @@
  *    call takes as many source splits as the context's scratch holds (make the
  *    call once before the capture for as many as it would take otherwise), and
  *    one that cannot do without more scratch (Monte Carlo, adjoint, an error
- *    report) returns HOLO_EDEVICE without queueing work.  Scratch that a graph
- *    was captured with stays until the context is destroyed.
+ *    report) returns HOLO_EDEVICE.  Scratch that a graph was captured with stays
+ *    until the context is destroyed.
  *  - Error report (err_rel_l2, nullable, of every call that returns a field
  *    or gradients): for HOLO_FP32_SPLIT the call also evaluates the FP64
  *    formulation r64 at count = min(M, 256) targets of its result r (M
@@ -110,6 +110,14 @@ void holo_destroy(holo_ctx *ctx);
  * must stay valid while it is the context's stream. */
 holo_status holo_set_stream(holo_ctx *ctx, void *stream);
 holo_status holo_synchronize(holo_ctx *ctx);
+/* Wait for the context's work and free its device scratch, which calls otherwise
+ * keep for the next one: staging copies of host arrays, split partials (up to
+ * 280 MB with automatic splits), Monte Carlo records (40 to 96 bytes a source)
+ * and, for HOLO_FP32_SPLIT calls without a plan of up to
+ * 2^22 sources, the buffers of the last one's plan (about 120 bytes a source, at
+ * most 0.5 GB).  Later calls allocate what they need again.  Scratch that a
+ * captured graph uses stays. */
+holo_status holo_trim(holo_ctx *ctx);
 
 /* Tuning knobs (process-wide): "r_f64", "r_f32" targets per lane (1, 2, 4;
  * the FP64 kernel takes fewer where that fills the GPU better, unless "splits" is set),
