@@ -35,18 +35,20 @@ struct PairTerms {
 
 __device__ __forceinline__ PairTerms pair_terms(float rx, float ry, float hx, float hy, float id,
                                                 float inv_lambda) {
-  const float id2 = id * id, ia = id * inv_lambda;
-  const float Pm = 2.f * rx * hx + hx * hx, Qm = 2.f * ry * hy + hy * hy;
-  const float big = fmaxf(Pm, Qm), sum = Pm + Qm;
-  const float c3 = 0.0625f * ia * id2 * id2;
+  // P, Q over D^2, and D / lambda: the same at every scale of lengths
+  const float id2 = id * id, dl = inv_lambda / id;
+  const float p = (2.f * rx * hx + hx * hx) * id2, q = (2.f * ry * hy + hy * hy) * id2;
+  const float big = fmaxf(p, q), sum = p + q;
   PairTerms t;
-  // alpha P, which cycles32 has to hold, and c2 P^2, in 2^-32 cycles an int32
-  t.in_range = 0.5f * ia * sum <= 0x1p17f && 0.125f * ia * id2 * big * big <= 0.25f;
-  t.cross = 1.5707964f * ia * id2 * Pm * Qm;
-  t.cubic = 18.849556f * c3 * Pm * Qm * sum;  // rad, the c3 part of C
-  t.cube = c3 * big * big * big;
-  t.sq = sum * id2;
-  t.q4 = 0.0390625f * sum * sum * sum * sum * ia * id2 * id2 * id2;
+  // alpha P, which cycles32 has to hold, and c2 P^2, in 2^-32 cycles an int32; w^2, which
+  // p is scaled by, is no denormal
+  t.in_range = 0.5f * dl * sum <= 0x1p17f && 0.125f * dl * big * big <= 0.25f &&
+               id * inv_lambda * id2 >= 0x1p-100f;
+  t.cross = 1.5707964f * dl * p * q;
+  t.cubic = 1.1780972f * dl * p * q * sum;  // rad, the c3 part of C
+  t.cube = 0.0625f * dl * big * big * big;
+  t.sq = sum;
+  t.q4 = 0.0390625f * dl * sum * sum * sum * sum;
   return t;
 }
 
