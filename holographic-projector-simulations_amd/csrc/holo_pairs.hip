@@ -33,8 +33,8 @@
 // Operands are f16 pairs x = hi + lo (both rounded to nearest), and a full
 // product is hi hi + hi lo + lo hi, in FP32: only lo lo (2^-22, of either sign)
 // is left out.  g_0 and the near form's g_1 are full products; the far form's g_1
-// (below 1e-3 of the sum) and g_2, g_3 (below 1.8e-3) take the phasors' and weights' hi
-// parts and both of T's, which are sums (T's hi parts alone: 3 to 4 % less time).  X
+// (below 1e-3 of the sum), g_2 (below 4.5e-4, full above) and g_3 (below 1.7e-4) take the
+// phasors' and weights' hi parts and both of T's, which are sums (T's hi parts alone: 3 to 4 % less time).  X
 // carries A over the planes' 1 / |dz|.  The matrix cores' FP32 sums are rounded to
 // one side: in T that is turned by X's phases, but in the second product it would
 // add up over the tiles (1.6e-7 of the field over 1024 tiles; 5e-7 when one
@@ -187,12 +187,14 @@ __device__ void pair_tail_weights(const PairPrep& a, double* s_red) {
 }
 
 // The largest cross a tile pair takes each form with.  The far form drops C^2 / 2 and
-// the near form C^4 / 24; lowering the constant to 1 - m^2 / 4, m the pair's largest
-// |C|, leaves at most m^2 / 4 (2.5e-7), and 1 / 2 to 1 / 2 - m^2 / 24 in the C^2 term at
-// most m^4 / 96 (1.4e-7).  These hold for one lit source in the worst corner of its
-// tile; over dense weights C's triangular distribution leaves less.  The f16 parts that
-// the small products drop are of the same size: 1e-3 2^-12 and 0.06^2 / 2 2^-12.
-constexpr float kCrossFar = 1e-3f, kCrossNear = 0.06f;
+// the near form C^4 / 24; with m the pair's largest |C|, lowering the constant to 1 -
+// m^2 / 4 leaves at most m^2 / 4 of the one (2.5e-7), and 1 - m^4 / 192 with 1 / 2 -
+// m^2 / 24 in the C^2 term at most m^4 / 192 of the other (5.2e-7).  These hold for one lit
+// source in the worst corner of its tile; over dense weights C's triangular
+// distribution leaves a tenth.  f16 hi parts leave about 2^-12 of a product: of C in the
+// far form (2.4e-7), of C^2 / 2 in the near form up to kCrossHi (1.1e-7; full products from
+// there on) and of C^3 / 6 above (4e-8).
+constexpr float kCrossFar = 1e-3f, kCrossHi = 0.03f, kCrossNear = 0.1f;
 
 // The source tile width for targets with the first and last tile centres (cx0, cy0),
 // (cx1, cy1): the wide tiles where the near form holds for every pair of them, but the
@@ -339,12 +341,12 @@ __device__ __forceinline__ Cplx8 operand_of(const pf16& Tr, const pf16& Ti, int 
 }
 
 // PART 0: the far form (g_0 full, g_1 hi parts); PART 1, 2: the near form's g_0,
-// g_1 (full) and g_2, g_3 (hi parts).  Adds the products of a tile with `steps`
+// g_1 (full) and g_2, g_3 (hi parts); PART 3: as 2 with g_2 full.  Adds the products of a tile with `steps`
 // steps of 16 columns (weights wt) into (Dr, Di).
 template <int PART, int SIGN, bool OBL>
 __device__ __forceinline__ void pair_products(const PairWave<SIGN, OBL>& pw, const pu4* wt,
                                               uint32_t steps, pf16& Dr, pf16& Di) {
-  constexpr bool NEAR = PART != 0;
+  constexpr bool NEAR = PART != 0, FULL_A = PART == 1 || PART == 3;
   constexpr float kSig = SIGN > 0 ? -1.f : 1.f;
   pf16 Ar = kZero16, Ai = kZero16, Br = kZero16, Bi = kZero16;
   pf16 Lr = kZero16, Li = kZero16;  // far form: the small parts, apart
@@ -380,8 +382,8 @@ __device__ __forceinline__ void pair_products(const PairWave<SIGN, OBL>& pw, con
         } else {
           const float q2 = q * q;
           const float hr = -q2 * __builtin_fmaf(kSig * pw.gQ, q, pw.half), hi = pw.gP * q;
-          ar[e] = hr * yr - hi * yi;
-          ai[e] = hr * yi + hi * yr;
+          ar[e] = formed(hr * yr - hi * yi);
+          ai[e] = formed(hr * yi + hi * yr);
           gr = -kSig * pw.gP * q2;
           gi = (-kSig / 6.f) * (q2 * q);
         }
@@ -401,11 +403,14 @@ __device__ __forceinline__ void pair_products(const PairWave<SIGN, OBL>& pw, con
       if constexpr (PART == 1) {
         split8(y.c, y.am, a.rh, a.rl);
         split8(y.s, y.am, a.ih, a.il);
+      } else if constexpr (PART == 3) {
+        split8(ar, pw.one, a.rh, a.rl);
+        split8(ai, pw.one, a.ih, a.il);
       } else {
         a.rh = half8(ar);
         a.ih = half8(ai);
       }
-      if constexpr (PART == 1) cmul_lo(w, a, Ar, Ai);
+      if constexpr (FULL_A) cmul_lo(w, a, Ar, Ai);
       cmul_hi(w, a, Ar, Ai);
     }
   }
@@ -444,14 +449,17 @@ __device__ __forceinline__ void pair_products(const PairWave<SIGN, OBL>& pw, con
         br[e] = formed(p * ar[e]);
         bi[e] = formed(p * ai[e]);
       }
-      if constexpr (PART == 1) {
+      if constexpr (FULL_A) {
         split8(ar, pw.one, a.rh, a.rl);
         split8(ai, pw.one, a.ih, a.il);
-        split8(br, pw.one, b.rh, b.rl);
-        split8(bi, pw.one, b.ih, b.il);
       } else {
         a.rh = half8(ar);
         a.ih = half8(ai);
+      }
+      if constexpr (PART == 1) {
+        split8(br, pw.one, b.rh, b.rl);
+        split8(bi, pw.one, b.ih, b.il);
+      } else {
         b.rh = half8(br);
         b.ih = half8(bi);
       }
@@ -462,12 +470,12 @@ __device__ __forceinline__ void pair_products(const PairWave<SIGN, OBL>& pw, con
       cmul_hi(b, tb, Lr, Li);
     } else {
       if constexpr (PART == 1) cmul_lo(b, tb, Dr, Di);
-      if constexpr (PART == 2) cmul_hl(b, tb, Dr, Di);
+      if constexpr (PART >= 2) cmul_hl(b, tb, Dr, Di);
       cmul_hi(b, tb, Dr, Di);
     }
     const Cplx8 ta = operand_of(Ar, Ai, s, pw.one);
     if constexpr (PART == 0) cmul_lo(a, ta, Lr, Li);
-    if constexpr (PART == 1) cmul_lo(a, ta, Dr, Di);
+    if constexpr (FULL_A) cmul_lo(a, ta, Dr, Di);
     if constexpr (PART == 2) cmul_hl(a, ta, Dr, Di);
     cmul_hi(a, ta, Dr, Di);
   }
@@ -602,7 +610,8 @@ __device__ __forceinline__ void pair_items(PairWave<SIGN, OBL>& pw, const PairSo
         const float iY = (1.f / kFourPi) * iw;  // 1 / wY
         const bool near = !(far >> k & 1);  // uniform
         pw.a0X = OBL ? (arz * id) * (arz * id) : arz * id;
-        if (!near) pw.a0X -= 0.25f * cross * cross * pw.a0X;
+        const float c2 = cross * cross;
+        pw.a0X -= (near ? (1.f / 192.f) * c2 * c2 : 0.25f * c2) * pw.a0X;
         pw.a1X = pw.a0X * ((OBL ? -1.f : -0.5f) * id2 * iw);
         pw.a1Y = (OBL ? -1.f : -0.5f) * id2 * iY;
         // every other tile enters the matrix cores with the opposite sign
@@ -629,12 +638,15 @@ __device__ __forceinline__ void pair_items(PairWave<SIGN, OBL>& pw, const PairSo
           pw.k11 = k11 * (id2 * iw) * (id2 * iY);
           pw.gP = (float)SIGN * 9.424778f * id2 * iY;              // s 6 pi c3 / (w^2 wY)
           pw.gQ = (float)SIGN * 9.424778f / kFourPi * id2 * iY;   // s 6 pi c3 / (w wY^2)
-          pw.half = __builtin_fmaf(-1.f / 24.f, cross * cross, 0.5f);
+          pw.half = __builtin_fmaf(-1.f / 24.f, c2, 0.5f);
           add(IC<1>{});
           // the same phasors again: kept from the first part, and with its results,
           // they would not fit the registers
           __asm__ volatile("" : "+v"(pw.FtX), "+v"(pw.FtY), "+v"(pw.PtX), "+v"(pw.PtY) : : "memory");
-          add(IC<2>{});
+          if (cross <= kCrossHi)  // uniform
+            add(IC<2>{});
+          else
+            add(IC<3>{});
         }
       }
     }
