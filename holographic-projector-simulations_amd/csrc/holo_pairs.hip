@@ -518,7 +518,6 @@ __device__ __forceinline__ void pair_items(PairWave<SIGN, OBL>& pw, const PairSo
   const double tau = ti * (h ? pt.py : pt.px);
   const double del = h ? ((double)j - midY) * sr.py : ti * sr.px;
   const double del3 = ((double)(32 + j) - midY) * sr.py;  // columns 32 .. 63 of a wide tile
-  const double tau2 = tau * tau, del2 = del * del, del32 = del3 * del3;
   // source tiles of this mode, tj per row; a wide tile may lack its second half,
   // whose weights are then 0
   const uint32_t stj = wide ? sr.tj : (sr.ny + 31) / 32;
@@ -578,14 +577,14 @@ __device__ __forceinline__ void pair_items(PairWave<SIGN, OBL>& pw, const PairSo
         const float iw = __builtin_amdgcn_rcpf(w), wY = kFourPi * w, wA = h ? wY : w;
         {
           const double r2 = 2.0 * (h ? ry : rx);
-          const double gt = __builtin_fma(r2, tau, tau2), gs = __builtin_fma(-r2, del, del2);
+          const double gt = tau * (tau + r2), gs = del * (del - r2);
           wave_sync();  // the previous tile's reads are done
           lds.tF[wv][lane] = cycles32(__builtin_fma(al, gt, h ? kCycles32 : kCycles32 + f));
           lds.tp[wv][lane] = wA * (float)gt;
           lds.sF[wv][lane] = cycles32(__builtin_fma(al, gs, kCycles32));
           lds.sp[wv][lane] = wA * (float)gs;
           if (wide) {  // uniform
-            const double g3 = __builtin_fma(-2.0 * ry, del3, del32);
+            const double g3 = del3 * (del3 - 2.0 * ry);
             if (!h) {
               lds.sF[wv][64 + j] = cycles32(__builtin_fma(al, g3, kCycles32));
               lds.sp[wv][64 + j] = wY * (float)g3;
