@@ -114,6 +114,16 @@ def cpu_baseline(stage, n_targets: int, repeats: int):
     return res, sub, y[:, 0] * np.exp(1j * y[:, 1])
 
 
+def fp32_kernel(a, lattice):
+    """The FP32-split kernel that takes the plane's lattice of targets."""
+    if lattice and a.lattice_tiles:
+        return ("lattice-to-lattice kernel" if a.lattice_tiles == 64 else
+                f"lattice kernel, {min(a.lattice_tiles, 16)}x{a.lattice_tiles} tiles")
+    if a.lattice_tiles and a.tile in (0, 64):
+        return "point-to-lattice kernel"
+    return f"tiled kernel, tiles of {a.tile}"
+
+
 def time_events(fn, repeats: int, warmup: int = 1):
     """fn() timed with HIP events on torch's current stream (the stream the
     library launches on): `warmup` untimed calls, then `repeats` timed ones.
@@ -292,8 +302,7 @@ def main():
             out["fp32_split"] = {
                 "workload": f"{src_desc} -> 1024^2 (z 0 -> {p3.v[0, 2]:g} m, 10 / 7.56 um, amp U[0,1), "
                             "phase U[0,2pi)), " + (
-                                f"lattice kernel, {min(a.lattice_tiles, 16)}x{a.lattice_tiles} tiles"
-                                if a.lattice_tiles and lattice3 else f"tiled kernel, tiles of {a.tile}"),
+                                fp32_kernel(a, bool(lattice3))),
                 "pairs": pairs,
                 "fp64_pairs_per_s": pairs / (t64["median_ms"] / 1e3),
                 "fp64_ms": t64,

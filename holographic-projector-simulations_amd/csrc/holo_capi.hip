@@ -1570,7 +1570,7 @@ holo_status holo_transform_full(holo_ctx* ctx, holo_precision precision, int sig
                             return plan_fp64_at(ctx, plan, sign, obl, lambda, holo::kPolar, da,
                                                 dp, e, count);
                           }));
-    HOLO_HIP(hipStreamSynchronize(ctx->stream));  // plan buffers die here
+    HOLO_HIP(hipStreamSynchronize(ctx->stream));  // a large call's plan ends here
   }
   return finish_out(ctx, y, dy, 2 * M, dev);
 }

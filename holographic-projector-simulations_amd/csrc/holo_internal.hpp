@@ -113,8 +113,9 @@ int choose_splits(size_t M, int R, size_t units, size_t min_units_per_split,
                   size_t max_splits = 64);
 
 // Source splits of the tiled kernel (tiles of at most 64 sources) and, grid_splits,
-// of the lattice kernels (tiles of 16 x 16 group): down to a tile each while M targets
-// (a lane each) leave the chip idle, runs of at least 64 and 16 tiles above.  Pairs
+// of the lattice kernels (tiles of 16 x 16 group): while M targets (a lane each) leave
+// the chip idle down to a tile each, 16 x 16 and 16 x 32 tiles to 16 and 8 (the
+// smaller lattices'), above runs of at least 64 and 16 tiles.  Pairs
 // too near for the GEMM forms, 256^2 sources, in us with runs at every size and now:
 // jittered to 16^2, 64^2 and 128^2 targets 900, 1130, 1380 and 125, 300, 800; lattice
 // to the same 734, 986, 767 and 106, 203, 558; 64^2 jittered to 64^2 1189 and 52.

@@ -32,7 +32,9 @@ Tuning& tuning() {
 // that takes c waves one after the other or together needs w (c + k), w = a wave's
 // pairs at kF64Pair[R] each and k the last wave's latency that nothing hides; c is
 // the largest count of workgroups per CU.  A workgroup loads the sin/cos table
-// (kF64Start), and a split writes partial values that a reduction reads.
+// (kF64Start for every kF64Resident of them on a CU: fitted, like the rest; 4 or 5
+// workgroups are resident, by the layout's variant), and a split writes partial values
+// that a reduction reads.
 struct F64Cost {
   int R;
   double pair, k;

@@ -3,8 +3,9 @@
 // plan's host builder (holo_capi.hip: complete_rows, row_length, uniform_z,
 // build_grid16), which needs the positions on the host.
 //
-// What bounds it: latency, five dependent launches of a few us and one 72-byte
-// copy back; the positions are read once, at 512^2 sources 6 us.  There the host
+// What bounds it: latency, three dependent launches of 3 to 4 us, a copy of 64 bytes
+// back, and the launch that cuts the tiles; the search reads the positions once, at
+// 512^2 sources 6 us.  There the host
 // builder took 1.5 ms: 0.6 ms to copy 6.3 MB into fresh pages, the rest to scan and
 // cut them, and 0.4 ms to upload the tiles.
 #include <hip/hip_runtime.h>

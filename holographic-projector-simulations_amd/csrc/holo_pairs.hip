@@ -28,14 +28,14 @@
 // k_pair_prep picks the width from the near form's bounds over all tile pairs
 // (pair_mode), or neither, and then the 16-row kernels run as if this kernel did not
 // exist.  (One form for a whole call, far up to cross = 2.4e-3 and near up to 0.12, left
-// 2.0e-6 of the field for one lit source in a tile's corner; now 5.8e-7.)
+// up to 2.8e-6 of the field for one lit source in a tile's corner; now 5.8e-7.)
 //
 // Operands are f16 pairs x = hi + lo (both rounded to nearest), and a full
 // product is hi hi + hi lo + lo hi, in FP32: only lo lo (2^-22, of either sign)
 // is left out.  g_0 and the near form's g_1 are full products; the far form's g_1
 // (below 1e-3 of the sum), g_2 (below 4.5e-4, full above) and g_3 (below 1.7e-4) take the
-// phasors' and weights' hi parts and both of T's, which are sums (T's hi parts alone: 3 to 4 % less time).  X
-// carries A over the planes' 1 / |dz|.  The matrix cores' FP32 sums are rounded to
+// phasors' and weights' hi parts and both of T's, which are sums (T's hi parts alone:
+// 3 to 4 % less time).  X carries A over the planes' 1 / |dz|.  The matrix cores' FP32 sums are rounded to
 // one side: in T that is turned by X's phases, but in the second product it would
 // add up over the tiles (1.6e-7 of the field over 1024 tiles; 5e-7 when one
 // accumulator ran over 16 tiles).  So each tile's products start from zero, every
@@ -58,12 +58,13 @@
 // phasors: X of target row j and Y of target column j.  Real and imaginary
 // parts are separate operands: T_re = Wr Yr + Wi (-Yi), T_im = Wr Yi + Wi Yr.
 //
-// What bounds it: VALU issue (650 instructions per 2^20 pairs in the far form before T's lo parts, half
-// of them for the phasors), beside the matrix cores; two waves per SIMD (253
-// VGPRs).  Per call, 1024^2 -> 1024^2 at 0.35 m: 2.37 ms, 3 % of the tile pairs near (one
-// form for all: 2.05 ms), where the 16 x 64 tiles of k_superpose_grid16 take 57.8 ms;
-// 512^2 -> 512^2 at 0.1 m 0.32 ms, 75 % near (8.2 ms); 64^2 -> 64^2: 28 us (34 us).  With
-// 32 x 32 source tiles the far form took 1.35 times as long at 1024^2.
+// What bounds it: VALU issue, 76 % busy (805 instructions per 2^20 pairs at 1024^2 and
+// 0.35 m, half of them for the phasors), beside matrix cores at 38 %; two waves per SIMD
+// (253 VGPRs).  Per call, 1024^2 -> 1024^2 at 0.35 m: 2.31 to 2.38 ms, 3 % of the tile
+// pairs near (one form for all: 2.03 to 2.09 ms), where the 16 x 64 tiles of
+// k_superpose_grid16 take 57.8 ms; 3.9 ms at 0.2 m (93 ms; one form 4.5 ms), 6.2 ms at
+// 0.1 m (140 ms); 512^2 -> 512^2 at 0.1 m 0.31 ms, 75 % near (8.2 ms); 64^2 -> 64^2: 25
+// to 29 us (34 us).  With 32 x 32 source tiles the far form took 1.35 times as long.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
