@@ -375,7 +375,9 @@ hipError_t launch_superpose_points(int sign, bool obliquity, const PointPlan& pp
                                    double lambda, int S, PairTargets* pt, uint32_t* flags,
                                    uint32_t* handled, double2* out, hipStream_t stream) {
   if (M == 0 || !pp.n_slots) return hipErrorInvalidValue;
-  const uint32_t n_probe = (uint32_t)std::min<size_t>(std::max<size_t>(M / kBlock, 1), kPairFlags);
+  // (eight sources a lane: one workgroup looked at 212040 weights for 66 us)
+  const uint32_t n_probe = (uint32_t)std::min<size_t>(
+      std::max<size_t>({M / kBlock, pp.n / (8 * kBlock), 1}), kPairFlags);
   const double il = 1.0 / lambda;
   k_point_prep<<<(pp.n_slots + kBlock - 1) / kBlock + n_probe, kBlock, 0, stream>>>(
       pp, (int)wf, w0, w1, v, (uint32_t)M, n_probe, il, obliquity ? 1u : 0u, pt, flags);
