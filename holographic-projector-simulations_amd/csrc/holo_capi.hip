@@ -215,9 +215,15 @@ holo_status noalloc_scratch(int device, void** out) {
   return HOLO_OK;
 }
 
-holo_status use_device(holo_ctx* ctx) {
+holo_status set_device(holo_ctx* ctx) {
   if (!ctx) return fail(HOLO_EINVAL, "null context");
   HOLO_HIP(hipSetDevice(ctx->device));
+  return HOLO_OK;
+}
+
+// The context's device, and whether its stream is being captured.
+holo_status use_device(holo_ctx* ctx) {
+  HOLO_TRY(set_device(ctx));
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
     (void)hipGetLastError();  // (the null stream beside another stream's capture)
@@ -1244,7 +1250,7 @@ holo_status plan_run_body(holo_ctx* ctx, const holo_plan* p, int precision, int 
     gt.rho_x = p->grid_rho_x;
     gt.rho_y = p->grid_rho_y;
     size_t pe;
-    HOLO_TRY(partial_room(ctx, elems(holo::grid_splits(M, nt, 1)), &pe));
+    HOLO_TRY(partial_room(ctx, elems(holo::grid8_splits(M, nt)), &pe));
     HOLO_HIP(holo::launch_superpose_grid(sign, obliquity, gt,
                                          static_cast<const float2*>(p->g_wc.ptr),
                                          static_cast<const uint4*>(p->g_wh.ptr),
@@ -1403,7 +1409,7 @@ void holo_destroy(holo_ctx* ctx) {
 }
 
 holo_status holo_set_stream(holo_ctx* ctx, void* stream) {
-  HOLO_TRY(use_device(ctx));
+  HOLO_TRY(set_device(ctx));
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (ctx->stream == s) return HOLO_OK;
   if (ctx->own_stream) {
@@ -1423,7 +1429,7 @@ holo_status holo_set_stream(holo_ctx* ctx, void* stream) {
 }
 
 holo_status holo_synchronize(holo_ctx* ctx) {
-  HOLO_TRY(use_device(ctx));
+  HOLO_TRY(set_device(ctx));
   HOLO_HIP(hipStreamSynchronize(ctx->stream));
   return HOLO_OK;
 }

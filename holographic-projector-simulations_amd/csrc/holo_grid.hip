@@ -335,12 +335,23 @@ __global__ __launch_bounds__(kBlock) void k_superpose_grid(
   if (mo < M) out[(size_t)blockIdx.y * M + mo] = make_double2(sr, si);
 }
 
+int grid8_splits(size_t M, size_t n_tiles) {
+  return n_tiles ? choose_splits(M, 1, n_tiles, 16) : 1;
+}
+
+// Whether a 16-row launch splits its sources in units of 16 x 64, whatever the tiles'
+// width: a wave that takes smaller tiles of the same sources then sums the pairs of
+// tiles that their own launch does.
+static bool split_by_units(size_t M) { return tuning().splits <= 0 && M < kFillTargets; }
+
 int grid_splits(size_t M, size_t n_tiles, int group) {
-  // below 32 tiles of 16 x 16 the reduction's launch costs what the splits give (a
-  // caller's own count holds)
-  if (n_tiles == 0 || (tuning().splits <= 0 && n_tiles * group < 32)) return 1;
-  return choose_splits(M, 1, n_tiles, M < kFillTargets ? (group == 4 ? 1 : 16 / group) : 16,
-                       kTileSplits);
+  // up to 8 tiles the reduction's launch costs what the splits give far away (a caller's
+  // own count holds)
+  if (n_tiles == 0 || (tuning().splits <= 0 && n_tiles * group <= 8)) return 1;
+  if (!split_by_units(M)) return choose_splits(M, 1, n_tiles, 16, kTileSplits);
+  const size_t units = (n_tiles * group + 3) / 4;
+  const size_t run = (units - 1) / choose_splits(M, 1, units, 1, kTileSplits) + 1;
+  return (int)((units - 1) / run + 1);
 }
 
 hipError_t launch_superpose_grid(int sign, bool obliquity, const GridTiles& gt,
@@ -349,7 +360,7 @@ hipError_t launch_superpose_grid(int sign, bool obliquity, const GridTiles& gt,
                                  double lambda, double2* y, double2* partial,
                                  size_t partial_cap, hipStream_t stream) {
   if (M == 0) return hipSuccess;
-  int S = grid_splits(M, gt.n_tiles, 1);
+  int S = grid8_splits(M, gt.n_tiles);
   while (S > 1 && (size_t)S * M > partial_cap) --S;
   const uint32_t chunk = gt.n_tiles ? (gt.n_tiles + S - 1) / S : 0;
   const dim3 grid((unsigned)((M + kBlock - 1) / kBlock), (unsigned)S);
@@ -1071,7 +1082,9 @@ hipError_t launch_superpose_grid16(int sign, bool obliquity, int nkc, const Grid
   if (gt.n_tail && (!gt.tail_perm || !gt.tail_wc)) return hipErrorInvalidValue;
   int S = grid_splits(M, gt.n_tiles, nkc);
   while (S > 1 && (size_t)S * M > partial_cap) --S;
-  const uint32_t chunk = gt.n_tiles ? (gt.n_tiles + S - 1) / S : 0;
+  const uint32_t unit = S > 1 && split_by_units(M) ? 4 / nkc : 1;  // tiles
+  const uint32_t units = (gt.n_tiles + unit - 1) / unit;
+  const uint32_t chunk = (units + S - 1) / S * unit;
   const dim3 grid((unsigned)((M + kBlock - 1) / kBlock), (unsigned)S);
   double2* out = S > 1 ? partial : y;
   const double il = 1.0 / lambda;

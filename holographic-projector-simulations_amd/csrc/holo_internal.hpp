@@ -113,12 +113,15 @@ int choose_splits(size_t M, int R, size_t units, size_t min_units_per_split,
                   size_t max_splits = 64);
 
 // Source splits of the tiled kernel (tiles of at most 64 sources) and, grid_splits,
-// of the lattice kernels (tiles of 16 x 16 group): while M targets (a lane each) leave
-// the chip idle down to a tile each, 16 x 16 and 16 x 32 tiles to 16 and 8 (the
-// smaller lattices'), above runs of at least 64 and 16 tiles.  Pairs
+// of the 16-row kernels (tiles of 16 x 16 group): down to a tile (16 x 64 sources) each
+// while M targets (a lane each) leave the chip idle, runs of at least 64 and 16 tiles
+// above.  Pairs
 // too near for the GEMM forms, 256^2 sources, in us with runs at every size and now:
 // jittered to 16^2, 64^2 and 128^2 targets 900, 1130, 1380 and 125, 300, 800; lattice
-// to the same 734, 986, 767 and 106, 203, 558; 64^2 jittered to 64^2 1189 and 52.
+// to the same 734, 986, 767 and 106, 203, 558; 64^2 jittered to 64^2 1189 and 52.  Up to
+// 8 tiles of 16 x 16 the lattice kernels stay in one launch: 16 x 128 far away 22.5 us
+// and 24 in two, but 64^2 to 64^2 32 and 24, near 324 and 94 (56 x 84 392 and 94).  The
+// 8 x 8 kernel keeps runs of 16 tiles (128^2 to 64^2 far away 31 us, in runs of one 38).
 constexpr size_t kTileSplits = 128, kFillTargets = size_t(1) << 18;
 int tile_splits(size_t M, int R, size_t n_tiles);
 
@@ -228,8 +231,10 @@ hipError_t launch_superpose_grid16(int sign, bool obliquity, int nkc, const Grid
                                    double lambda, double2* y, double2* partial,
                                    size_t partial_cap, hipStream_t stream,
                                    const uint32_t* skip = nullptr, int Sp = 1);
-// Source splits the lattice kernel uses for M targets over n_tiles tiles.
+// Source splits the 16-row kernels use for M targets over n_tiles tiles of 16 x 16
+// group, and the 8 x 8 kernel over n_tiles of its own.
 int grid_splits(size_t M, size_t n_tiles, int group);
+int grid8_splits(size_t M, size_t n_tiles);
 
 // Lattice-to-lattice kernel (holo_pairs.hip): the sources of a uniform lattice
 // x0 + i px, y0 + j py, z (n = i ny + j, i < nx, j < ny), cut into 32 x 64 tiles
