@@ -131,7 +131,7 @@ holo_status holo_trim(holo_ctx *ctx);
  * HOLO_FP32_SPLIT to targets on a uniform lattice, 256 or more, uses the
  * lattice-to-lattice kernel where the sources are on a uniform lattice too,
  * and the point-to-lattice kernel for 256 or more sources elsewhere, within
- * their far-field bounds; default 1),
+ * their bounds and for weights that are finite in FP32; default 1),
  * "grid" (0/1: HOLO_FP32_SPLIT on lattice sources uses the matrix-core
  * lattice kernel; default 1), "grid16" (0/1: on a uniform lattice that
  * kernel uses 16 x 16 tiles, padded to multiples of 16; default 1), "grid32"
