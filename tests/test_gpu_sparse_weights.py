@@ -71,3 +71,19 @@ def test_few_lit_sources(pkg, ctx, oracle, geometry, cross, lit, sign, obliquity
     err = np.linalg.norm(y - ref)
     print(f"{err / np.linalg.norm(ref):.2e} of the field, {err / alone:.2e} of the sources alone")
     assert err <= 1e-6 * max(np.linalg.norm(ref), alone)
+
+
+@pytest.mark.parametrize("scale", [1e-38, 1e-30, 1.0, 1e30])
+@pytest.mark.parametrize("src", [(16, 16), (33, 65), (64, 96)])
+def test_polar_weights_of_any_scale(pkg, ctx, oracle, scale, src):
+    """Amplitudes (of either sign) whose tiles differ by 1e6, and tiles of zeros: a tile's
+    scale comes from its largest modulus."""
+    u, v = lattice(*src, 10e-6, 9e-6), lattice(33, 44, 8e-6, 8e-6, 5e-4, 0, 0.3)
+    g = np.random.default_rng(5)
+    a = g.standard_normal(src)
+    a[32:] *= 1e-6
+    a[:, 64:] = 0.0
+    amp, phase = a.ravel(), g.random(a.size) * 2 * np.pi
+    y = ctx.plan(u).transform(amp * scale, phase, v, 1, LAM, pkg.FP32_SPLIT) / scale
+    ref = oracle.transform_full(1, LAM, amp, phase, u, v)
+    assert np.linalg.norm(y - ref) <= 1e-6 * np.linalg.norm(ref)
