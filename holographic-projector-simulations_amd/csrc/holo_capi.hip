@@ -90,6 +90,8 @@ struct holo_ctx {
   ~holo_ctx();
   int device = 0;
   hipStream_t stream = nullptr;
+  // The context's own stream, made by the first call that uses it (use_device): most
+  // programs set theirs before, and to make and destroy one takes 25 to 600 us.
   bool own_stream = false;
   // staging buffers for host-pointer calls and scratch
   DevBuf amp, phase, u, v, y, w, partial, small, b, pos, ph;
@@ -224,6 +226,8 @@ holo_status set_device(holo_ctx* ctx) {
 // The context's device, and whether its stream is being captured.
 holo_status use_device(holo_ctx* ctx) {
   HOLO_TRY(set_device(ctx));
+  if (ctx->own_stream && !ctx->stream)
+    HOLO_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
     (void)hipGetLastError();  // (the null stream beside another stream's capture)
@@ -1385,16 +1389,8 @@ holo_status holo_create(holo_ctx** out, int device, void* stream) {
   HOLO_TRY(noalloc_scratch(device, &scratch_ptr));
   holo_ctx* c = new holo_ctx();
   c->device = device;
-  if (stream) {
-    c->stream = static_cast<hipStream_t>(stream);
-  } else {
-    hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
-    if (e != hipSuccess) {
-      delete c;
-      return fail(HOLO_EDEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(e));
-    }
-    c->own_stream = true;
-  }
+  c->stream = static_cast<hipStream_t>(stream);
+  c->own_stream = !stream;
   *out = c;
   return HOLO_OK;
 }
@@ -1402,8 +1398,8 @@ holo_status holo_create(holo_ctx** out, int device, void* stream) {
 void holo_destroy(holo_ctx* ctx) {
   if (!ctx) return;
   (void)hipSetDevice(ctx->device);
-  (void)hipStreamSynchronize(ctx->stream);
-  if (ctx->own_stream) (void)hipStreamDestroy(ctx->stream);
+  if (!ctx->own_stream || ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+  if (ctx->own_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
   if (ctx->switched) (void)hipEventDestroy(ctx->switched);
   delete ctx;
 }
@@ -1411,10 +1407,12 @@ void holo_destroy(holo_ctx* ctx) {
 holo_status holo_set_stream(holo_ctx* ctx, void* stream) {
   HOLO_TRY(set_device(ctx));
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (ctx->stream == s) return HOLO_OK;
+  if (!ctx->own_stream && ctx->stream == s) return HOLO_OK;
   if (ctx->own_stream) {
-    HOLO_HIP(hipStreamSynchronize(ctx->stream));
-    HOLO_HIP(hipStreamDestroy(ctx->stream));
+    if (ctx->stream) {
+      HOLO_HIP(hipStreamSynchronize(ctx->stream));
+      HOLO_HIP(hipStreamDestroy(ctx->stream));
+    }
     ctx->own_stream = false;
   } else {
     // work queued on the previous stream may still use the context's scratch
@@ -1430,7 +1428,7 @@ holo_status holo_set_stream(holo_ctx* ctx, void* stream) {
 
 holo_status holo_synchronize(holo_ctx* ctx) {
   HOLO_TRY(set_device(ctx));
-  HOLO_HIP(hipStreamSynchronize(ctx->stream));
+  if (!ctx->own_stream || ctx->stream) HOLO_HIP(hipStreamSynchronize(ctx->stream));
   return HOLO_OK;
 }
 

@@ -98,7 +98,7 @@ const char *holo_status_string(holo_status status);
 const char *holo_last_error(void);
 
 /* Create a context on HIP device `device` using `stream` (a hipStream_t, or
- * NULL for a stream owned by the context).  Replaces the per-call stream and
+ * NULL for a stream owned by the context, made by the first call that uses it).  Replaces the per-call stream and
  * cuBLAS-handle creation of cuda/transform.cu:233-241. */
 holo_status holo_create(holo_ctx **ctx, int device, void *stream);
 void holo_destroy(holo_ctx *ctx);
