@@ -344,10 +344,17 @@ int grid8_splits(size_t M, size_t n_tiles) {
 // tiles that their own launch does.
 static bool split_by_units(size_t M) { return tuning().splits <= 0 && M < kFillTargets; }
 
+// Whether a workgroup's waves share the sources of 64 targets instead of taking 256:
+// lattices below 32 tiles of 16 x 16, where a reduction's launch, which calls to a lattice
+// of targets would pay too, costs what more splits give.  64^2 sources to 64^2 scattered
+// targets: 32 us in one split, 23 with four and a reduction, 21 so; near 320, 100 and 89.
+// Up to four tiles there is nothing to share.
+static bool waves_share(size_t M, size_t n_tiles, int group) {
+  return split_by_units(M) && n_tiles * group < 32 && n_tiles * group > 4;
+}
+
 int grid_splits(size_t M, size_t n_tiles, int group) {
-  // up to 8 tiles the reduction's launch costs what the splits give far away (a caller's
-  // own count holds)
-  if (n_tiles == 0 || (tuning().splits <= 0 && n_tiles * group <= 8)) return 1;
+  if (n_tiles == 0 || (tuning().splits <= 0 && n_tiles * group < 32)) return 1;
   if (!split_by_units(M)) return choose_splits(M, 1, n_tiles, 16, kTileSplits);
   const size_t units = (n_tiles * group + 3) / 4;
   const size_t run = (units - 1) / choose_splits(M, 1, units, 1, kTileSplits) + 1;
@@ -1008,12 +1015,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
     const double4* __restrict__ centre16, GridBounds gb16, const double* __restrict__ axes,
     LatticeAxes ax,
     const int32_t* __restrict__ tail_perm, const float2* __restrict__ tail_wc, uint32_t n_tail,
-    const uint32_t* __restrict__ skip, double2* __restrict__ out) {
+    const uint32_t* __restrict__ skip, uint32_t shared, double2* __restrict__ out) {
   if (skip && *skip) return;
   __shared__ Grid16Lds lds;
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const uint32_t base = blockIdx.x * kBlock + wv * 64;
-  const uint32_t t0 = blockIdx.y * chunk;
+  // shared: the workgroup's waves take the splits of 64 targets
+  const uint32_t base = shared ? blockIdx.x * 64 : blockIdx.x * kBlock + wv * 64;
+  const uint32_t split = __builtin_amdgcn_readfirstlane(shared ? wv : blockIdx.y);
+  const uint32_t t0 = min(n_tiles, split * chunk);
   const uint32_t t1 = min(n_tiles, t0 + chunk);
   const uint32_t mo = base + lane;
   const size_t mm = mo < M ? mo : M - 1;
@@ -1050,7 +1059,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
                                        vz, inv_lambda, px, py, b16, axes, ax, false, ex_r, ex_i);
   }
   // in blocks of 256 sources, so that each FP32 partial sum stays short
-  if (blockIdx.y == 0)
+  if (split == 0)
     for (uint32_t s0 = 0; s0 < n_tail; s0 += 256)
       exact_tile_pairs<SIGN, OBL>(u, tail_perm + s0, tail_wc + s0, (int)min(256u, n_tail - s0),
                                   vx, vy, vz, inv_lambda, ex_r, ex_i);
@@ -1062,6 +1071,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
   for (int q = 0; q < 4; ++q) {  // fixed order: deterministic
     sr += lds.rr[wv][lane >> 4][16 * q + (lane & 15)];
     si += lds.ri[wv][lane >> 4][16 * q + (lane & 15)];
+  }
+  if (shared) {  // uniform over the launch
+    __syncthreads();  // every wave has read its sums
+    lds.rr[wv][0][lane] = sr;
+    lds.ri[wv][0][lane] = si;
+    __syncthreads();
+    if (wv) return;
+    for (int k = 1; k < kGridWaves; ++k) {  // fixed order: deterministic
+      sr += lds.rr[k][0][lane];
+      si += lds.ri[k][0][lane];
+    }
   }
   if (mo < M) out[(size_t)blockIdx.y * M + mo] = make_double2(sr, si);
 }
@@ -1082,10 +1102,13 @@ hipError_t launch_superpose_grid16(int sign, bool obliquity, int nkc, const Grid
   if (gt.n_tail && (!gt.tail_perm || !gt.tail_wc)) return hipErrorInvalidValue;
   int S = grid_splits(M, gt.n_tiles, nkc);
   while (S > 1 && (size_t)S * M > partial_cap) --S;
-  const uint32_t unit = S > 1 && split_by_units(M) ? 4 / nkc : 1;  // tiles
+  const bool shared = waves_share(M, gt.n_tiles, nkc);  // (then S is 1)
+  const uint32_t parts = shared ? kGridWaves : (uint32_t)S;
+  const uint32_t unit = parts > 1 && split_by_units(M) ? 4 / nkc : 1;  // tiles
   const uint32_t units = (gt.n_tiles + unit - 1) / unit;
-  const uint32_t chunk = (units + S - 1) / S * unit;
-  const dim3 grid((unsigned)((M + kBlock - 1) / kBlock), (unsigned)S);
+  const uint32_t chunk = (units + parts - 1) / parts * unit;
+  const unsigned per = shared ? 64 : kBlock;  // targets of a workgroup
+  const dim3 grid((unsigned)((M + per - 1) / per), (unsigned)S);
   double2* out = S > 1 ? partial : y;
   const double il = 1.0 / lambda;
   const int series = tuning().grid_series ? 1 : 0;
@@ -1110,17 +1133,17 @@ hipError_t launch_superpose_grid16(int sign, bool obliquity, int nkc, const Grid
         k_superpose_grid16<sg.value, (bool)obl.value, 4><<<grid, kBlock, 0, stream>>>(
             gt.centre, gt.perm, gt.u, wc, wq, wqn, tscale, gt.n_tiles, chunk, v, (uint32_t)M,
             il, gt.px, gt.py, gb, pairs.centre, gb32, halves.centre, gb16, axes, ax,
-            gt.tail_perm, gt.tail_wc, gt.n_tail, skip, out);
+            gt.tail_perm, gt.tail_wc, gt.n_tail, skip, shared ? 1u : 0u, out);
       else if (nkc == 2)
         k_superpose_grid16<sg.value, (bool)obl.value, 2><<<grid, kBlock, 0, stream>>>(
             gt.centre, gt.perm, gt.u, wc, wq, wqn, tscale, gt.n_tiles, chunk, v, (uint32_t)M,
             il, gt.px, gt.py, gb, gt.centre, gb, halves.centre, gb16, axes, ax, gt.tail_perm,
-            gt.tail_wc, gt.n_tail, skip, out);
+            gt.tail_wc, gt.n_tail, skip, shared ? 1u : 0u, out);
       else
         k_superpose_grid16<sg.value, (bool)obl.value, 1><<<grid, kBlock, 0, stream>>>(
             gt.centre, gt.perm, gt.u, wc, wq, wqn, tscale, gt.n_tiles, chunk, v, (uint32_t)M,
             il, gt.px, gt.py, gb, gt.centre, gb, gt.centre, gb, axes, ax, gt.tail_perm,
-            gt.tail_wc, gt.n_tail, skip, out);
+            gt.tail_wc, gt.n_tail, skip, shared ? 1u : 0u, out);
     });
   });
   hipError_t e = hipGetLastError();

@@ -118,10 +118,9 @@ int choose_splits(size_t M, int R, size_t units, size_t min_units_per_split,
 // above.  Pairs
 // too near for the GEMM forms, 256^2 sources, in us with runs at every size and now:
 // jittered to 16^2, 64^2 and 128^2 targets 900, 1130, 1380 and 125, 300, 800; lattice
-// to the same 734, 986, 767 and 106, 203, 558; 64^2 jittered to 64^2 1189 and 52.  Up to
-// 8 tiles of 16 x 16 the lattice kernels stay in one launch: 16 x 128 far away 22.5 us
-// and 24 in two, but 64^2 to 64^2 32 and 24, near 324 and 94 (56 x 84 392 and 94).  The
-// 8 x 8 kernel keeps runs of 16 tiles (128^2 to 64^2 far away 31 us, in runs of one 38).
+// to the same 734, 986, 767 and 106, 203, 558; 64^2 jittered to 64^2 1189 and 52.  Below
+// 32 tiles of 16 x 16 the waves of a workgroup share the sources instead.  The 8 x 8
+// kernel keeps runs of 16 tiles (128^2 to 64^2 far away 31 us, in runs of one 38).
 constexpr size_t kTileSplits = 128, kFillTargets = size_t(1) << 18;
 int tile_splits(size_t M, int R, size_t n_tiles);
 
