@@ -100,7 +100,7 @@ struct holo_ctx {
   DevBuf pos64, ph64;            // FP64 Monte Carlo records for the error report
   // recorded on the previous stream when holo_set_stream switches streams
   hipEvent_t switched = nullptr;
-  bool capturing = false;        // the stream, as the call found it
+  int capturing = -1;            // whether the stream is (-1: the call has not asked)
   std::vector<DevBuf> retired;   // outgrown scratch that a captured graph still uses
   // FP32-split calls without a plan: the buffers of the last one (about 120 bytes a
   // source, at most kShotSources of them)
@@ -223,25 +223,32 @@ holo_status set_device(holo_ctx* ctx) {
   return HOLO_OK;
 }
 
-// The context's device, and whether its stream is being captured.
+// The context's device and stream, for a call.
 holo_status use_device(holo_ctx* ctx) {
   HOLO_TRY(set_device(ctx));
   if (ctx->own_stream && !ctx->stream)
     HOLO_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
-    (void)hipGetLastError();  // (the null stream beside another stream's capture)
-    st = hipStreamCaptureStatusNone;
-  }
-  ctx->capturing = st != hipStreamCaptureStatusNone;
+  ctx->capturing = -1;
   return HOLO_OK;
+}
+
+bool capturing(holo_ctx* ctx) {
+  if (ctx->capturing < 0) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
+      (void)hipGetLastError();  // (the null stream beside another stream's capture)
+      st = hipStreamCaptureStatusNone;
+    }
+    ctx->capturing = st != hipStreamCaptureStatusNone;
+  }
+  return ctx->capturing != 0;
 }
 
 // Context scratch of at least `bytes`.  Nothing is allocated while the stream is being
 // captured, and what a captured graph uses is kept when a later call outgrows it.
 holo_status ensure(holo_ctx* ctx, DevBuf& b, size_t bytes) {
   const bool fits = bytes <= b.bytes && b.ptr;
-  if (ctx->capturing) {
+  if (capturing(ctx)) {
     if (!fits)
       return fail(HOLO_EDEVICE, "scratch cannot be allocated during a capture: make the call "
                                 "once before it");
@@ -256,7 +263,7 @@ holo_status ensure(holo_ctx* ctx, DevBuf& b, size_t bytes) {
 // launch then takes fewer splits).
 holo_status partial_room(holo_ctx* ctx, size_t want, size_t* cap) {
   *cap = want;
-  if (ctx->capturing) *cap = std::min(want, ctx->partial.bytes / sizeof(double2));
+  if (want && capturing(ctx)) *cap = std::min(want, ctx->partial.bytes / sizeof(double2));
   return *cap ? ensure(ctx, ctx->partial, *cap * sizeof(double2)) : HOLO_OK;
 }
 
@@ -1434,7 +1441,7 @@ holo_status holo_synchronize(holo_ctx* ctx) {
 
 holo_status holo_trim(holo_ctx* ctx) {
   HOLO_TRY(use_device(ctx));
-  if (ctx->capturing) return fail(HOLO_EINVAL, "the context's stream is being captured");
+  if (capturing(ctx)) return fail(HOLO_EINVAL, "the context's stream is being captured");
   HOLO_HIP(hipStreamSynchronize(ctx->stream));
   ctx->shot.reset();
   for (DevBuf* b : {&ctx->amp, &ctx->phase, &ctx->u, &ctx->v, &ctx->y, &ctx->w, &ctx->partial,
